@@ -263,11 +263,10 @@ def probe_units(kernel: str, w: int, h: int) -> tuple[str, float]:
         # three DC planes in (float), three quantized planes out (int32)
         return "bytes", 24.0 * blocks
     if kernel == "DifferencesKernel":
-        # per scale (full and half resolution, one launch each; the mean
-        # launch covers 1.25 / 2 of the full-resolution pixels): 10 + 10
-        # psycho planes, both blurred activities, MaskY and MaskDcY in, the
-        # two final planes out
-        return "bytes", 104.0 * w * h * 1.25 / 2
+        # full and half resolution in one launch (1.25 of the full-resolution
+        # pixels): 10 + 10 psycho planes, both blurred activities, MaskY and
+        # MaskDcY in, the two final planes out
+        return "bytes", 104.0 * w * h * 1.25
     if kernel == "CandidateCostKernel":
         # binary64 DCT flops of all candidates over the 7 launches
         return "flops", candidate_flops(w, h) / 7.0

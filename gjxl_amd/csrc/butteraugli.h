@@ -47,7 +47,6 @@ struct GJXLAmdButteraugli {
   int xborder = 0, yborder = 0;
   bool prepared = false;
   gjxl_amd::ButteraugliScale scale[2];
-  float* taps = nullptr;       // kSigmaCount x 33 unscaled kernel taps
   float* map = nullptr;        // requested extent
   uint32_t* score_bits = nullptr;  // max of the map, as float bits
   void* allocation = nullptr;  // one block for everything above

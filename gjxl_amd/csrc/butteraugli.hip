@@ -3,20 +3,20 @@
 //
 //   OpsinDynamicsKernel   5x5 mirrored blur + opsin dynamics (Gamma via the
 //                         unfused FastLog2), butteraugli_internal.cpp:622-700
-//   BlurRows/ColsKernel   separable Gaussian of radius 3, 6, 7 or 16 with the
+//   BlurKernel            separable Gaussian of radius 16, 7, 3 or 6 with the
 //                         reference's interior summation order and its
-//                         renormalised border columns (:245-620)
-//   LowSplit/HighSplit/UltraSplit
-//                         SeparateFrequencies (:702-846), as epilogues of the
-//                         blurs' column passes
-//   MaskSource/MaskKernel masking activity, blur, fuzzy erosion, MaskY/MaskDcY
+//                         renormalised border columns (:245-620), both passes
+//                         in one kernel; SeparateFrequencies (:702-846) and
+//                         the masking activity are the blurs' epilogues
+//   MaskKernel            fuzzy erosion, MaskY/MaskDcY
 //   DifferencesKernel     MaltaDiffMap of the six stages (butteraugli_
 //                         distance_internal.cpp:482-577, zero outside the
 //                         image), their accumulation (UHF, HF, MF), the L2
 //                         terms, masked AC Y and the final composition
 //                         (:657-870), per tile
-//   Subsample/Expand/ComposeKernel
-//                         the two-scale map and its maximum (:872-1003)
+//   Expand/ComposeKernel  the two-scale map and its maximum (:872-1003); the
+//                         half-scale image is formed where the opsin kernel
+//                         reads it
 //   ReduceKernel          ReduceButteraugliDistanceMap (butteraugli.cpp:
 //                         116-222)
 //
@@ -24,6 +24,13 @@
 // order (binary32, no contraction; binary64 where the reference promotes), so
 // the maps equal the CPU's bit for bit.  The reference image's planes and
 // masking terms are computed once per prepare and stay resident.
+//
+// Every launch covers both scales: the work groups of the half scale follow
+// those of the full one.  An image has some fifty kernels' worth of stages,
+// and below about two megapixels each of them is over before the next launch
+// could have filled the chip (a 512x512 comparison and preparation took 88
+// launches of 4 to 16 us each; now 13).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -36,15 +43,17 @@ namespace gjxl_amd {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTapStride = 64;  // 33 unscaled taps, then 17 scaled taps
+// A blur's taps travel in its kernel's arguments: read through a pointer they
+// were vector loads at every use, since the planes a kernel writes may alias
+// them as far as the compiler knows.
+struct Taps {
+  float k[33], sk[17];
+};
 constexpr float kSigmas[kSigmaCount] = {1.2f, 7.15593339443f, 3.22489901262f,
                                         1.56416327805f, 2.7f};
 
-__device__ __forceinline__ int BMirror(int c, int size) {
-  while (c < 0 || c >= size) c = c < 0 ? -c - 1 : 2 * size - 1 - c;
-  return c;
-}
-// BMirror for -size <= c < 2 * size (one reflection), by selects.
+// Mirrored coordinate for -size <= c < 2 * size (one reflection), by selects.
+// (Both scales are at least 8 pixels a side.)
 __device__ __forceinline__ int BMirrorOnce(int c, int size) {
   c = c < 0 ? -c - 1 : c;
   return c >= size ? 2 * size - 1 - c : c;
@@ -71,193 +80,323 @@ __device__ __forceinline__ float ConvolveInterior(const float* s, const float* s
   return r;
 }
 
-// A border output of ConvolutionWithTranspose (fewer than R samples on one
-// side): the taps that fall inside the line, renormalised; sample(sx) gives
-// the line's sample sx.  Every tap is visited in ascending order and the
-// ones outside the line are skipped by selects, so the sums are the
-// reference's; samples are read at clamped positions, which stay within
-// pos - R .. pos + R.
-template <int R, typename Sample>
-__device__ __forceinline__ float ConvolveBorder(Sample sample, int pos, int len,
-                                                const float* __restrict__ k) {
+// 1 / the weight of the taps that fall inside a line of `len` samples around
+// the border position of index `i`: positions 0 .. R - 1 have the indexes 0 ..
+// R - 1, those of the other end R .. 2R - 1 (BorderPosition).  Every tap is
+// visited in ascending order and the ones outside are skipped by selects, so
+// the sum is the reference's.
+template <int R>
+__device__ __forceinline__ int BorderPosition(int i, int len) {
+  return i < R ? i : max(R, len - R) + i - R;
+}
+template <int R>
+__device__ __forceinline__ int BorderIndex(int pos, int len) {
+  return pos < R ? pos : R + pos - max(R, len - R);
+}
+template <int R>
+__device__ __forceinline__ float BorderScale(int i, int len, const float* k) {
+  const int pos = BorderPosition<R>(i, len);
   float weight = 0.0f;
 #pragma unroll
-  for (int i = 0; i <= 2 * R; ++i) {
-    const int sx = pos - R + i;
-    const float next = weight + k[i];
+  for (int t = 0; t <= 2 * R; ++t) {
+    const int sx = pos - R + t;
+    const float next = weight + k[t];
     weight = sx >= 0 && sx < len ? next : weight;
   }
-  const float scale = 1.0f / weight;
-  float v[2 * R + 1];
-#pragma unroll
-  for (int i = 0; i <= 2 * R; ++i) {
-    const int sx = pos - R + i;
-    v[i] = sample(sx < 0 ? 0 : sx < len ? sx : len - 1);
-  }
+  return 1.0f / weight;
+}
+
+// A border output of ConvolutionWithTranspose (fewer than R samples on one
+// side): the taps that fall inside the line, in ascending order, renormalised
+// by `scale`; sample(t) is the sample under tap t (any value outside),
+// inside(t) whether it lies in the line.
+template <int R, typename Sample, typename Inside>
+__device__ __forceinline__ float ConvolveBorder(Sample sample, Inside inside, float scale,
+                                                const float* k) {
   float sum = 0.0f;
 #pragma unroll
-  for (int i = 0; i <= 2 * R; ++i) {
-    const int sx = pos - R + i;
-    const float next = sum + v[i] * k[i];
-    sum = sx >= 0 && sx < len ? next : sum;
+  for (int t = 0; t <= 2 * R; ++t) {
+    const float next = sum + sample(t) * k[t];
+    sum = inside(t) ? next : sum;
   }
   return sum * scale;
 }
 
-// One output of ConvolutionWithTranspose: position `pos` of a line of `len`
-// samples spaced `stride` floats apart.
+// ---- the fused blur ---------------------------------------------------------
+//
+// A work group blurs a strip of kStripW columns by a segment of rows, both
+// passes, without writing the row pass to memory.  It walks down the segment
+// kBandH input rows at a time: the rows and their halo columns go to LDS
+// (`stage`, fetched into registers while the previous band is computed), the
+// row pass leaves them blurred in a ring of the last kGroups bands, and the
+// column pass takes kBandH output rows from the ring.
+//   * Row pass: a lane makes four adjacent outputs from one window of 16-byte
+//     LDS reads (conflict-free).
+//   * Column pass: a lane makes kOut outputs down one column from one window
+//     of kOut + 2R ring rows; the epilogue consumes them (Load(row, x, in)
+//     reads what the split of a pixel needs, Store(row, x, v, in) writes its
+//     results; row, the offset of a whole row, is uniform, so the addresses
+//     are scalar; a lane reads everything before its first store, which may
+//     alias its reads as far as the compiler knows).
+//   * Border rows and columns take the renormalised border convolution, with
+//     the 2R reciprocal weights of each axis computed once per work group.
+// What bounds it: at 12 megapixels the two passes' arithmetic, 2 (3R + 5)
+// operations per output in the reference's order, and the latencies between
+// a band's two barriers; below about two megapixels those latencies alone,
+// which is why 512 lanes share a band (four outputs each) and not 256 (eight):
+// radius 16 at 77x45 34 to 23 us, at 1537x1153 75 to 66, at 4032x3024 250 to
+// 230.  The separate row and column kernels that this replaces wrote and read
+// a plane more per pass, re-read 8 + 2R rows for every eight outputs of a
+// column, and took 22 launches per image and scale pair where this takes
+// four (all four radii at 4032x3024, reference image: 830 to 540 us; whole
+// preparation and comparison at 1537x1153: 1063 to 490).
+constexpr int kStripW = 128, kBandH = 16;
+constexpr int kBlurThreads = 512;
+
 template <int R>
-__device__ __forceinline__ float ConvolveLine(const float* __restrict__ line,
-                                              int stride, int pos, int len,
-                                              const float* __restrict__ taps) {
-  const float* k = taps;
-  const float* sk = taps + 33;
-  const int first = len < R ? len : R;
-  const int last = len > R ? len - R : 0;
-  if (pos >= first && pos < last) {
-    const float* s = line + static_cast<ptrdiff_t>(pos - R) * stride;
-    float window[2 * R + 1];
-#pragma unroll
-    for (int i = 0; i <= 2 * R; ++i) window[i] = s[i * stride];
-    return ConvolveInterior<R>(window, sk);
+struct BlurShape {
+  // samples x - R .. x + 3 + R of a lane's outputs x .. x + 3, whole float4s
+  static constexpr int kWindow = (2 * R + 4 + 3) / 4 * 4;
+  static constexpr int kStageW = kStripW - 4 + kWindow;
+  // bands of rows that an output band needs
+  static constexpr int kGroups = (kBandH + 2 * R + kBandH - 1) / kBandH;
+};
+
+template <int R>
+struct BlurShared {
+  __align__(16) float stage[kBandH][BlurShape<R>::kStageW];
+  __align__(16) float ring[BlurShape<R>::kGroups * kBandH][kStripW];
+  float xscale[2 * R], yscale[2 * R];  // BorderScale of each border index
+  // the unscaled taps, for the border outputs (in scalar registers beside the
+  // scaled ones they spill)
+  float taps[2 * R + 1];
+};
+
+// Fills the border scales; the first barrier of BlurSegment orders them.
+template <int R>
+__device__ __forceinline__ void BlurBegin(BlurShared<R>& sh, int w, int h,
+                                          const Taps& taps) {
+  const int t = threadIdx.x;
+  if (t <= 2 * R) sh.taps[t] = taps.k[t];
+  if (t < 4 * R) {
+    const bool rows = t >= 2 * R;
+    const float scale = BorderScale<R>(rows ? t - 2 * R : t, rows ? h : w, taps.k);
+    (rows ? sh.yscale : sh.xscale)[rows ? t - 2 * R : t] = scale;
   }
-  return ConvolveBorder<R>(
-    [&](int sx) { return line[static_cast<ptrdiff_t>(sx) * stride]; }, pos, len, k);
 }
 
-// Rows: a work group blurs kRowRows rows of kRowSpan pixels, one wave per
-// row, from an LDS copy of the rows and their halo.  Each lane produces four
-// adjacent outputs from one register window that it reads with 16-byte LDS
-// reads (lanes read consecutive 16-byte words: conflict-free).
-constexpr int kRowSpan = 256;
-constexpr int kRowLanes = kRowSpan / 4;
-constexpr int kRowRows = kThreads / kRowLanes;
-
-template <int R>
-__global__ __launch_bounds__(kThreads) void BlurRowsKernel(
-  const float* __restrict__ in, int w, int h, const float* __restrict__ taps,
-  float* __restrict__ out) {
-  // samples x - R .. x + 3 + R of a lane's outputs x .. x + 3, whole float4s
-  constexpr int kWindow = (2 * R + 4 + 3) / 4 * 4;
-  constexpr int kUsed = kRowSpan - 4 + kWindow;
-  // whole loads per lane, so that every load issues before the first store
-  constexpr int kLoads = (kUsed + kRowLanes - 1) / kRowLanes;
-  constexpr int kStride = kLoads * kRowLanes;
-  __shared__ __align__(16) float tile[kRowRows][kStride];
-  const TileIndex tile_index = XcdTile();
-  const int x0 = tile_index.x * kRowSpan;
-  const int row = threadIdx.x / kRowLanes, lane = threadIdx.x % kRowLanes;
-  const int y = tile_index.y * kRowRows + row;
-  // tile column c holds sample x0 - R + c of the row
-  const float* src = in + static_cast<size_t>(y < h ? y : h - 1) * w;
+// Rows y0 .. y1 - 1 (y1 - y0 a multiple of kBandH unless y1 is h) of the
+// columns x0 .. of the planes that `epilogue` names: plane k of its order is
+// epilogue.Input(k), and epilogue.Visit(k, f) calls f with that plane's split.
+//
+// The code is kept small: a work group runs each part of it a few times only,
+// and straight-line code that no wave has run yet comes in at the latency of
+// the instruction fetch.  So the planes share one copy (a uniform switch picks
+// the split), interior outputs are computed for every row and lane, and
+// the border outputs of a column are one rolled loop over the taps.  (Unrolled
+// per plane and output, the 110 KB of the radius-16 kernel made the work groups
+// at an image's border 2.5 times as long as the others.)
+template <int R, int kT, typename Epilogue>
+__device__ __forceinline__ void BlurSegment(BlurShared<R>& sh, int w, int h, int x0, int y0,
+                                            int y1, const Taps& taps, int first_plane,
+                                            int planes, const Epilogue& epilogue) {
+  using S = BlurShape<R>;
+  const float* sk = taps.sk;
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  constexpr int kWaveRows = kBandH / (kT / 64);
+  constexpr int kOut = kStripW * kBandH / kT;  // outputs per lane and pass
+  constexpr int kRowSets = kOut / 4;           // quads of outputs in the row pass
+  constexpr int kRowStep = kBandH / kRowSets;
+  constexpr int kLoads = (S::kStageW + 63) / 64;
+  const int first_x = min(w, R), last_x = max(w - R, 0);
+  const int first_y = min(h, R), last_y = max(h - R, 0);
+  // stage column c holds sample x0 - R + c (clamped into the row: what lies
+  // outside is never used)
+  unsigned column[kLoads];
 #pragma unroll
   for (int k = 0; k < kLoads; ++k) {
-    const int c = lane + k * kRowLanes;
-    const int gx = x0 - R + c;
-    // clamped reads and a select instead of a branch per load
-    const float v = src[gx < 0 ? 0 : gx < w ? gx : w - 1];
-    tile[row][c] = gx >= 0 && gx < w && y < h ? v : 0.0f;
+    column[k] = min(max(x0 - R + min(lane + 64 * k, S::kStageW - 1), 0), w - 1);
   }
-  __syncthreads();
-  if (y >= h) return;
-  const float* line = tile[row];
-  const float* sk = taps + 33;
-  const int first = w < R ? w : R;
-  const int last = w > R ? w - R : 0;
-  // interior outputs: four adjacent ones per lane
-  const int x = x0 + 4 * lane;
-  float* dst = out + static_cast<size_t>(y) * w;
-  if (x >= first && x + 3 < last) {
-    float window[kWindow];
-    const float4* s4 = reinterpret_cast<const float4*>(&line[4 * lane]);
-#pragma unroll
-    for (int m = 0; m < kWindow / 4; ++m) {
-      const float4 v = s4[m];
-      window[4 * m] = v.x;
-      window[4 * m + 1] = v.y;
-      window[4 * m + 2] = v.z;
-      window[4 * m + 3] = v.w;
+  const int bands = (y1 - y0 + kBandH - 1) / kBandH;
+  const int groups = bands + S::kGroups - 1;
+  float next[kWaveRows][kLoads];
+  // group g of plane k; past a plane's last group, the next plane's first
+  auto fetch = [&](int k, int g) {
+    if (g == groups) {
+      ++k;
+      g = 0;
     }
-    float r[4];
+    if (k == planes) return;
+    const float* in = epilogue.Input(k);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = ConvolveInterior<R>(window + j, sk);
-    if ((w & 3) == 0) {
-      // rows start on 16-byte boundaries
-      *reinterpret_cast<float4*>(dst + x) = make_float4(r[0], r[1], r[2], r[3]);
-    } else {
+    for (int r = 0; r < kWaveRows; ++r) {
+      const int y = min(max(y0 - R + kBandH * g + wave * kWaveRows + r, 0), h - 1);
+      const float* row = in + static_cast<size_t>(y) * w;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) dst[x + j] = r[j];
+      for (int c = 0; c < kLoads; ++c) next[r][c] = row[column[c]];
     }
-  } else {
-    // a lane that straddles an end of the interior
+  };
+  // the strip's border columns: `left` from x0, then `right` from right_begin
+  const int left = min(max(first_x - x0, 0), kStripW);
+  const int right_begin = max(max(last_x, first_x), x0);
+  const int border = left + max(min(w, x0 + kStripW) - right_begin, 0);
+  // column pass: this lane's column and its kOut rows of a band
+  const int col = tid % kStripW, part = wave / (kStripW / 64);
+  const unsigned x = x0 + col;
+  fetch(first_plane, 0);
 #pragma unroll 1
-    for (int j = 0; j < 4; ++j) {
-      const int xj = x + j;
-      if (xj >= first && xj < last && xj < w) {
-        dst[xj] = ConvolveInterior<R>(line + 4 * lane + j, sk);
+  for (int k = first_plane; k < planes; ++k) {
+    int slot = 0;  // ring band of group g: g % kGroups
+#pragma unroll 1
+    for (int g = 0; g < groups; ++g) {
+#pragma unroll
+      for (int r = 0; r < kWaveRows; ++r) {
+#pragma unroll
+        for (int c = 0; c < kLoads; ++c) {
+          const int at = lane + 64 * c;
+          if (at < S::kStageW) sh.stage[wave * kWaveRows + r][at] = next[r][c];
+        }
       }
+      __syncthreads();
+      fetch(k, g + 1);
+      {
+        const int q = tid % (kStripW / 4);
+#pragma unroll 1
+        for (int m = 0; m < kRowSets; ++m) {
+          const int row = tid / (kStripW / 4) + m * kRowStep;
+          float window[S::kWindow];
+          const float4* s4 = reinterpret_cast<const float4*>(&sh.stage[row][4 * q]);
+#pragma unroll
+          for (int j = 0; j < S::kWindow / 4; ++j) {
+            const float4 v = s4[j];
+            window[4 * j] = v.x;
+            window[4 * j + 1] = v.y;
+            window[4 * j + 2] = v.z;
+            window[4 * j + 3] = v.w;
+          }
+          float r[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) r[j] = ConvolveInterior<R>(window + j, sk);
+          // (a border column's lane writes its own output after this one)
+          float* ring = &sh.ring[slot * kBandH + row][0];
+          *reinterpret_cast<float4*>(ring + 4 * q) = make_float4(r[0], r[1], r[2], r[3]);
+        }
+      }
+      if (border > 0) {
+        // at most 2R <= 32 border columns, all rows: one lane per output, in
+        // the wave that has written the interior form of the same rows
+        const int b = tid % 32;
+        const int xb = b < left ? x0 + b : right_begin + (b - left);
+        const float scale = sh.xscale[b < border ? BorderIndex<R>(xb, w) : 0];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int m = 0; m < kRowSets; ++m) {
+          const int row = tid / 32 + m * kRowStep;
+          if (b < border) {
+            const float* line = &sh.stage[row][xb - x0];
+            sh.ring[slot * kBandH + row][xb - x0] =
+              ConvolveBorder<R>([&](int t) { return line[t]; },
+                                [&](int t) {
+                                  return static_cast<unsigned>(xb - R + t) <
+                                         static_cast<unsigned>(w);
+                                },
+                                scale, sh.taps);
+          }
+        }
+      }
+      __syncthreads();
+      const int next_slot = slot + 1 == S::kGroups ? 0 : slot + 1;
+      const int yb = y0 + kBandH * (g - (S::kGroups - 1)) + kOut * part;  // wave-uniform
+      if (g >= S::kGroups - 1 && yb < y1 && x < static_cast<unsigned>(w)) {
+        float split[kOut][Epilogue::kLoads];
+        epilogue.Visit(k, [&](auto s) {
+#pragma unroll
+          for (int p = 0; p < kOut; ++p) {
+            s.Load(static_cast<size_t>(min(yb + p, h - 1)) * w, x, split[p]);
+          }
+        });
+        // the oldest band of the ring is the first that this band needs
+        constexpr int kBlocks = (2 * R) / kOut + 1 + ((2 * R) % kOut != 0);
+        constexpr int kBandBlocks = kBandH / kOut;
+        float window[kOut * kBlocks];
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) {
+          int block = kBandBlocks * next_slot + part + j;  // ring rows in blocks of kOut
+          block = block >= kBandBlocks * S::kGroups ? block - kBandBlocks * S::kGroups : block;
+#pragma unroll
+          for (int i = 0; i < kOut; ++i) {
+            if (kOut * j + i < kOut + 2 * R) window[kOut * j + i] = sh.ring[kOut * block + i][col];
+          }
+        }
+        float v[kOut];
+#pragma unroll
+        for (int p = 0; p < kOut; ++p) v[p] = ConvolveInterior<R>(window + p, sk);
+        if (yb < first_y || yb + kOut - 1 >= last_y) {
+          // the taps of all outputs one after another: at tap t output p
+          // needs ring row p + t of the window
+          float sum[kOut] = {}, samples[kOut];
+          auto ring_row = [&](int i) {
+            int r = kBandH * next_slot + kOut * part + i;
+            r = r >= S::kGroups * kBandH ? r - S::kGroups * kBandH : r;
+            return sh.ring[r][col];
+          };
+#pragma unroll
+          for (int p = 0; p < kOut; ++p) samples[p] = ring_row(p);
+#pragma unroll 1
+          for (int t = 0; t <= 2 * R; ++t) {
+            const float after = ring_row(min(kOut + t, kOut - 1 + 2 * R));
+            const float tap = sh.taps[t];
+#pragma unroll
+            for (int p = 0; p < kOut; ++p) {
+              const float moved = sum[p] + samples[p] * tap;
+              const bool inside = static_cast<unsigned>(yb + p - R + t) < static_cast<unsigned>(h);
+              sum[p] = inside ? moved : sum[p];
+              samples[p] = p + 1 < kOut ? samples[p + 1 < kOut ? p + 1 : p] : after;
+            }
+          }
+#pragma unroll
+          for (int p = 0; p < kOut; ++p) {
+            const int y = yb + p;
+            const bool interior = y >= first_y && y < last_y;
+            const float scale = sh.yscale[interior ? 0 : BorderIndex<R>(min(y, h - 1), h)];
+            v[p] = interior ? v[p] : sum[p] * scale;
+          }
+        }
+        epilogue.Visit(k, [&](auto s) {
+#pragma unroll
+          for (int p = 0; p < kOut; ++p) {
+            if (yb + p < y1) s.Store(static_cast<size_t>(yb + p) * w, x, v[p], split[p]);
+          }
+        });
+      }
+      slot = next_slot;
     }
-  }
-  // border outputs (x < first or x >= max(first, last)), one per lane: at
-  // most R at each end of the row
-  const int left = min(max(first - x0, 0), kRowSpan);
-  const int right_begin = max(max(last, first), x0);
-  const int right = max(min(w, x0 + kRowSpan) - right_begin, 0);
-  if (lane < left + right) {
-    const int xb = lane < left ? x0 + lane : right_begin + (lane - left);
-    dst[xb] = ConvolveBorder<R>([&](int sx) { return line[sx - x0 + R]; }, xb, w, taps);
   }
 }
 
-// Columns: each thread produces kColOutputs outputs down one column from
-// one register window (coalesced across the wave).  The epilogue takes the
-// blurred value v of pixel i: a store, or the frequency split that consumes
-// the blur, so that the blurred plane is never written.  `Load(i, src, in)`
-// reads the kLoads values the split of pixel i needs (src: the blur's
-// input plane) and `Store(i, v, in)`
-// writes its results; a thread reads its window and every output's split
-// inputs before it stores anything (its stores may alias its later reads
-// as far as the compiler knows, which would otherwise make each output
-// wait for its own reads).
-constexpr int kColOutputs = 8;
+// ---- launches over both scales ------------------------------------------------
 
-template <int R, typename Epilogue>
-__global__ __launch_bounds__(kThreads) void BlurColsKernel(
-  const float* __restrict__ in, int w, int h, const float* __restrict__ taps,
-  Epilogue epilogue) {
-  constexpr int kOutputs = kColOutputs;
-  // dispatch order (no XCD remap): horizontally adjacent groups read the
-  // same rows, and a band's halo rows are re-read from L2 either way
-  const int x = blockIdx.x * blockDim.x + threadIdx.x, y0 = blockIdx.y * kOutputs;
-  if (x >= w) return;
-  const int first = h < R ? h : R;
-  const int last = h > R ? h - R : 0;
-  if (y0 >= first && y0 + kOutputs - 1 < last) {
-    float window[kOutputs + 2 * R];
-#pragma unroll
-    for (int j = 0; j < kOutputs + 2 * R; ++j) {
-      window[j] = in[static_cast<size_t>(y0 - R + j) * w + x];
-    }
-    float split[kOutputs][Epilogue::kLoads];
-#pragma unroll
-    for (int p = 0; p < kOutputs; ++p) epilogue.Load(static_cast<size_t>(y0 + p) * w + x, in, split[p]);
-    const float* sk = taps + 33;
-#pragma unroll
-    for (int p = 0; p < kOutputs; ++p) {
-      epilogue.Store(static_cast<size_t>(y0 + p) * w + x, ConvolveInterior<R>(window + p, sk),
-                     split[p]);
-    }
-    return;
+// The tiles of the full scale, then those of the half scale, in one
+// one-dimensional grid; within a scale in the XCD-aware order (XcdTile).
+struct ScaleTile {
+  int scale, x, y, unit;
+};
+struct ScaleBlocks {
+  unsigned tiles_w[2] = {1, 1}, count[2] = {0, 0};
+  unsigned units = 1;  // work groups per tile, consecutive
+  dim3 Grid() const { return dim3(count[0] + count[1]); }
+  __device__ __forceinline__ ScaleTile Tile() const {
+    constexpr unsigned kXcds = 8;
+    const int scale = blockIdx.x >= count[0] ? 1 : 0;
+    const unsigned i = blockIdx.x - (scale ? count[0] : 0);
+    const unsigned per = count[scale] / kXcds;
+    const unsigned t = i < per * kXcds ? (i % kXcds) * per + i / kXcds : i;
+    const unsigned tile = t / units;
+    return {scale, static_cast<int>(tile % tiles_w[scale]), static_cast<int>(tile / tiles_w[scale]),
+            static_cast<int>(t % units)};
   }
-  for (int p = 0; p < kOutputs; ++p) {
-    const int y = y0 + p;
-    if (y >= h) break;
-    const size_t i = static_cast<size_t>(y) * w + x;
-    float split[Epilogue::kLoads];
-    epilogue.Load(i, in, split);
-    epilogue.Store(i, ConvolveLine<R>(in + x, w, y, h, taps), split);
-  }
-}
+};
 
 // ---- opsin dynamics ---------------------------------------------------------
 
@@ -295,21 +434,34 @@ __device__ __forceinline__ void Absorbance(float r, float g, float b, bool clamp
 // One work group per 64x16 tile: the three planes' tile with a mirrored
 // 2-pixel halo in LDS, then per pixel the 5-tap horizontal sums of the five
 // rows it needs and their vertical combination, in the reference's order.
+// The half scale's image (SubSample2x of the linear one) is formed as its
+// tiles are read: four reads per sample of an image that the full scale has
+// just pulled into the caches, instead of a launch that wrote and re-read
+// three planes.
 constexpr int kOpsinTileW = 64, kOpsinTileH = 16;
 constexpr int kOpsinRows = kOpsinTileH / (kThreads / kOpsinTileW);  // per thread
 
-// kOnce: w and h are at least 2, so every coordinate of the 2-pixel halo
-// needs one reflection.
-template <bool kOnce>
-__global__ __launch_bounds__(kThreads) void OpsinDynamicsKernel(
-  const float* __restrict__ rgb, int w, int h, float intensity,
-  const float* __restrict__ taps, float* __restrict__ xyb) {
+struct OpsinArgs {
+  ScaleBlocks blocks;
+  const float* rgb;  // the full scale's image
+  int w[2], h[2];
+  float* xyb[2];
+  float intensity;
+  Taps taps;
+  uint32_t* score;  // cleared for the comparison that follows, or null
+};
+
+__global__ __launch_bounds__(kThreads) void OpsinDynamicsKernel(OpsinArgs args) {
   constexpr int TW = kOpsinTileW + 4, TH = kOpsinTileH + 4;
   __shared__ float tile[3][TH][TW];
-  const TileIndex tile_index = XcdTile();
-  const int x0 = tile_index.x * kOpsinTileW, y0 = tile_index.y * kOpsinTileH;
+  const ScaleTile at = args.blocks.Tile();
+  const int x0 = at.x * kOpsinTileW, y0 = at.y * kOpsinTileH;
+  const int w = args.w[at.scale], h = args.h[at.scale];
   const size_t n = static_cast<size_t>(w) * h;
-  auto mirror = [](int c, int size) { return kOnce ? BMirrorOnce(c, size) : BMirror(c, size); };
+  const float intensity = args.intensity;
+  const float* __restrict__ rgb = args.rgb;
+  float* __restrict__ xyb = args.xyb[at.scale];
+  if (args.score != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *args.score = 0;
   // The tile's 3 x TH rows of TW = 64 + 4 columns: each wave reads kWaveRows
   // whole rows, one lane per column of the first 64, with the row address
   // uniform (scalar arithmetic); the last 4 columns of every row are one
@@ -320,20 +472,60 @@ __global__ __launch_bounds__(kThreads) void OpsinDynamicsKernel(
   constexpr int kStripCount = 3 * TH * 4;
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / 64));
-  const int sx = mirror(x0 - 2 + lane, w);
+  const int sx = BMirrorOnce(x0 - 2 + lane, w);
+  const int e = min(static_cast<int>(threadIdx.x), kStripCount - 1);
+  const int strip_c = e / 4 / TH;
+  const int strip_y = BMirrorOnce(y0 - 2 + e / 4 % TH, h);
+  const int strip_x = BMirrorOnce(x0 - 2 + 64 + e % 4, w);
   float rows[kWaveRows];
-#pragma unroll
-  for (int i = 0; i < kWaveRows; ++i) {
-    const int row = wave * kWaveRows + i;
-    const int c = row / TH, r = row % TH;
-    rows[i] = rgb[c * n + static_cast<size_t>(mirror(y0 - 2 + r, h)) * w + sx];
-  }
   float strip;
-  {
-    const int e = min(static_cast<int>(threadIdx.x), kStripCount - 1);
-    const int row = e / 4, c = row / TH, r = row % TH;
-    strip = rgb[c * n + static_cast<size_t>(mirror(y0 - 2 + r, h)) * w +
-                mirror(x0 - 2 + 64 + e % 4, w)];
+  if (at.scale == 0) {
+#pragma unroll
+    for (int i = 0; i < kWaveRows; ++i) {
+      const int row = wave * kWaveRows + i;
+      const int c = row / TH, r = row % TH;
+      rows[i] = rgb[c * n + static_cast<size_t>(BMirrorOnce(y0 - 2 + r, h)) * w + sx];
+    }
+    strip = rgb[strip_c * n + static_cast<size_t>(strip_y) * w + strip_x];
+  } else {
+    const int fw = args.w[0], fh = args.h[0];
+    const size_t fn = static_cast<size_t>(fw) * fh;
+    // the four samples under half-scale sample (x, y) of plane c, clamped
+    // into the image
+    struct Quad {
+      float a, b, d, e;
+    };
+    auto read = [&](int c, int x, int y) {
+      const int x1 = 2 * x + 1 < fw ? 2 * x + 1 : 2 * x;
+      const float* r0 = rgb + c * fn + static_cast<size_t>(2 * y) * fw;
+      const float* r1 = rgb + c * fn + static_cast<size_t>(min(2 * y + 1, fh - 1)) * fw;
+      return Quad{r0[2 * x], r0[x1], r1[2 * x], r1[x1]};
+    };
+    // their sum over the in-image ones, in the reference's order
+    auto sum = [&](Quad q, int x, int y) {
+      // (the empty asm keeps the compiler from moving a read under its select)
+      asm volatile("" : "+v"(q.a), "+v"(q.b), "+v"(q.d), "+v"(q.e));
+      const bool right = 2 * x + 1 < fw, below = 2 * y + 1 < fh;
+      float v = 0.0f + 0.25f * q.a;
+      v = right ? v + 0.25f * q.b : v;
+      const float lower = v + 0.25f * q.d;
+      v = below ? (right ? lower + 0.25f * q.e : lower) : v;
+      if ((fw & 1) && x == w - 1) v *= 2.0f;
+      if ((fh & 1) && y == h - 1) v *= 2.0f;
+      return v;
+    };
+    Quad quads[kWaveRows];
+#pragma unroll
+    for (int i = 0; i < kWaveRows; ++i) {
+      const int row = wave * kWaveRows + i;
+      quads[i] = read(row / TH, sx, BMirrorOnce(y0 - 2 + row % TH, h));
+    }
+    const Quad strip_quad = read(strip_c, strip_x, strip_y);
+#pragma unroll
+    for (int i = 0; i < kWaveRows; ++i) {
+      rows[i] = sum(quads[i], sx, BMirrorOnce(y0 - 2 + (wave * kWaveRows + i) % TH, h));
+    }
+    strip = sum(strip_quad, strip_x, strip_y);
   }
 #pragma unroll
   for (int i = 0; i < kWaveRows; ++i) {
@@ -343,7 +535,7 @@ __global__ __launch_bounds__(kThreads) void OpsinDynamicsKernel(
     (&tile[0][0][0])[(threadIdx.x / 4) * TW + 64 + threadIdx.x % 4] = strip;
   }
   __syncthreads();
-  const float w0 = taps[33 + 2], w1 = taps[33 + 1], w2 = taps[33 + 0];
+  const float w0 = args.taps.sk[2], w1 = args.taps.sk[1], w2 = args.taps.sk[0];
   const int lx = threadIdx.x % kOpsinTileW;
   const int ly0 = (threadIdx.x / kOpsinTileW) * kOpsinRows;
   const int x = x0 + lx;
@@ -413,107 +605,202 @@ __device__ __forceinline__ float AmplifyRange(float v, float width) {
   return v + v;
 }
 
-// Column-pass epilogues of the separable blurs (SeparateFrequencies).
+// The blurs of SeparateFrequencies and their splits.  A blur reads its whole
+// neighbourhood, so no split writes the plane that its blur reads: the MF
+// planes before their blur, the HF planes before theirs and the masking
+// activity before its own are scratch planes.  A split reads kLoads values
+// per pixel; where the second plane of a work group needs the first one's
+// result at the same pixel, the same lane has written it.
 
-// Each split reads kLoads values per pixel with unconditional reads: a
-// value a channel does not use is read from the blur's own input at the
-// same pixel, which the thread's window has just read (no branch around a
-// read, no extra memory traffic).
 struct StoreBlur {
-  static constexpr int kLoads = 1;
   float* out;
-  __device__ __forceinline__ void Load(size_t, const float*, float (&in)[kLoads]) const {
-    in[0] = 0.0f;
-  }
-  __device__ __forceinline__ void Store(size_t i, float v, const float (&)[kLoads]) const {
-    out[i] = v;
+  __device__ __forceinline__ void Load(size_t, unsigned, float* in) const { in[0] = 0.0f; }
+  __device__ __forceinline__ void Store(size_t row, unsigned x, float v, const float*) const {
+    (out + row)[x] = v;
   }
 };
 
-// The LF blur v of channel c: MF = XYB - LF, then the LF plane scaled.  The
-// channels go Y, X, B: Y's LF stays raw until B's pass, which needs it and
-// then scales it.
+// The LF blur v of channel C: MF = XYB - LF, then the LF plane scaled.  Y's
+// LF stays raw until B's pass, which needs it and then scales it.
+template <int C>
 struct LowSplit {
-  static constexpr int kLoads = 2;
-  int c;
   const float* xyb;
-  float* psycho;
+  float* lf;
+  float* mf;
   size_t n;
-  __device__ __forceinline__ void Load(size_t i, const float* blur_in, float (&in)[kLoads]) const {
-    in[0] = xyb[c * n + i];
-    in[1] = (c == 2 ? psycho + n : blur_in)[i];  // raw LF Y for channel 2
+  __device__ __forceinline__ void Load(size_t row, unsigned x, float* in) const {
+    in[0] = (xyb + C * n + row)[x];
+    if constexpr (C == 2) in[1] = (lf + n + row)[x];
   }
-  __device__ __forceinline__ void Store(size_t i, float v, const float (&in)[kLoads]) const {
-    float* lf = psycho;
-    float* mf = psycho + 3 * n;
-    mf[c * n + i] = in[0] - v;
-    if (c == 0) {
-      lf[i] = v * 33.832837186260f;
-    } else if (c == 1) {
-      lf[n + i] = v;
+  __device__ __forceinline__ void Store(size_t row, unsigned x, float v, const float* in) const {
+    (mf + C * n + row)[x] = in[0] - v;
+    if constexpr (C == 0) {
+      (lf + row)[x] = v * 33.832837186260f;
+    } else if constexpr (C == 1) {
+      (lf + n + row)[x] = v;
     } else {
       const float ly = in[1];
-      lf[2 * n + i] = (-0.362267051518f * ly + v) * 49.87984651440f;
-      lf[n + i] = ly * 14.458268100570f;
+      (lf + 2 * n + row)[x] = (-0.362267051518f * ly + v) * 49.87984651440f;
+      (lf + n + row)[x] = ly * 14.458268100570f;
     }
   }
 };
 
-// The 3.22 blur v of MF channel c: HF and MF of channel c; channel 1 also
+// The 3.22 blur v of MF channel C: HF and MF of channel C; channel 1 also
 // applies SuppressXByY to HF X.
+template <int C>
 struct HighSplit {
-  static constexpr int kLoads = 2;
-  int c;
-  float* psycho;
+  const float* raw;  // the MF planes before the blur
+  float* mf;
+  float* hf;
   size_t n;
-  __device__ __forceinline__ void Load(size_t i, const float* blur_in, float (&in)[kLoads]) const {
-    in[0] = (c == 2 ? blur_in : psycho + (3 + c) * n)[i];  // MF of channels 0, 1
-    in[1] = (c == 1 ? psycho + 6 * n : blur_in)[i];        // HF X for channel 1
+  __device__ __forceinline__ void Load(size_t row, unsigned x, float* in) const {
+    in[0] = C == 2 ? 0.0f : (raw + C * n + row)[x];
+    if constexpr (C == 1) in[1] = (hf + row)[x];
   }
-  __device__ __forceinline__ void Store(size_t i, float v, const float (&in)[kLoads]) const {
-    float* mf = psycho + 3 * n;
-    float* hf = psycho + 6 * n;
-    if (c == 2) {
-      mf[2 * n + i] = v;
+  __device__ __forceinline__ void Store(size_t row, unsigned x, float v, const float* in) const {
+    if constexpr (C == 2) {
+      (mf + 2 * n + row)[x] = v;
       return;
     }
     const float high = in[0] - v;
-    hf[c * n + i] = high;
-    mf[c * n + i] = c == 0 ? RemoveRange(v, 0.29f) : AmplifyRange(v, 0.1f);
-    if (c == 1) {
+    (hf + C * n + row)[x] = high;
+    (mf + C * n + row)[x] = C == 0 ? RemoveRange(v, 0.29f) : AmplifyRange(v, 0.1f);
+    if constexpr (C == 1) {
       constexpr float kS = 46.0f, kMin = 0.653020556257f;
       const float scaler = (kS / (high * high + kS)) * (1.0f - kMin) + kMin;
-      hf[i] = scaler * in[1];
+      (hf + row)[x] = scaler * in[1];
     }
   }
 };
 
-// The 1.56 blur v of HF channel c: UHF and HF of channel c.
+// The 1.56 blur v of HF channel C: UHF and HF of channel C; channel 1 also
+// forms the masking activity (CombineChannelsForMasking + DiffPrecompute).
+template <int C>
 struct UltraSplit {
-  static constexpr int kLoads = 1;
-  int c;
-  float* psycho;
+  const float* raw;  // the HF planes before the blur
+  float* hf;
+  float* uhf;
+  float* activity;
   size_t n;
-  __device__ __forceinline__ void Load(size_t i, const float*, float (&in)[kLoads]) const {
-    in[0] = psycho[(6 + c) * n + i];
+  __device__ __forceinline__ void Load(size_t row, unsigned x, float* in) const {
+    in[0] = (raw + C * n + row)[x];
+    if constexpr (C == 1) {
+      in[1] = (uhf + row)[x];
+      in[2] = (hf + row)[x];
+    }
   }
-  __device__ __forceinline__ void Store(size_t i, float v, const float (&in)[kLoads]) const {
-    float* hf = psycho + (6 + c) * n;
-    float* uhf = psycho + (8 + c) * n;
+  __device__ __forceinline__ void Store(size_t row, unsigned x, float v, const float* in) const {
     const float original = in[0];
     float hv = v;
-    if (c == 0) {
-      uhf[i] = RemoveRange(original - hv, 0.04f);
-      hf[i] = RemoveRange(hv, 1.5f);
+    if constexpr (C == 0) {
+      (uhf + row)[x] = RemoveRange(original - hv, 0.04f);
+      (hf + row)[x] = RemoveRange(hv, 1.5f);
     } else {
       hv = MaximumClamp(hv, 28.4691806922f);
       float uv = original - hv;
       uv = MaximumClamp(uv, 5.19175294647f);
-      uhf[i] = uv * 2.69313763794f;
-      hf[i] = AmplifyRange(hv * 2.155f, 0.132f);
+      const float uhf_y = uv * 2.69313763794f;
+      const float hf_y = AmplifyRange(hv * 2.155f, 0.132f);
+      (uhf + n + row)[x] = uhf_y;
+      (hf + n + row)[x] = hf_y;
+      constexpr float kMul = 6.19424080439f;
+      const float bias = kMul * 12.61050594197f;
+      const float sqrt_bias = sqrtf(bias);
+      const float xd = (in[1] + in[2]) * 2.5f;
+      const float yd = uhf_y * 0.4f + hf_y * 0.4f;
+      const float a = sqrtf(xd * xd + yd * yd);
+      (activity + row)[x] = sqrtf(kMul * fabsf(a) + bias) - sqrt_bias;
     }
   }
 };
+
+// One scale of a blur: the planes it reads, the psycho image it writes and
+// the scratch planes that the next blur reads.
+struct BlurScale {
+  const float* in;
+  float* psycho;
+  float* scratch;
+  int w, h;
+  size_t n;
+};
+struct BlurArgs {
+  ScaleBlocks blocks;  // tiles of kStripW columns by `rows` rows
+  BlurScale scale[2];
+  Taps taps;
+  int rows;
+};
+
+// The planes of each blur in the order a work group takes them: the one that
+// stands alone, then the two of which the second needs the first one's result.
+// With two units in the grid, unit 1 takes the first plane and unit 0 the
+// others.
+
+// in: XYB; scratch: the raw MF planes.  X, Y, B.
+struct LowPlanes {
+  static constexpr int kLoads = 2;
+  const BlurScale& s;
+  __device__ __forceinline__ const float* Input(int k) const { return s.in + k * s.n; }
+  template <typename F>
+  __device__ __forceinline__ void Visit(int k, F&& f) const {
+    if (k == 0) f(LowSplit<0>{s.in, s.psycho, s.scratch, s.n});
+    else if (k == 1) f(LowSplit<1>{s.in, s.psycho, s.scratch, s.n});
+    else f(LowSplit<2>{s.in, s.psycho, s.scratch, s.n});
+  }
+};
+
+// in: the raw MF planes; scratch: the raw HF planes.  B, X, Y.
+struct HighPlanes {
+  static constexpr int kLoads = 2;
+  const BlurScale& s;
+  __device__ __forceinline__ const float* Input(int k) const {
+    return s.in + (k == 0 ? 2 : k - 1) * s.n;
+  }
+  template <typename F>
+  __device__ __forceinline__ void Visit(int k, F&& f) const {
+    float* mf = s.psycho + 3 * s.n;
+    if (k == 0) f(HighSplit<2>{s.in, mf, s.scratch, s.n});
+    else if (k == 1) f(HighSplit<0>{s.in, mf, s.scratch, s.n});
+    else f(HighSplit<1>{s.in, mf, s.scratch, s.n});
+  }
+};
+
+// in: the raw HF planes; scratch: the masking activity.  X, Y.
+struct UltraPlanes {
+  static constexpr int kLoads = 3;
+  const BlurScale& s;
+  __device__ __forceinline__ const float* Input(int k) const { return s.in + k * s.n; }
+  template <typename F>
+  __device__ __forceinline__ void Visit(int k, F&& f) const {
+    float* hf = s.psycho + 6 * s.n;
+    float* uhf = s.psycho + 8 * s.n;
+    if (k == 0) f(UltraSplit<0>{s.in, hf, uhf, s.scratch, s.n});
+    else f(UltraSplit<1>{s.in, hf, uhf, s.scratch, s.n});
+  }
+};
+
+// in: the masking activity; scratch: the blurred activity.
+struct MaskPlanes {
+  static constexpr int kLoads = 1;
+  const BlurScale& s;
+  __device__ __forceinline__ const float* Input(int) const { return s.in; }
+  template <typename F>
+  __device__ __forceinline__ void Visit(int, F&& f) const {
+    f(StoreBlur{s.scratch});
+  }
+};
+
+template <int R, int kT, typename Planes, int kPlanes>
+__global__ __launch_bounds__(kT, 4) void BlurKernel(BlurArgs a) {
+  __shared__ BlurShared<R> sh;
+  const ScaleTile t = a.blocks.Tile();
+  const BlurScale s = a.scale[t.scale];
+  const int x0 = t.x * kStripW, y0 = t.y * a.rows;
+  const bool split = a.blocks.units == 2;
+  BlurBegin<R>(sh, s.w, s.h, a.taps);
+  BlurSegment<R, kT>(sh, s.w, s.h, x0, y0, min(y0 + a.rows, s.h), a.taps, split && t.unit == 0 ? 1 : 0,
+                 split && t.unit == 1 ? 1 : kPlanes, Planes{s});
+}
 
 // ---- difference stages -------------------------------------------------------
 
@@ -690,14 +977,40 @@ struct MaltaScales {
 // first three maps read back; without it only the partial sums and the
 // final map are written.
 // Three stages of LDS (34.6 KB) let four work groups share a CU.
+struct DifferencesScale {
+  const float* ps0;
+  const float* ps1;
+  const float* ref_blurred;
+  const float* dist_blurred;
+  const float* mask_y;
+  const float* mask_dc;
+  float* stages;
+  int w, h;
+};
+struct DifferencesArgs {
+  ScaleBlocks blocks;
+  DifferencesScale scale[2];
+  MaltaScales ms;
+  L2Weights lw;
+  float x_multiplier;
+};
 template <bool kKeepStages>
-__global__ __launch_bounds__(kThreads) void DifferencesKernel(
-  const float* __restrict__ ps0, const float* __restrict__ ps1, int w, int h,
-  MaltaScales ms, L2Weights lw, const float* __restrict__ ref_blurred,
-  const float* __restrict__ dist_blurred, const float* __restrict__ mask_y,
-  const float* __restrict__ mask_dc, float x_multiplier, float* __restrict__ stages) {
+__global__ __launch_bounds__(kThreads) void DifferencesKernel(DifferencesArgs args) {
   __shared__ __align__(16) float tile[3][kMaltaLh][kMaltaLw];
-  const TileIndex tile_index = XcdTile();
+  const ScaleTile at = args.blocks.Tile();
+  const DifferencesScale& sc = args.scale[at.scale];
+  const float* __restrict__ ps0 = sc.ps0;
+  const float* __restrict__ ps1 = sc.ps1;
+  const float* __restrict__ ref_blurred = sc.ref_blurred;
+  const float* __restrict__ dist_blurred = sc.dist_blurred;
+  const float* __restrict__ mask_y = sc.mask_y;
+  const float* __restrict__ mask_dc = sc.mask_dc;
+  float* __restrict__ stages = sc.stages;
+  const int w = sc.w, h = sc.h;
+  const MaltaScales& ms = args.ms;
+  const L2Weights& lw = args.lw;
+  const float x_multiplier = args.x_multiplier;
+  const TileIndex tile_index{at.x, at.y};
   const int x0 = tile_index.x * kMaltaTileW, y0 = tile_index.y * kMaltaTileH;
   const size_t n = static_cast<size_t>(w) * h;
   const int tid = threadIdx.x;
@@ -981,22 +1294,6 @@ __global__ __launch_bounds__(kThreads) void DifferencesKernel(
   }
 }
 
-// CombineChannelsForMasking + DiffPrecompute.
-__global__ __launch_bounds__(kThreads) void MaskSourceKernel(
-  const float* __restrict__ ps, size_t n, float* __restrict__ out) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float* hf = ps + 6 * n;
-  const float* uhf = ps + 8 * n;
-  constexpr float kMul = 6.19424080439f;
-  const float bias = kMul * 12.61050594197f;
-  const float sqrt_bias = sqrtf(bias);
-  const float xd = (uhf[i] + hf[i]) * 2.5f;
-  const float yd = uhf[n + i] * 0.4f + hf[n + i] * 0.4f;
-  const float activity = sqrtf(xd * xd + yd * yd);
-  out[i] = sqrtf(kMul * fabsf(activity) + bias) - sqrt_bias;
-}
-
 // StoreMin3 of the reference as selects: the same comparisons decide the
 // same moves, also when m0 <= m1 <= m2 does not hold.
 __device__ __forceinline__ void StoreMin3(float v, float& m0, float& m1, float& m2) {
@@ -1013,10 +1310,26 @@ __device__ __forceinline__ void StoreMin3(float v, float& m0, float& m1, float& 
 
 // FuzzyErosion of the reference's blurred activity, and MaskY / MaskDcY of
 // the result.
-__global__ __launch_bounds__(kThreads) void MaskKernel(
-  const float* __restrict__ in, int w, int h, float* __restrict__ mask,
-  float* __restrict__ mask_y, float* __restrict__ mask_dc) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
+struct MaskScale {
+  const float* in;
+  float* mask;
+  float* mask_y;
+  float* mask_dc;
+  int w, h;
+};
+struct MaskArgs {
+  ScaleBlocks blocks;  // tiles of kThreads pixels of a row
+  MaskScale scale[2];
+};
+__global__ __launch_bounds__(kThreads) void MaskKernel(MaskArgs args) {
+  const ScaleTile tile = args.blocks.Tile();
+  const MaskScale& sc = args.scale[tile.scale];
+  const float* __restrict__ in = sc.in;
+  float* __restrict__ mask = sc.mask;
+  float* __restrict__ mask_y = sc.mask_y;
+  float* __restrict__ mask_dc = sc.mask_dc;
+  const int w = sc.w, h = sc.h;
+  const int x = tile.x * kThreads + threadIdx.x, y = tile.y;
   if (x >= w) return;
   constexpr int s = 3;
   // every neighbour is read (at clamped positions) before the selection,
@@ -1053,31 +1366,6 @@ __global__ __launch_bounds__(kThreads) void MaskKernel(
 }
 
 // ---- scales ------------------------------------------------------------------
-
-__global__ __launch_bounds__(kThreads) void SubsampleKernel(
-  const float* __restrict__ in, int w, int h, float* __restrict__ out) {
-  const int sw = (w + 1) / 2, sh = (h + 1) / 2;
-  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-  const int c = blockIdx.z;
-  if (x >= sw) return;
-  const float* p = in + static_cast<size_t>(c) * w * h;
-  const int x0 = 2 * x, y0 = 2 * y;
-  // the four reads are unconditional (clamped into the image); the sum takes
-  // the in-image ones in the reference's order
-  const bool right = x0 + 1 < w, below = y0 + 1 < h;
-  const size_t r0 = static_cast<size_t>(y0) * w, r1 = static_cast<size_t>(below ? y0 + 1 : y0) * w;
-  const int x1 = right ? x0 + 1 : x0;
-  float a = p[r0 + x0], b = p[r0 + x1], d = p[r1 + x0], e = p[r1 + x1];
-  // (the empty asm keeps the compiler from moving a read under its select)
-  asm volatile("" : "+v"(a), "+v"(b), "+v"(d), "+v"(e));
-  float v = 0.0f + 0.25f * a;
-  v = right ? v + 0.25f * b : v;
-  const float lower = v + 0.25f * d;
-  v = below ? (right ? lower + 0.25f * e : lower) : v;
-  if ((w & 1) && x == sw - 1) v *= 2.0f;
-  if ((h & 1) && y == sh - 1) v *= 2.0f;
-  out[static_cast<size_t>(c) * sw * sh + static_cast<size_t>(y) * sw + x] = v;
-}
 
 // ExpandImage for extents below 8: edge-replicated into ew x eh.
 __global__ __launch_bounds__(kThreads) void ExpandKernel(
@@ -1118,10 +1406,6 @@ __global__ __launch_bounds__(kThreads) void ComposeKernel(
   }
   BlockReduceU32(best, U32Max());
   if (threadIdx.x == 0) atomicMax(score_bits, best[0]);
-}
-
-__global__ void FillWordKernel(uint32_t* p, uint32_t value) {
-  if (threadIdx.x == 0) *p = value;
 }
 
 // ---- a17 reduction ------------------------------------------------------------
@@ -1196,8 +1480,8 @@ __global__ __launch_bounds__(kThreads) void ReduceKernel(
 
 // ---- host side -------------------------------------------------------------------
 
-void HostTaps(float sigma, float* out) {
-  float k[33] = {};
+Taps HostTaps(float sigma) {
+  Taps out{};
   const float scaled = 2.25f * std::fabs(sigma);
   int radius = static_cast<int>(scaled);
   radius = radius < 1 ? 1 : radius;
@@ -1206,13 +1490,13 @@ void HostTaps(float sigma, float* out) {
   // compiler from folding it
   volatile double exponent_scale = -1.0 / (2.0 * sigma * sigma);
   for (int i = -radius; i <= radius; ++i) {
-    k[i + radius] = static_cast<float>(std::exp(exponent_scale * i * i));
+    out.k[i + radius] = static_cast<float>(std::exp(exponent_scale * i * i));
   }
   float full = 0.0f;
-  for (int i = 0; i < size; ++i) full += k[i];
+  for (int i = 0; i < size; ++i) full += out.k[i];
   const float scale = 1.0f / full;
-  for (int i = 0; i < 33; ++i) out[i] = k[i];
-  for (int i = 0; i < 17; ++i) out[33 + i] = i <= radius ? k[i] * scale : 0.0f;
+  for (int i = 0; i <= radius; ++i) out.sk[i] = out.k[i] * scale;
+  return out;
 }
 
 inline dim3 Grid2(int w, int h, int z = 1) {
@@ -1222,66 +1506,116 @@ inline dim3 Grid1(size_t n) {
   return dim3(static_cast<uint32_t>((n + kThreads - 1) / kThreads));
 }
 
-const float* Taps(const GJXLAmdButteraugli* b, ButteraugliSigma s) {
-  return b->taps + s * kTapStride;
+const Taps& TapsOf(ButteraugliSigma s) {
+  static const struct Table {
+    Taps taps[kSigmaCount];
+    Table() {
+      for (int k = 0; k < kSigmaCount; ++k) taps[k] = HostTaps(kSigmas[k]);
+    }
+  } table;
+  return table.taps[s];
 }
 
-template <int R, typename Epilogue>
-GJXLResult Blur(hipStream_t st, const float* in, int w, int h, const float* taps,
-                float* tmp, Epilogue epilogue) {
-  hipLaunchKernelGGL(BlurRowsKernel<R>,
-                     dim3(CeilDiv(static_cast<uint32_t>(w), kRowSpan),
-                          CeilDiv(static_cast<uint32_t>(h), kRowRows)),
-                     dim3(kThreads), 0, st, in, w, h, taps, tmp);
-  hipLaunchKernelGGL((BlurColsKernel<R, Epilogue>),
-                     dim3(CeilDiv(static_cast<uint32_t>(w), kThreads),
-                          CeilDiv(static_cast<uint32_t>(h), kColOutputs)),
-                     dim3(kThreads), 0, st, tmp, w, h, taps, epilogue);
-  return CheckLaunch("BlurKernel");
-}
+int Scales(const GJXLAmdButteraugli* b) { return b->has_subscale ? 2 : 1; }
 
-// Opsin dynamics and frequency separation of `in` into `psycho`.
-GJXLResult Psycho(GJXLAmdButteraugli* b, ButteraugliScale& s, const float* in,
-                  float* psycho) {
-  hipStream_t st = b->device->stream;
-  const int w = s.width, h = s.height;
-  const size_t n = s.n;
-  const dim3 opsin_grid(CeilDiv(static_cast<uint32_t>(w), kOpsinTileW),
-                        CeilDiv(static_cast<uint32_t>(h), kOpsinTileH));
-  if (w >= 2 && h >= 2) {
-    hipLaunchKernelGGL(OpsinDynamicsKernel<true>, opsin_grid, dim3(kThreads), 0, st, in, w, h,
-                       b->params.intensity_target, Taps(b, kSigmaOpsin), s.xyb);
-  } else {
-    hipLaunchKernelGGL(OpsinDynamicsKernel<false>, opsin_grid, dim3(kThreads), 0, st, in, w,
-                       h, b->params.intensity_target, Taps(b, kSigmaOpsin), s.xyb);
+ScaleBlocks Blocks(const GJXLAmdButteraugli* b, uint32_t tile_w, uint32_t tile_h,
+                   unsigned units = 1) {
+  ScaleBlocks r;
+  r.units = units;
+  for (int k = 0; k < Scales(b); ++k) {
+    r.tiles_w[k] = CeilDiv(static_cast<uint32_t>(b->scale[k].width), tile_w);
+    r.count[k] = r.tiles_w[k] * CeilDiv(static_cast<uint32_t>(b->scale[k].height), tile_h) * units;
   }
+  return r;
+}
+
+// The grid of a blur of radius R.  A segment of n bands filters n + kGroups - 1
+// of them by rows and n by columns, so tall segments filter fewer halo rows;
+// but the work groups of a CU end one after another (the oldest is served
+// first) and the last one runs alone, so there must be enough of them:
+// 4-band segments once the image leaves kWorkGroups of those, shorter ones
+// below.  Where even single bands leave CUs idle the planes are split over two
+// work groups (`split`).  Measured, radius 16, us with 1 / 2 / 3 / 4 bands:
+// 1537x1153 75 / 70 / 66 / 76, 4032x3024 319 / 260 / 252 / 230; one and two
+// units at 77x45 32 and 23, at 512x512 33 and 32, at 1537x1153 75 and 80.
+template <int R>
+BlurArgs BlurGrid(const GJXLAmdButteraugli* b, ButteraugliSigma sigma, bool split) {
+  constexpr uint32_t kWorkGroups = BlurShape<R>::kGroups > 2 ? 400 : 700;
+  uint32_t bands = 0;
+  for (int k = 0; k < Scales(b); ++k) {
+    bands += CeilDiv(static_cast<uint32_t>(b->scale[k].width), kStripW) *
+             CeilDiv(static_cast<uint32_t>(b->scale[k].height), kBandH);
+  }
+  const uint32_t per = std::min(4u, std::max(1u, (bands + kWorkGroups / 2) / kWorkGroups));
+  BlurArgs a{};
+  a.rows = static_cast<int>(per * kBandH);
+  a.blocks = Blocks(b, kStripW, per * kBandH, split && bands <= 256 ? 2 : 1);
+  a.taps = TapsOf(sigma);
+  return a;
+}
+
+float* PsychoPlanes(const ButteraugliScale& s, bool reference) {
+  return reference ? s.ref_psycho : s.dist_psycho;
+}
+// Scratch of one pass over an image, in planes that hold nothing then: the
+// raw MF planes, the raw HF planes and the masking activity (the half
+// scale's image is never stored, the full scale's only when it is expanded,
+// and then the opsin kernel has consumed it).
+float* RawMf(const ButteraugliScale& s) { return s.tmp[0]; }
+float* RawHf(const ButteraugliScale& s) { return s.input; }
+float* Activity(const ButteraugliScale& s) { return s.input + 2 * s.n; }
+// The compared image's blurred activity (after the raw MF planes).
+float* DistortedBlurred(const ButteraugliScale& s) { return s.tmp[2]; }
+
+// Opsin dynamics and frequency separation of `in` at both scales into the
+// reference's or the compared image's psycho planes, and their masking
+// activity.
+GJXLResult Psycho(GJXLAmdButteraugli* b, const float* in, bool reference) {
+  hipStream_t st = b->device->stream;
+  OpsinArgs o{};
+  o.blocks = Blocks(b, kOpsinTileW, kOpsinTileH);
+  o.rgb = in;
+  for (int k = 0; k < Scales(b); ++k) {
+    o.w[k] = b->scale[k].width;
+    o.h[k] = b->scale[k].height;
+    o.xyb[k] = b->scale[k].xyb;
+  }
+  o.intensity = b->params.intensity_target;
+  o.taps = TapsOf(kSigmaOpsin);
+  o.score = reference ? nullptr : b->score_bits;
+  hipLaunchKernelGGL(OpsinDynamicsKernel, o.blocks.Grid(), dim3(kThreads), 0, st, o);
   GJXL_AMD_TRY(CheckLaunch("OpsinDynamicsKernel"));
-  // LF of Y, X, B with the MF = XYB - LF split (B's pass scales Y's LF)
-  const int lf_order[3] = {1, 0, 2};
-  for (int c : lf_order) {
-    GJXL_AMD_TRY(Blur<16>(st, s.xyb + c * n, w, h, Taps(b, kSigmaLow), s.tmp[0],
-                          LowSplit{c, s.xyb, psycho, n}));
-  }
-  for (int c = 0; c < 3; ++c) {
-    GJXL_AMD_TRY(Blur<7>(st, psycho + (3 + c) * n, w, h, Taps(b, kSigmaHigh), s.tmp[0],
-                         HighSplit{c, psycho, n}));
-  }
-  for (int c = 0; c < 2; ++c) {
-    GJXL_AMD_TRY(Blur<3>(st, psycho + (6 + c) * n, w, h, Taps(b, kSigmaUltra), s.tmp[0],
-                         UltraSplit{c, psycho, n}));
-  }
-  return GJXL_OK;
+  auto scales = [&](BlurArgs& a, auto in_of, auto scratch_of) {
+    for (int k = 0; k < Scales(b); ++k) {
+      const ButteraugliScale& s = b->scale[k];
+      a.scale[k] = BlurScale{in_of(s), PsychoPlanes(s, reference), scratch_of(s), s.width,
+                             s.height, s.n};
+    }
+  };
+  BlurArgs low = BlurGrid<16>(b, kSigmaLow, true);
+  scales(low, [](const ButteraugliScale& s) { return s.xyb; }, RawMf);
+  hipLaunchKernelGGL((BlurKernel<16, kBlurThreads, LowPlanes, 3>), low.blocks.Grid(), dim3(kBlurThreads), 0, st, low);
+  GJXL_AMD_TRY(CheckLaunch("LowBlurKernel"));
+  BlurArgs high = BlurGrid<7>(b, kSigmaHigh, true);
+  scales(high, RawMf, RawHf);
+  hipLaunchKernelGGL((BlurKernel<7, kBlurThreads, HighPlanes, 3>), high.blocks.Grid(), dim3(kBlurThreads), 0, st, high);
+  GJXL_AMD_TRY(CheckLaunch("HighBlurKernel"));
+  BlurArgs ultra = BlurGrid<3>(b, kSigmaUltra, false);
+  scales(ultra, RawHf, Activity);
+  hipLaunchKernelGGL((BlurKernel<3, kBlurThreads, UltraPlanes, 2>), ultra.blocks.Grid(), dim3(kBlurThreads), 0, st, ultra);
+  return CheckLaunch("UltraBlurKernel");
 }
 
-// Blurred masking activity of a psycho image into `out`.
-GJXLResult MaskActivity(GJXLAmdButteraugli* b, ButteraugliScale& s, const float* psycho,
-                        float* out) {
-  hipStream_t st = b->device->stream;
-  hipLaunchKernelGGL(MaskSourceKernel, Grid1(s.n), dim3(kThreads), 0, st, psycho, s.n,
-                     s.tmp[0]);
-  GJXL_AMD_TRY(CheckLaunch("MaskSourceKernel"));
-  return Blur<6>(st, s.tmp[0], s.width, s.height, Taps(b, kSigmaMask), s.tmp[1],
-                 StoreBlur{out});
+// The blurred masking activity of the image that Psycho has just separated.
+GJXLResult MaskActivity(GJXLAmdButteraugli* b, bool reference) {
+  BlurArgs a = BlurGrid<6>(b, kSigmaMask, false);
+  for (int k = 0; k < Scales(b); ++k) {
+    const ButteraugliScale& s = b->scale[k];
+    a.scale[k] = BlurScale{Activity(s), nullptr, reference ? s.ref_blurred : DistortedBlurred(s),
+                           s.width, s.height, s.n};
+  }
+  hipLaunchKernelGGL((BlurKernel<6, kBlurThreads, MaskPlanes, 1>), a.blocks.Grid(), dim3(kBlurThreads), 0, b->device->stream, a);
+  return CheckLaunch("MaskBlurKernel");
 }
 
 constexpr double kMaltaWeights[6] = {37.0819870399, 8246.75321353, 18.7237414387,
@@ -1292,10 +1626,8 @@ constexpr float kL2[9] = {400.0f, 1.50815703118f, 0.0f, 2150.0f, 10.6195433239f,
                           16.2176043152f, 29.2353797994f, 0.844626970982f,
                           0.703646627719f};
 
-GJXLResult Differences(GJXLAmdButteraugli* b, ButteraugliScale& s, bool keep_stages) {
+GJXLResult Differences(GJXLAmdButteraugli* b, bool keep_stages) {
   hipStream_t st = b->device->stream;
-  const int w = s.width, h = s.height;
-  const size_t n = s.n;
   const float asym = b->params.hf_asymmetry;
   const float sqrt_asym = std::sqrt(asym);
   const double up[6] = {kMaltaWeights[0], kMaltaWeights[1], kMaltaWeights[2] * sqrt_asym,
@@ -1325,22 +1657,22 @@ GJXLResult Differences(GJXLAmdButteraugli* b, ButteraugliScale& s, bool keep_sta
     lw.mf[c] = kL2[3 + c];
     lw.lf[c] = kL2[6 + c];
   }
-  // the difference kernel addresses a plane with 32-bit byte offsets
-  if (static_cast<uint64_t>(w) * h >= (uint64_t{1} << 30)) {
-    return Fail(GJXL_ERROR_UNSUPPORTED, "Butteraugli differences: plane of 2^30 or more pixels");
+  DifferencesArgs args{};
+  args.blocks = Blocks(b, kMaltaTileW, kMaltaTileH);
+  for (int k = 0; k < Scales(b); ++k) {
+    const ButteraugliScale& s = b->scale[k];
+    args.scale[k] = DifferencesScale{s.ref_psycho, s.dist_psycho, s.ref_blurred,
+                                     DistortedBlurred(s), s.mask_y, s.mask_dc, s.stages,
+                                     s.width, s.height};
   }
-  GJXL_AMD_TRY(MaskActivity(b, s, s.dist_psycho, s.tmp[2]));
-  const dim3 tiles(CeilDiv(static_cast<uint32_t>(w), kMaltaTileW),
-                   CeilDiv(static_cast<uint32_t>(h), kMaltaTileH));
+  args.ms = ms;
+  args.lw = lw;
+  args.x_multiplier = b->params.x_multiplier;
   const bool probed = ProbeBegin(b->device, GJXL_AMD_KERNEL_BUTTERAUGLI_DIFFERENCES);
   if (keep_stages) {
-    hipLaunchKernelGGL(DifferencesKernel<true>, tiles, dim3(kThreads), 0, st, s.ref_psycho,
-                       s.dist_psycho, w, h, ms, lw, s.ref_blurred, s.tmp[2], s.mask_y,
-                       s.mask_dc, b->params.x_multiplier, s.stages);
+    hipLaunchKernelGGL(DifferencesKernel<true>, args.blocks.Grid(), dim3(kThreads), 0, st, args);
   } else {
-    hipLaunchKernelGGL(DifferencesKernel<false>, tiles, dim3(kThreads), 0, st, s.ref_psycho,
-                       s.dist_psycho, w, h, ms, lw, s.ref_blurred, s.tmp[2], s.mask_y,
-                       s.mask_dc, b->params.x_multiplier, s.stages);
+    hipLaunchKernelGGL(DifferencesKernel<false>, args.blocks.Grid(), dim3(kThreads), 0, st, args);
   }
   ProbeEnd(b->device, probed);
   return CheckLaunch("DifferencesKernel");
@@ -1353,6 +1685,10 @@ constexpr int kScalePlanes = 3 + 3 + 10 + 10 + 3 + 9 + 3;
 GJXLResult ButteraugliCompare(GJXLAmdButteraugli* b, const float* distorted,
                               float* map_out, bool keep_stages) {
   hipStream_t st = b->device->stream;
+  // the difference kernel addresses a plane with 32-bit byte offsets
+  if (static_cast<uint64_t>(b->scale[0].width) * b->scale[0].height >= (uint64_t{1} << 30)) {
+    return Fail(GJXL_ERROR_UNSUPPORTED, "Butteraugli differences: plane of 2^30 or more pixels");
+  }
   ButteraugliScale& m = b->scale[0];
   const float* main_in = distorted;
   if (b->expanded) {
@@ -1362,21 +1698,15 @@ GJXLResult ButteraugliCompare(GJXLAmdButteraugli* b, const float* distorted,
     GJXL_AMD_TRY(CheckLaunch("ExpandKernel"));
     main_in = m.input;
   }
-  GJXL_AMD_TRY(Psycho(b, m, main_in, m.dist_psycho));
-  GJXL_AMD_TRY(Differences(b, m, keep_stages));
+  GJXL_AMD_TRY(Psycho(b, main_in, false));
+  GJXL_AMD_TRY(MaskActivity(b, false));
+  GJXL_AMD_TRY(Differences(b, keep_stages));
   const float* sub_map = nullptr;
   int sw = 0;
   if (b->has_subscale) {
-    ButteraugliScale& s = b->scale[1];
-    hipLaunchKernelGGL(SubsampleKernel, Grid2(s.width, s.height, 3), dim3(kThreads), 0, st,
-                       distorted, b->width, b->height, s.input);
-    GJXL_AMD_TRY(CheckLaunch("SubsampleKernel"));
-    GJXL_AMD_TRY(Psycho(b, s, s.input, s.dist_psycho));
-    GJXL_AMD_TRY(Differences(b, s, keep_stages));
-    sub_map = s.stages + 8 * s.n;
-    sw = s.width;
+    sub_map = b->scale[1].stages + 8 * b->scale[1].n;
+    sw = b->scale[1].width;
   }
-  hipLaunchKernelGGL(FillWordKernel, dim3(1), dim3(64), 0, st, b->score_bits, 0u);
   hipLaunchKernelGGL(ComposeKernel,
                      dim3(ReductionGroups(static_cast<size_t>(b->width) * b->height)),
                      dim3(kThreads), 0, st,
@@ -1406,7 +1736,7 @@ size_t ButteraugliGeometry(GJXLAmdButteraugli* b, uint32_t width, uint32_t heigh
   b->scale[0].height = mh;
   b->scale[1].width = (static_cast<int>(width) + 1) / 2;
   b->scale[1].height = (static_cast<int>(height) + 1) / 2;
-  size_t floats = kSigmaCount * 64 + static_cast<size_t>(width) * height + 64;
+  size_t floats = static_cast<size_t>(width) * height + 64;
   const int scales = b->has_subscale ? 2 : 1;
   for (int k = 0; k < scales; ++k) {
     auto& s = b->scale[k];
@@ -1418,8 +1748,6 @@ size_t ButteraugliGeometry(GJXLAmdButteraugli* b, uint32_t width, uint32_t heigh
 
 void CarveButteraugli(GJXLAmdButteraugli* b) {
   float* p = static_cast<float*>(b->allocation);
-  b->taps = p;
-  p += kSigmaCount * 64;
   b->score_bits = reinterpret_cast<uint32_t*>(p);
   p += 64;
   b->map = p;
@@ -1448,7 +1776,6 @@ GJXLResult ResizeButteraugli(GJXLAmdButteraugli* b, uint32_t width, uint32_t hei
   if (ButteraugliGeometry(&probe, width, height) > b->capacity_floats) {
     return Fail(GJXL_ERROR_INVALID_ARGUMENT, "extent exceeds the Butteraugli capacity");
   }
-  // the taps stay where they are: they lead the allocation at every extent
   (void)ButteraugliGeometry(b, width, height);
   CarveButteraugli(b);
   b->prepared = false;
@@ -1486,17 +1813,6 @@ GJXLResult gjxl_amd_butteraugli_create(GJXLAmdDevice* device, uint32_t width,
   }
   b->capacity_floats = floats;
   gjxl_amd::CarveButteraugli(b);
-  float host[gjxl_amd::kSigmaCount * 64] = {};
-  for (int k = 0; k < gjxl_amd::kSigmaCount; ++k) {
-    gjxl_amd::HostTaps(gjxl_amd::kSigmas[k], host + k * 64);
-  }
-  r = Check(hipMemcpyAsync(b->taps, host, sizeof(host), hipMemcpyHostToDevice, device->stream),
-            "hipMemcpyAsync(Butteraugli taps)");
-  if (r == GJXL_OK) r = Check(hipStreamSynchronize(device->stream), "hipStreamSynchronize");
-  if (r != GJXL_OK) {
-    gjxl_amd_butteraugli_destroy(b);
-    return r;
-  }
   *out = b;
   return GJXL_OK;
 }
@@ -1520,28 +1836,26 @@ GJXLResult gjxl_amd_butteraugli_prepare(GJXLAmdButteraugli* b,
   using namespace gjxl_amd;
   b->prepared = false;
   hipStream_t st = b->device->stream;
-  for (int k = 0; k < (b->has_subscale ? 2 : 1); ++k) {
-    ButteraugliScale& s = b->scale[k];
-    const float* in = reference_linear;
-    if (k == 0 && b->expanded) {
-      hipLaunchKernelGGL(ExpandKernel, Grid2(s.width, s.height, 3), dim3(kThreads), 0, st,
-                         reference_linear, b->width, b->height, b->xborder, b->yborder,
-                         s.width, s.height, s.input);
-      GJXL_AMD_TRY(CheckLaunch("ExpandKernel"));
-      in = s.input;
-    } else if (k == 1) {
-      hipLaunchKernelGGL(SubsampleKernel, Grid2(s.width, s.height, 3), dim3(kThreads), 0,
-                         st, reference_linear, b->width, b->height, s.input);
-      GJXL_AMD_TRY(CheckLaunch("SubsampleKernel"));
-      in = s.input;
-    }
-    GJXL_AMD_TRY(Psycho(b, s, in, s.ref_psycho));
-    GJXL_AMD_TRY(MaskActivity(b, s, s.ref_psycho, s.ref_blurred));
-    hipLaunchKernelGGL(MaskKernel, Grid2(s.width, s.height), dim3(kThreads), 0, st,
-                       s.ref_blurred, s.width, s.height, s.stages + 6 * s.n, s.mask_y,
-                       s.mask_dc);
-    GJXL_AMD_TRY(CheckLaunch("MaskKernel"));
+  ButteraugliScale& m = b->scale[0];
+  const float* in = reference_linear;
+  if (b->expanded) {
+    hipLaunchKernelGGL(ExpandKernel, Grid2(m.width, m.height, 3), dim3(kThreads), 0, st,
+                       reference_linear, b->width, b->height, b->xborder, b->yborder, m.width,
+                       m.height, m.input);
+    GJXL_AMD_TRY(CheckLaunch("ExpandKernel"));
+    in = m.input;
   }
+  GJXL_AMD_TRY(Psycho(b, in, true));
+  GJXL_AMD_TRY(MaskActivity(b, true));
+  MaskArgs args{};
+  args.blocks = Blocks(b, kThreads, 1);
+  for (int k = 0; k < Scales(b); ++k) {
+    const ButteraugliScale& s = b->scale[k];
+    args.scale[k] = MaskScale{s.ref_blurred, s.stages + 6 * s.n, s.mask_y, s.mask_dc, s.width,
+                              s.height};
+  }
+  hipLaunchKernelGGL(MaskKernel, args.blocks.Grid(), dim3(kThreads), 0, st, args);
+  GJXL_AMD_TRY(CheckLaunch("MaskKernel"));
   b->prepared = true;
   return GJXL_OK;
 }

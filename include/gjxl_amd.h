@@ -91,7 +91,7 @@ enum {
   GJXL_AMD_KERNEL_NONE = 0,
   GJXL_AMD_KERNEL_CANDIDATE_COST = 1,           /* one launch per strategy */
   GJXL_AMD_KERNEL_DC_QUANT = 2,                 /* the DC wavefront */
-  GJXL_AMD_KERNEL_BUTTERAUGLI_DIFFERENCES = 3,  /* one launch per scale */
+  GJXL_AMD_KERNEL_BUTTERAUGLI_DIFFERENCES = 3,  /* both scales */
   GJXL_AMD_KERNEL_COUNT = 4
 };
 enum { GJXL_AMD_PROBE_SLOTS = 64 };

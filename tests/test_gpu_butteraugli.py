@@ -49,6 +49,28 @@ def test_butteraugli_parity(device, w, h):
     b.close()
 
 
+@pytest.mark.parametrize("w,h", [
+    (129, 17),     # one column past a strip, one row past a band; two units
+    (143, 161),    # the border taps of a strip end in the next one
+    (701, 700),    # one unit, one-band segments
+    (1001, 1003),  # two-band segments at radius 16, one-band at the others
+    (1301, 1203),  # three-band and two-band segments
+])
+def test_butteraugli_blur_segments(device, w, h):
+    """The blurs' strips, segments and units against the oracle, bit for bit
+    (4032x3024, four-band segments, is covered by the plain path's digests)."""
+    print(f"butteraugli segments {w}x{h}", flush=True)
+    r, d = _pair(w, h, w + h, 0.04)
+    b = gjxl_amd.Butteraugli(device, w, h)
+    b.prepare(device.array(r))
+    out = device.empty((h, w))
+    b.compare(device.array(d), out)
+    want, want_score = binding.butteraugli_distance(r, d)
+    assert _bits_equal(out.numpy(), want)
+    assert b.score() == want_score
+    b.close()
+
+
 def test_butteraugli_stages(device):
     w, h = 48, 40
     r, d = _pair(w, h, 3)
