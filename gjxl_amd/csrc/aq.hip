@@ -8,15 +8,17 @@
 //   AdjustFieldKernel       AdjustQuantField (adaptive_quantization.cpp:740)
 //   MatrixStatsKernel       X/B matrix-scale statistics (workflow.cpp:1318)
 //   RangeKernel             min/max of the adjusted field
-//   Radix*Kernel            exact median and MAD of the quant field
-//   RawQuantKernel          CreateQuantizerFromField's raw quant
+//   QuantizerKernel, SelectPassKernel, RawQuantKernel
+//                           exact median and MAD of the quant field and
+//                           CreateQuantizerFromField
 //   FinalCflKernel          ComputeFinalColorCorrelationMap (fast LS)
 //   CodeTransformKernel     one transform of ComputeQuantizedCoefficients
 //   DcQuantKernel           prediction-aware DC, weighted predictor,
 //                           evaluated as a wavefront over each DC group
-//   EpfSigmaKernel          ComputeEpfInverseSigma
-//   SmoothDcKernel          SmoothDcCoefficients
+//   BlockFieldsKernel       DC reconstruction, SmoothDcCoefficients,
+//                           ComputeEpfInverseSigma
 //   ReconstructKernel       ReconstructQuantizedCoefficients
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -123,8 +125,41 @@ __global__ __launch_bounds__(1024) void AnchorLayoutKernel(
 
 // ---- per-strategy transform kernels -----------------------------------------
 //
-// Each launch handles the transforms of one strategy (from its list), kK of
-// them per work group, with compile-time extents.
+// A work group handles kK transforms of one strategy (from its list) with
+// compile-time extents.  One launch takes the work groups of all strategies,
+// those of the largest transforms first, and each kernel switches to its
+// strategy's code: seven launches one after another each ended with a wave of
+// few work groups, and in frames below two megapixels none of them filled the
+// chip (coding and reconstruction of a 512x512 frame 214 to 49 us).  All
+// strategies' forms fit the same LDS and registers (at most 40.5 KB and 106
+// VGPRs: four work groups per CU).
+
+// Work groups of each strategy in launch order (32x32 first): stage
+// kStrategyStages - 1 - i ends at end[i].
+struct StageGrid {
+  uint32_t end[kStrategyStages];
+};
+
+// Calls f.operator()<strategy>(work group within the strategy, stage).
+template <typename F>
+__device__ __forceinline__ void DispatchStage(const StageGrid& g, F&& f) {
+  const uint32_t i = blockIdx.x;
+  if (i < g.end[0]) f.template operator()<kDct32x32>(i, 6);
+  else if (i < g.end[1]) f.template operator()<kDct16x32>(i - g.end[0], 5);
+  else if (i < g.end[2]) f.template operator()<kDct32x16>(i - g.end[1], 4);
+  else if (i < g.end[3]) f.template operator()<kDct16x16>(i - g.end[2], 3);
+  else if (i < g.end[4]) f.template operator()<kDct8x16>(i - g.end[3], 2);
+  else if (i < g.end[5]) f.template operator()<kDct16x8>(i - g.end[4], 1);
+  else f.template operator()<kDct8>(i - g.end[5], 0);
+}
+
+// The LDS of a kernel over all strategies: the largest of the strategies'.
+template <template <int> class Shared>
+constexpr size_t SharedBytes() {
+  return std::max({sizeof(Shared<kDct8>), sizeof(Shared<kDct16x8>), sizeof(Shared<kDct8x16>),
+                   sizeof(Shared<kDct16x16>), sizeof(Shared<kDct32x16>),
+                   sizeof(Shared<kDct16x32>), sizeof(Shared<kDct32x32>)});
+}
 
 constexpr int kAqThreads = 256;
 constexpr int kSlots = 3072;
@@ -142,14 +177,14 @@ struct TransformSlot {
   int ok;
 };
 
-// Thread k < kK decodes this group's k-th list entry.
+// Thread k < kK decodes the k-th list entry of work group `group`.
 template <int kK>
-__device__ __forceinline__ void LoadSlots(const uint32_t* __restrict__ entries,
+__device__ __forceinline__ void LoadSlots(uint32_t group, const uint32_t* __restrict__ entries,
                                           uint32_t count,
                                           const uint32_t* __restrict__ offsets, int bw,
                                           TransformSlot* slots) {
   if (threadIdx.x < kK) {
-    const uint32_t idx = blockIdx.x * kK + threadIdx.x;
+    const uint32_t idx = group * kK + threadIdx.x;
     TransformSlot t{0, 0, 0u, 0};
     if (idx < count) {
       const uint32_t packed = entries[idx];
@@ -274,20 +309,38 @@ __device__ __forceinline__ void InverseCols(const double* __restrict__ iv, const
   }
 }
 
-// Forward DCT of the three channels of every transform of one strategy into
-// the coefficient store (3 planes of groups * 65536 floats).
+// Forward DCT of the three channels of every transform into the coefficient
+// store (3 planes of groups * 65536 floats).
+struct AnchorDctArgs {
+  int width, height;
+  size_t store;
+  uint32_t counts[kStrategyStages];
+  size_t capacity;  // of each strategy's list
+};
+
 template <int kStrategy>
-__global__ __launch_bounds__(kAqThreads) void AnchorDctKernel(
-  const float* __restrict__ opsin, int width, int height,
-  const uint32_t* __restrict__ entries, uint32_t count,
-  const uint32_t* __restrict__ offsets, const double* __restrict__ bases,
-  size_t store, float* __restrict__ coefs) {
+struct AnchorDctShared {
+  using S = AnchorShape<kStrategy>;
+  double tmp[S::kK * 3 * S::kH * (S::kW + 1)];
+  float pix[S::kK * 3 * S::kN];  // transposed: [p][x][y]
+  TransformSlot slots[S::kK];
+};
+
+template <int kStrategy>
+__device__ __forceinline__ void AnchorDct(AnchorDctShared<kStrategy>& sh, uint32_t group,
+                                          const uint32_t* __restrict__ entries, uint32_t count,
+                                          const float* __restrict__ opsin,
+                                          const uint32_t* __restrict__ offsets,
+                                          const double* __restrict__ bases,
+                                          float* __restrict__ coefs, const AnchorDctArgs& a) {
   using S = AnchorShape<kStrategy>;
   constexpr int W = S::kW, H = S::kH, N = S::kN, K = S::kK;
-  __shared__ float pix[K * 3 * N];            // transposed: [p][x][y]
-  __shared__ double tmp[K * 3 * H * (W + 1)];
-  __shared__ TransformSlot slots[K];
-  LoadSlots<K>(entries, count, offsets, width / 8, slots);
+  const int width = a.width, height = a.height;
+  const size_t store = a.store;
+  float* pix = sh.pix;
+  double* tmp = sh.tmp;
+  TransformSlot* slots = sh.slots;
+  LoadSlots<K>(group, entries, count, offsets, width / 8, slots);
   __syncthreads();
   const size_t plane = static_cast<size_t>(width) * height;
   for (int e = threadIdx.x; e < K * 3 * N; e += kAqThreads) {
@@ -303,6 +356,20 @@ __global__ __launch_bounds__(kAqThreads) void AnchorDctKernel(
   ForwardCols<W, H, 3 * K>(bases + BasisOffsetT(H), tmp, [&](int p, int i, float v) {
     const TransformSlot& t = slots[p / 3];
     if (t.ok) coefs[(p % 3) * store + t.offset + i] = v;
+  });
+}
+
+// (The buffers are arguments of their own: as members of a struct they lose
+// their __restrict__, and with it the scalar loads of the bases.)
+__global__ __launch_bounds__(kAqThreads) void AnchorDctKernel(
+  StageGrid grid, AnchorDctArgs a, const float* __restrict__ opsin,
+  const uint32_t* __restrict__ entries, const uint32_t* __restrict__ offsets,
+  const double* __restrict__ bases, float* __restrict__ coefs) {
+  __shared__ __align__(16) unsigned char lds[SharedBytes<AnchorDctShared>()];
+  DispatchStage(grid, [&]<int kStrategy>(uint32_t group, int stage) __attribute__((always_inline)) {
+    AnchorDct<kStrategy>(*reinterpret_cast<AnchorDctShared<kStrategy>*>(lds), group,
+                         entries + stage * a.capacity, a.counts[stage], opsin, offsets, bases,
+                         coefs, a);
   });
 }
 
@@ -387,62 +454,63 @@ __global__ __launch_bounds__(256) void RangeKernel(const float* __restrict__ v,
 }
 
 // ---- exact median / MAD (radix select on non-negative float bits) ----------
+//
+// The median of the field, then the median of the absolute deviations from
+// it, by radix selection on the float bits in digits of 11, 11 and 10 bits;
+// then the quantizer's parameters and the raw quant of every block
+// (CreateQuantizerFromField).  The work is tiny and what it costs is launches
+// and their gaps, so a field that fits the registers of one work group is one
+// launch, and a larger one takes one launch per digit, whose last work group
+// to finish picks the digit.  (Before: 21 launches of 2 to 7 us for any size,
+// 135 us at 4032x3024 and 90 us at 512x512; now 54 and 16.)
 
-// state: [0] prefix, [1] k (rank within the prefix), [2] median bits,
-// [3..] unused; hist: 256 counters.
-__device__ __forceinline__ uint32_t SelectKey(const float* v, size_t i,
-                                              int pass_kind, uint32_t median) {
-  if (pass_kind == 0) return __float_as_uint(v[i]);
-  return __float_as_uint(fabsf(v[i] - __uint_as_float(median)));
+constexpr int kSelectThreads = 1024;
+constexpr int kSelectBins = 2048;
+constexpr int kSelectKeys = 16;  // per thread of the one-group form
+constexpr size_t kSelectOneGroup = static_cast<size_t>(kSelectThreads) * kSelectKeys;
+constexpr int kSelectPasses = 3;
+constexpr int kSelectBatch = 4;  // blocks per thread and step of the larger form
+__host__ __device__ constexpr int SelectShift(int pass) { return pass == 0 ? 21 : pass == 1 ? 10 : 0; }
+__host__ __device__ constexpr int SelectBits(int pass) { return pass == 2 ? 10 : 11; }
+
+struct SelectState {
+  uint32_t prefix;   // the digits picked so far
+  uint32_t k;        // rank within the prefix
+  uint32_t median, mad;
+  uint32_t arrived;  // work groups that have added their counts; zero between launches
+};
+constexpr int kSelectStateWords = 16;
+static_assert(sizeof(SelectState) <= 4 * kSelectStateWords, "state in front of the counters");
+static_assert(kSelectScratchWords == kSelectStateWords + kSelectBins, "scratch size");
+
+__device__ __forceinline__ uint32_t SelectKey(float v, bool deviation, uint32_t median) {
+  return __float_as_uint(deviation ? fabsf(v - __uint_as_float(median)) : v);
+}
+__device__ __forceinline__ bool SelectMatches(uint32_t key, uint32_t prefix, int pass) {
+  return pass == 0 || (key ^ prefix) >> (SelectShift(pass) + SelectBits(pass)) == 0;
+}
+__device__ __forceinline__ int SelectDigit(uint32_t key, int pass) {
+  return (key >> SelectShift(pass)) & ((1 << SelectBits(pass)) - 1);
 }
 
-__global__ __launch_bounds__(256) void RadixHistogramKernel(
-  const float* __restrict__ v, size_t n, int shift, int pass_kind,
-  const uint32_t* __restrict__ state, uint32_t* __restrict__ hist) {
-  __shared__ uint32_t local[256];
-  local[threadIdx.x] = 0;
-  __syncthreads();
-  const uint32_t prefix = state[0];
-  const uint32_t mask = shift == 24 ? 0u : (0xffffffffu << (shift + 8));
-  for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const uint32_t key = SelectKey(v, i, pass_kind, state[2]);
-    if ((key & mask) == (prefix & mask)) atomicAdd(&local[(key >> shift) & 255], 1u);
+// The digit that holds rank k, from two counts per thread: hands found(digit,
+// rank within it) to the one thread that owns it.  Every thread calls it.
+template <typename Found>
+__device__ __forceinline__ void SelectPick(uint32_t c0, uint32_t c1, uint32_t k, Found found) {
+  uint32_t total;
+  const uint32_t before = BlockExclusiveScanU32(c0 + c1, &total);
+  const int digit = 2 * static_cast<int>(threadIdx.x);
+  if (k >= before && k - before < c0) {
+    found(digit, k - before);
+  } else if (k >= before + c0 && k - before - c0 < c1) {
+    found(digit + 1, k - before - c0);
   }
-  __syncthreads();
-  if (local[threadIdx.x]) atomicAdd(&hist[threadIdx.x], local[threadIdx.x]);
-}
-
-__global__ void RadixPickKernel(uint32_t* __restrict__ hist, int shift,
-                                int pass_kind, uint32_t* __restrict__ state) {
-  if (threadIdx.x != 0) return;
-  uint32_t k = state[1];
-  uint32_t bin = 0;
-  for (; bin < 256; ++bin) {
-    if (k < hist[bin]) break;
-    k -= hist[bin];
-  }
-  state[0] |= bin << shift;
-  state[1] = k;
-  for (int i = 0; i < 256; ++i) hist[i] = 0;
-  if (shift == 0 && pass_kind == 0) state[2] = state[0];  // median found
-  if (shift == 0 && pass_kind == 1) state[3] = state[0];  // MAD found
-}
-
-__global__ void RadixResetKernel(uint32_t* state, uint32_t k, int pass_kind) {
-  state[0] = 0;
-  state[1] = k;
-  (void)pass_kind;
 }
 
 // ComputeQuantizerParams + Quantizer::Create (src/codec/quantization.cpp:
-// 59-115, core/quantizer.h:33-82), one thread.
-__global__ void QuantizerParamsKernel(const uint32_t* __restrict__ state,
-                                      float quant_dc,
-                                      QuantizerState* __restrict__ out) {
-  if (threadIdx.x != 0) return;
-  const float median = __uint_as_float(state[2]);
-  const float mad = __uint_as_float(state[3]);
+// 59-115, core/quantizer.h:33-82).
+__device__ __forceinline__ QuantizerState QuantizerParams(float median, float mad,
+                                                          float quant_dc) {
   float scale = 65536.0f * (median - mad) / 5.0f;
   scale = scale < 1.0f ? 1.0f : (32768.0f < scale ? 32768.0f : scale);
   int32_t global_scale = static_cast<int32_t>(scale);
@@ -463,7 +531,135 @@ __global__ void QuantizerParamsKernel(const uint32_t* __restrict__ state,
     q.dc_steps[c] = inv_qdc / kInvDc[c];
     q.inverse_dc_steps[c] = kInvDc[c] * q.scale * static_cast<float>(qdc);
   }
-  *out = q;
+  return q;
+}
+
+__device__ __forceinline__ int32_t RawQuant(float field, float inverse_global_scale) {
+  float r = field * inverse_global_scale + 0.5f;
+  r = r < 1.0f ? 1.0f : (256.0f < r ? 256.0f : r);
+  return static_cast<int32_t>(r);
+}
+
+// The whole quantizer of a field of at most kSelectOneGroup blocks.
+__global__ __launch_bounds__(kSelectThreads) void QuantizerKernel(
+  const float* __restrict__ field, int n, float quant_dc, QuantizerState* __restrict__ q,
+  int32_t* __restrict__ raw) {
+  __shared__ uint32_t hist[kSelectBins];
+  __shared__ uint32_t prefix, rank;
+  const int t = threadIdx.x;
+  float v[kSelectKeys];
+#pragma unroll
+  for (int j = 0; j < kSelectKeys; ++j) {
+    const int i = t + j * kSelectThreads;
+    v[j] = field[i < n ? i : n - 1];
+  }
+  uint32_t median = 0, mad = 0;
+#pragma unroll 1
+  for (int kind = 0; kind < 2; ++kind) {
+    if (t == 0) {
+      prefix = 0;
+      rank = static_cast<uint32_t>(n / 2);
+    }
+#pragma unroll 1
+    for (int pass = 0; pass < kSelectPasses; ++pass) {
+      hist[2 * t] = 0;
+      hist[2 * t + 1] = 0;
+      __syncthreads();
+      const uint32_t high = prefix, k = rank;
+#pragma unroll
+      for (int j = 0; j < kSelectKeys; ++j) {
+        const uint32_t key = SelectKey(v[j], kind == 1, median);
+        if (t + j * kSelectThreads < n && SelectMatches(key, high, pass)) {
+          atomicAdd(&hist[SelectDigit(key, pass)], 1u);
+        }
+      }
+      __syncthreads();
+      SelectPick(hist[2 * t], hist[2 * t + 1], k, [&](int digit, uint32_t r) {
+        prefix = high | static_cast<uint32_t>(digit) << SelectShift(pass);
+        rank = r;
+      });
+      __syncthreads();
+    }
+    (kind == 0 ? median : mad) = prefix;
+    __syncthreads();
+  }
+  const QuantizerState state =
+    QuantizerParams(__uint_as_float(median), __uint_as_float(mad), quant_dc);
+  if (t == 0) *q = state;
+#pragma unroll
+  for (int j = 0; j < kSelectKeys; ++j) {
+    const int i = t + j * kSelectThreads;
+    if (i < n) raw[i] = RawQuant(v[j], state.inverse_global_scale);
+  }
+}
+
+// One digit of a larger field.  Counts go to `hist` in device memory, all
+// zero between launches; the last work group to arrive picks the digit, clears
+// the counts and after the last digit forms the quantizer.
+__global__ __launch_bounds__(kSelectThreads) void SelectPassKernel(
+  const float* __restrict__ field, size_t n, int kind, int pass, float quant_dc,
+  SelectState* __restrict__ state, uint32_t* __restrict__ hist, QuantizerState* __restrict__ q) {
+  __shared__ uint32_t local[kSelectBins];
+  __shared__ bool last;
+  const int t = threadIdx.x;
+  local[2 * t] = 0;
+  local[2 * t + 1] = 0;
+  __syncthreads();
+  const uint32_t high = pass == 0 ? 0u : state->prefix;
+  const uint32_t k = pass == 0 ? static_cast<uint32_t>(n / 2) : state->k;
+  const uint32_t median = kind == 1 ? state->median : 0u;
+  const size_t step = static_cast<size_t>(gridDim.x) * kSelectThreads;
+  for (size_t i = static_cast<size_t>(blockIdx.x) * kSelectThreads + t; i < n;
+       i += kSelectBatch * step) {
+    float v[kSelectBatch];
+#pragma unroll
+    for (int j = 0; j < kSelectBatch; ++j) v[j] = field[i + j * step < n ? i + j * step : i];
+#pragma unroll
+    for (int j = 0; j < kSelectBatch; ++j) {
+      const uint32_t key = SelectKey(v[j], kind == 1, median);
+      if (i + j * step < n && SelectMatches(key, high, pass)) {
+        atomicAdd(&local[SelectDigit(key, pass)], 1u);
+      }
+    }
+  }
+  __syncthreads();
+  // Everything that crosses work groups is an atomic at device scope, in the
+  // order that waiting for its result gives; a fence there would write the
+  // whole L2 back (23 us a launch instead of 8).
+  uint32_t added = 0;
+  for (int b = 2 * t; b < 2 * t + 2; ++b) {
+    if (local[b]) {
+      added += __hip_atomic_fetch_add(&hist[b], local[b], __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" : : "v"(added) : "memory");
+  __syncthreads();
+  if (t == 0) {
+    last = __hip_atomic_fetch_add(&state->arrived, 1u, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x;
+  }
+  __syncthreads();
+  if (!last) return;
+  uint32_t c[2];
+  for (int b = 0; b < 2; ++b) {
+    c[b] = __hip_atomic_load(&hist[2 * t + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    hist[2 * t + b] = 0;
+  }
+  if (t == 0) state->arrived = 0;
+  SelectPick(c[0], c[1], k, [&](int digit, uint32_t r) {
+    const uint32_t value = high | static_cast<uint32_t>(digit) << SelectShift(pass);
+    state->prefix = value;
+    state->k = r;
+    if (pass + 1 == kSelectPasses) {
+      if (kind == 0) {
+        state->median = value;
+      } else {
+        state->mad = value;
+        *q = QuantizerParams(__uint_as_float(median), __uint_as_float(value), quant_dc);
+      }
+    }
+  });
 }
 
 __global__ __launch_bounds__(256) void RawQuantKernel(
@@ -471,9 +667,7 @@ __global__ __launch_bounds__(256) void RawQuantKernel(
   int32_t* __restrict__ raw) {
   const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float r = field[i] * q->inverse_global_scale + 0.5f;
-  r = r < 1.0f ? 1.0f : (256.0f < r ? 256.0f : r);
-  raw[i] = static_cast<int32_t>(r);
+  raw[i] = RawQuant(field[i], q->inverse_global_scale);
 }
 
 // ---- final CfL, fast least squares (chroma_from_luma.cpp:543-670, :112-
@@ -813,32 +1007,59 @@ __device__ void AdjustQuantDecide(float err_sum, float val_sum, const float (&nz
   *raw_quant = adjusted;
 }
 
-// One launch per strategy: kK transforms per work group.  All threads form
+// kK transforms per work group.  All threads form
 // the terms of the AdjustQuantForChannel scans, three threads per transform
 // run their ordered sums and decisions, one thread per transform decides the
 // shared raw quant and converts the DC values, and all threads quantise.
+struct CodeArgs {
+  size_t store, dc_plane;
+  int bw;
+  uint32_t counts[kStrategyStages];
+  size_t capacity;  // of each strategy's list
+  CodingParams params;
+};
+
 template <int kStrategy>
-__global__ __launch_bounds__(kAqThreads) void CodeTransformKernel(
-  const float* __restrict__ coefs, size_t store, const uint32_t* __restrict__ entries,
-  uint32_t count, const uint32_t* __restrict__ offsets, int bw,
+struct CodeShared {
+  using S = AnchorShape<kStrategy>;
+  static constexpr int K = S::kK, N = S::kN;
+  float2 terms[K][3][N];
+  float coef[K][3][N];
+  float chain_sum[K][3][kScanChains];
+  float chain_max[K][3][4];
+  float thr_y[K][4];
+  int32_t cand[K][3];
+  int32_t decided[K];
+  float cfl[K][2];
+  TransformSlot slots[K];
+  int32_t raw_k[K];
+};
+
+template <int kStrategy>
+__device__ __forceinline__ void CodeTransform(
+  CodeShared<kStrategy>& sh, uint32_t group, const uint32_t* __restrict__ entries, uint32_t count,
+  const float* __restrict__ coefs, const uint32_t* __restrict__ offsets,
   int32_t* __restrict__ raw, const int8_t* __restrict__ y_to_x,
   const int8_t* __restrict__ y_to_b, const QuantizerState* __restrict__ qstate,
-  const float* __restrict__ tables, CodingParams params,
-  int32_t* __restrict__ quantized, float* __restrict__ dc, size_t dc_plane) {
+  const float* __restrict__ tables, int32_t* __restrict__ quantized, float* __restrict__ dc,
+  const CodeArgs& a) {
   using S = AnchorShape<kStrategy>;
   constexpr int W = S::kW, H = S::kH, N = S::kN, K = S::kK;
   constexpr int cols = W > H ? W : H, rows = W > H ? H : W;
-  __shared__ float coef[K][3][N];
-  __shared__ float2 terms[K][3][N];
-  __shared__ float chain_sum[K][3][kScanChains];
-  __shared__ float chain_max[K][3][4];
-  __shared__ float thr_y[K][4];
-  __shared__ int32_t cand[K][3];
-  __shared__ int32_t decided[K];
-  __shared__ float cfl[K][2];
-  __shared__ TransformSlot slots[K];
-  __shared__ int32_t raw_k[K];
-  LoadSlots<K>(entries, count, offsets, bw, slots);
+  const size_t store = a.store, dc_plane = a.dc_plane;
+  const int bw = a.bw;
+  const CodingParams& params = a.params;
+  auto& coef = sh.coef;
+  auto& terms = sh.terms;
+  auto& chain_sum = sh.chain_sum;
+  auto& chain_max = sh.chain_max;
+  auto& thr_y = sh.thr_y;
+  auto& cand = sh.cand;
+  auto& decided = sh.decided;
+  auto& cfl = sh.cfl;
+  auto& slots = sh.slots;
+  auto& raw_k = sh.raw_k;
+  LoadSlots<K>(group, entries, count, offsets, bw, slots);
   __syncthreads();
   const QuantizerState q = *qstate;
   // every global read that depends only on the slots, issued together: the
@@ -1010,6 +1231,20 @@ __global__ __launch_bounds__(kAqThreads) void CodeTransformKernel(
   }
 }
 
+__global__ __launch_bounds__(kAqThreads) void CodeTransformKernel(
+  StageGrid grid, CodeArgs a, const float* __restrict__ coefs,
+  const uint32_t* __restrict__ entries, const uint32_t* __restrict__ offsets,
+  int32_t* __restrict__ raw, const int8_t* __restrict__ y_to_x,
+  const int8_t* __restrict__ y_to_b, const QuantizerState* __restrict__ qstate,
+  const float* __restrict__ tables, int32_t* __restrict__ quantized, float* __restrict__ dc) {
+  __shared__ __align__(16) unsigned char lds[SharedBytes<CodeShared>()];
+  DispatchStage(grid, [&]<int kStrategy>(uint32_t group, int stage) __attribute__((always_inline)) {
+    CodeTransform<kStrategy>(*reinterpret_cast<CodeShared<kStrategy>*>(lds), group,
+                             entries + stage * a.capacity, a.counts[stage], coefs, offsets, raw,
+                             y_to_x, y_to_b, qstate, tables, quantized, dc, a);
+  });
+}
+
 // ---- prediction-aware DC with the weighted predictor ----------------------
 //
 // src/codec/vardct/dc_quantization.cpp:121-240 with
@@ -1036,6 +1271,7 @@ __global__ __launch_bounds__(kAqThreads) void CodeTransformKernel(
 // the Y wave of its row wrote into a per-row LDS ring D steps earlier.
 
 constexpr int kDcGroup = 256;
+constexpr int kDcExtraPrecision = 1;
 constexpr int kDcBatch = 8;            // steps per barrier (D)
 constexpr int kDcEdgeRing = 32;        // > 2D + 2 slots of a band edge
 constexpr int kDcYRing = 16;           // >= 2D slots of quantized Y per row
@@ -1443,82 +1679,125 @@ __global__ __launch_bounds__(256) void DcReconstructKernel(
   }
 }
 
-// ComputeEpfInverseSigma (src/codec/epf.cpp:207-290), neutral sharpness.
-__global__ __launch_bounds__(256) void EpfSigmaKernel(
-  const uint8_t* __restrict__ cells, int bw, int bh,
-  const int32_t* __restrict__ raw, const QuantizerState* __restrict__ q,
-  float* __restrict__ out) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-  if (x >= bw) return;
-  const uint8_t c = cells[static_cast<size_t>(y) * bw + x];
-  if (!(c & 1)) return;
-  const float sigma_quant =
-    0.46f / (q->scale * static_cast<float>(raw[static_cast<size_t>(y) * bw + x]) *
-             -1.1715728752538099024f);
-  float sigma = sigma_quant * (4.0f / 7.0f);
-  sigma = DStdMin(-1.0e-4f, sigma);
-  const float value = 1.0f / sigma;
-  const int cw = CoveredW(c >> 1), ch = CoveredH(c >> 1);
-  for (int dy = 0; dy < ch; ++dy)
-    for (int dx = 0; dx < cw; ++dx) out[static_cast<size_t>(y + dy) * bw + x + dx] = value;
-}
-
-// SmoothDcCoefficients (src/codec/dc_smoothing.cpp).
-__global__ __launch_bounds__(256) void SmoothDcKernel(
-  const float* __restrict__ dc, int bw, int bh,
-  const QuantizerState* __restrict__ qstate, float* __restrict__ out) {
+// What a frame's reconstruction needs of its blocks, one thread per block, in
+// one launch: the reconstructed DC (DcReconstructKernel's, formed again for the
+// neighbours instead of read back), SmoothDcCoefficients (src/codec/
+// dc_smoothing.cpp) and, per anchor, ComputeEpfInverseSigma (src/codec/epf.cpp:
+// 207-290, neutral sharpness).
+__global__ __launch_bounds__(256) void BlockFieldsKernel(
+  const int32_t* __restrict__ quantized, int bw, int bh,
+  const QuantizerState* __restrict__ qstate, int extra_precision,
+  const uint8_t* __restrict__ cells, const int32_t* __restrict__ raw,
+  float* __restrict__ reconstructed, float* __restrict__ smoothed_out,
+  float* __restrict__ inverse_sigma) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
   if (x >= bw) return;
   const size_t n = static_cast<size_t>(bw) * bh;
   const size_t i = static_cast<size_t>(y) * bw + x;
-  if (y == 0 || x == 0 || y + 1 >= bh || x + 1 >= bw) {
-    for (int c = 0; c < 3; ++c) out[c * n + i] = dc[c * n + i];
-    return;
-  }
-  constexpr float kSide = 0.20345139757231578f, kCorner = 0.0334829185968739f;
+  const QuantizerState q = *qstate;
+  const float precision = static_cast<float>(1u << extra_precision);
+  // the 3x3 neighbourhood, clamped into the frame, then its DC values
+  int32_t qv[3][3][3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+      for (int dx = 0; dx < 3; ++dx) {
+        const int yy = min(max(y + dy - 1, 0), bh - 1), xx = min(max(x + dx - 1, 0), bw - 1);
+        qv[c][dy][dx] = quantized[c * n + static_cast<size_t>(yy) * bw + xx];
+      }
+  const uint8_t cell = cells[i];
+  const int32_t raw_quant = raw[i];
+  float dc[3][3][3];
+#pragma unroll
+  for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx) {
+      const float ry = static_cast<float>(qv[1][dy][dx]) * (q.dc_steps[1] / precision);
+      dc[1][dy][dx] = ry;
+      dc[0][dy][dx] = static_cast<float>(qv[0][dy][dx]) * (q.dc_steps[0] / precision);
+      dc[2][dy][dx] =
+        __builtin_fmaf(ry, 1.0f, static_cast<float>(qv[2][dy][dx]) * (q.dc_steps[2] / precision));
+    }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) reconstructed[c * n + i] = dc[c][1][1];
+  const bool edge = y == 0 || x == 0 || y + 1 >= bh || x + 1 >= bw;
+  constexpr float kSide = 0.20345139757231578f, kCorner = 0.0334829185966739f;
   constexpr float kCenter = 1.0f - 4.0f * (kSide + kCorner);
-  float center[3], smoothed[3];
+  float smoothed[3];
   float gap = 0.5f;
+#pragma unroll
   for (int c = 0; c < 3; ++c) {
-    const float* top = dc + c * n + static_cast<size_t>(y - 1) * bw;
-    const float* row = dc + c * n + static_cast<size_t>(y) * bw;
-    const float* bottom = dc + c * n + static_cast<size_t>(y + 1) * bw;
-    const float corners = (top[x - 1] + top[x + 1]) + (bottom[x - 1] + bottom[x + 1]);
-    const float sides = (row[x - 1] + row[x + 1]) + (top[x] + bottom[x]);
-    center[c] = row[x];
+    const float corners = (dc[c][0][0] + dc[c][0][2]) + (dc[c][2][0] + dc[c][2][2]);
+    const float sides = (dc[c][1][0] + dc[c][1][2]) + (dc[c][0][1] + dc[c][2][1]);
     smoothed[c] = __builtin_fmaf(corners, kCorner,
-                                 __builtin_fmaf(sides, kSide, row[x] * kCenter));
-    gap = DStdMax(gap, fabsf((row[x] - smoothed[c]) / qstate->dc_steps[c]));
+                                 __builtin_fmaf(sides, kSide, dc[c][1][1] * kCenter));
+    gap = DStdMax(gap, fabsf((dc[c][1][1] - smoothed[c]) / q.dc_steps[c]));
   }
   const float factor = DStdMax(0.0f, __builtin_fmaf(-4.0f, gap, 3.0f));
+#pragma unroll
   for (int c = 0; c < 3; ++c) {
-    out[c * n + i] = __builtin_fmaf(smoothed[c] - center[c], factor, center[c]);
+    const float center = dc[c][1][1];
+    smoothed_out[c * n + i] =
+      edge ? center : __builtin_fmaf(smoothed[c] - center, factor, center);
   }
+  if (!(cell & 1)) return;
+  const float sigma_quant =
+    0.46f / (q.scale * static_cast<float>(raw_quant) * -1.1715728752538099024f);
+  float sigma = sigma_quant * (4.0f / 7.0f);
+  sigma = DStdMin(-1.0e-4f, sigma);
+  const float value = 1.0f / sigma;
+  const int cw = CoveredW(cell >> 1), ch = CoveredH(cell >> 1);
+  for (int dy = 0; dy < ch; ++dy)
+    for (int dx = 0; dx < cw; ++dx)
+      inverse_sigma[static_cast<size_t>(y + dy) * bw + x + dx] = value;
 }
 
-// ReconstructQuantizedCoefficients (src/codec/reconstruction.cpp:790-936),
-// one launch per strategy: dequantise, add CfL, restore the LLF from the
-// smoothed DC, inverse DCT straight into the padded XYB image.
+// ReconstructQuantizedCoefficients (src/codec/reconstruction.cpp:790-936):
+// dequantise, add CfL, restore the LLF from the smoothed DC, inverse DCT
+// straight into the padded XYB image.
+struct ReconstructArgs {
+  size_t store;
+  int width, height;
+  uint32_t counts[kStrategyStages];
+  size_t capacity;  // of each strategy's list
+  CodingParams params;
+};
+
 template <int kStrategy>
-__global__ __launch_bounds__(kAqThreads) void ReconstructKernel(
-  const int32_t* __restrict__ quantized, size_t store,
-  const uint32_t* __restrict__ entries, uint32_t count,
-  const uint32_t* __restrict__ offsets, int width, int height,
+struct ReconstructShared {
+  using S = AnchorShape<kStrategy>;
+  static constexpr int K = S::kK, N = S::kN;
+  double tmp[K * 3 * S::kH * (S::kW + 1)];
+  float coef[K * 3 * N];
+  TransformSlot slots[K];
+  float cfl[K][2];
+  float scale[K][3];
+};
+
+template <int kStrategy>
+__device__ __forceinline__ void Reconstruct(
+  ReconstructShared<kStrategy>& sh, uint32_t group, const uint32_t* __restrict__ entries,
+  uint32_t count, const int32_t* __restrict__ quantized, const uint32_t* __restrict__ offsets,
   const int32_t* __restrict__ raw, const int8_t* __restrict__ y_to_x,
   const int8_t* __restrict__ y_to_b, const QuantizerState* __restrict__ qstate,
   const float* __restrict__ tables, const double* __restrict__ bases,
-  CodingParams params, const float* __restrict__ smoothed_dc, float* __restrict__ out) {
+  const float* __restrict__ smoothed_dc, float* __restrict__ out, const ReconstructArgs& a) {
   using S = AnchorShape<kStrategy>;
   constexpr int W = S::kW, H = S::kH, N = S::kN, K = S::kK;
-  __shared__ float coef[K * 3 * N];
-  __shared__ double tmp[K * 3 * H * (W + 1)];
-  __shared__ TransformSlot slots[K];
-  __shared__ float cfl[K][2];
-  __shared__ float scale[K][3];
+  const size_t store = a.store;
+  const int width = a.width, height = a.height;
+  const CodingParams& params = a.params;
+  auto& coef = sh.coef;
+  auto& tmp = sh.tmp;
+  auto& slots = sh.slots;
+  auto& cfl = sh.cfl;
+  auto& scale = sh.scale;
   const int bw = width / 8, bh = height / 8;
   const double* ih = bases + BasisOffset(W, false);
   const double* iv = bases + BasisOffset(H, false);
-  LoadSlots<K>(entries, count, offsets, bw, slots);
+  LoadSlots<K>(group, entries, count, offsets, bw, slots);
   __syncthreads();
   const QuantizerState q = *qstate;
   // every global read that depends only on the slots, issued together:
@@ -1599,6 +1878,21 @@ __global__ __launch_bounds__(kAqThreads) void ReconstructKernel(
   });
 }
 
+__global__ __launch_bounds__(kAqThreads) void ReconstructKernel(
+  StageGrid grid, ReconstructArgs a, const int32_t* __restrict__ quantized,
+  const uint32_t* __restrict__ entries, const uint32_t* __restrict__ offsets,
+  const int32_t* __restrict__ raw, const int8_t* __restrict__ y_to_x,
+  const int8_t* __restrict__ y_to_b, const QuantizerState* __restrict__ qstate,
+  const float* __restrict__ tables, const double* __restrict__ bases,
+  const float* __restrict__ smoothed_dc, float* __restrict__ out) {
+  __shared__ __align__(16) unsigned char lds[SharedBytes<ReconstructShared>()];
+  DispatchStage(grid, [&]<int kStrategy>(uint32_t group, int stage) __attribute__((always_inline)) {
+    Reconstruct<kStrategy>(*reinterpret_cast<ReconstructShared<kStrategy>*>(lds), group,
+                           entries + stage * a.capacity, a.counts[stage], quantized, offsets, raw,
+                           y_to_x, y_to_b, qstate, tables, bases, smoothed_dc, out, a);
+  });
+}
+
 DcBasisTable HostDcBasis() {
   DcBasisTable t{};
   const double sqrt2 = 1.4142135623730951, pi = 3.141592653589793;
@@ -1644,10 +1938,9 @@ GJXLResult LaunchAnchorLayout(hipStream_t s, const uint8_t* cells, int width,
                               uint32_t* strategy_lists, size_t capacity,
                               uint32_t* strategy_counts) {
   const AqLayout l = MakeAqLayout(width, height);
-  hipLaunchKernelGGL(FillWordsKernel, dim3(1), dim3(64), 0, s, error, 1, 0u);
-  if (strategy_lists != nullptr) {
-    hipLaunchKernelGGL(FillWordsKernel, dim3(1), dim3(64), 0, s, strategy_counts,
-                       kStrategyStages, 0u);
+  // with strategy lists the caller has cleared *error and the counts
+  if (strategy_lists == nullptr) {
+    hipLaunchKernelGGL(FillWordsKernel, dim3(1), dim3(64), 0, s, error, 1, 0u);
   }
   hipLaunchKernelGGL(AnchorLayoutKernel, dim3(l.groups), dim3(kGroupAnchors), 0, s, cells,
                      l.bw, l.bh, offsets, list, count, error, strategy_lists, capacity,
@@ -1657,25 +1950,20 @@ GJXLResult LaunchAnchorLayout(hipStream_t s, const uint8_t* cells, int width,
 
 namespace {
 
-// Calls launch.template operator()<strategy>(entries, count) for every
-// strategy with transforms in the lists.
-template <typename Launch>
-GJXLResult ForEachStrategy(const StrategyLists& lists, Launch&& launch) {
-  const uint32_t* e = lists.entries;
-  const size_t c = lists.capacity;
-  if (lists.counts[0]) GJXL_AMD_TRY(launch.template operator()<kDct8>(e, lists.counts[0]));
-  if (lists.counts[1]) GJXL_AMD_TRY(launch.template operator()<kDct16x8>(e + c, lists.counts[1]));
-  if (lists.counts[2]) GJXL_AMD_TRY(launch.template operator()<kDct8x16>(e + 2 * c, lists.counts[2]));
-  if (lists.counts[3]) GJXL_AMD_TRY(launch.template operator()<kDct16x16>(e + 3 * c, lists.counts[3]));
-  if (lists.counts[4]) GJXL_AMD_TRY(launch.template operator()<kDct32x16>(e + 4 * c, lists.counts[4]));
-  if (lists.counts[5]) GJXL_AMD_TRY(launch.template operator()<kDct16x32>(e + 5 * c, lists.counts[5]));
-  if (lists.counts[6]) GJXL_AMD_TRY(launch.template operator()<kDct32x32>(e + 6 * c, lists.counts[6]));
-  return GJXL_OK;
-}
-
-template <int kStrategy>
-dim3 StrategyGrid(uint32_t count) {
-  return dim3((count + AnchorShape<kStrategy>::kK - 1) / AnchorShape<kStrategy>::kK);
+// The work groups of every strategy of the lists.
+StageGrid GridOf(const StrategyLists& lists) {
+  constexpr uint32_t kPerGroup[kStrategyStages] = {
+    AnchorShape<kDct8>::kK,     AnchorShape<kDct16x8>::kK,  AnchorShape<kDct8x16>::kK,
+    AnchorShape<kDct16x16>::kK, AnchorShape<kDct32x16>::kK, AnchorShape<kDct16x32>::kK,
+    AnchorShape<kDct32x32>::kK};
+  StageGrid g{};
+  uint32_t at = 0;
+  for (int i = 0; i < kStrategyStages; ++i) {
+    const int stage = kStrategyStages - 1 - i;
+    at += CeilDiv(lists.counts[stage], kPerGroup[stage]);
+    g.end[i] = at;
+  }
+  return g;
 }
 
 }  // namespace
@@ -1683,13 +1971,12 @@ dim3 StrategyGrid(uint32_t count) {
 GJXLResult LaunchAnchorDct(GJXLAmdDevice* d, const float* opsin, int width,
                            int height, const uint32_t* offsets,
                            const StrategyLists& lists, float* coefs) {
-  const AqLayout l = MakeAqLayout(width, height);
-  return ForEachStrategy(lists, [&]<int kStrategy>(const uint32_t* entries, uint32_t count) {
-    hipLaunchKernelGGL(AnchorDctKernel<kStrategy>, StrategyGrid<kStrategy>(count),
-                       dim3(kAqThreads), 0, d->stream, opsin, width, height, entries, count,
-                       offsets, d->dct_bases, l.store, coefs);
-    return CheckLaunch("AnchorDctKernel");
-  });
+  AnchorDctArgs a{width, height, MakeAqLayout(width, height).store, {}, lists.capacity};
+  std::copy_n(lists.counts, kStrategyStages, a.counts);
+  const StageGrid g = GridOf(lists);
+  hipLaunchKernelGGL(AnchorDctKernel, dim3(g.end[kStrategyStages - 1]), dim3(kAqThreads), 0,
+                     d->stream, g, a, opsin, lists.entries, offsets, d->dct_bases, coefs);
+  return CheckLaunch("AnchorDctKernel");
 }
 
 GJXLResult LaunchAdjustField(hipStream_t s, const uint8_t* cells, int width,
@@ -1709,7 +1996,6 @@ GJXLResult LaunchAdjustField(hipStream_t s, const uint8_t* cells, int width,
 GJXLResult LaunchMatrixStats(hipStream_t s, const float* opsin, int width,
                              int height, int padded_w, int padded_h,
                              uint32_t* stats) {
-  hipLaunchKernelGGL(FillWordsKernel, dim3(1), dim3(64), 0, s, stats, 3, 0u);
   hipLaunchKernelGGL(MatrixStatsKernel,
                      dim3(ReductionGroups(static_cast<size_t>(width) * height)), dim3(256), 0,
                      s, opsin, width, height, padded_w,
@@ -1718,31 +2004,33 @@ GJXLResult LaunchMatrixStats(hipStream_t s, const float* opsin, int width,
 }
 
 GJXLResult LaunchRange(hipStream_t s, const float* v, size_t n, uint32_t* range) {
-  hipLaunchKernelGGL(FillWordsKernel, dim3(1), dim3(64), 0, s, range, 1, 0xffffffffu);
-  hipLaunchKernelGGL(FillWordsKernel, dim3(1), dim3(64), 0, s, range + 1, 1, 0u);
   hipLaunchKernelGGL(RangeKernel, dim3(ReductionGroups(n)), dim3(256),
                      0, s, v, n, range);
   return CheckLaunch("RangeKernel");
 }
 
-// select: state (4 words), hist (256 words) of device scratch.
+// select: kSelectScratchWords words of device scratch, zero before the first
+// call and left zero where the next one needs it.
 GJXLResult LaunchQuantizer(hipStream_t s, const float* field, size_t n,
-                           float quant_dc, uint32_t* select_state,
-                           uint32_t* hist, QuantizerState* q, int32_t* raw) {
-  hipLaunchKernelGGL(FillWordsKernel, dim3(1), dim3(256), 0, s, hist, 256, 0u);
-  const uint32_t k = static_cast<uint32_t>(n / 2);
-  const int blocks = static_cast<int>(std::min<size_t>(CeilDiv(static_cast<uint32_t>(n), 256), 1024));
+                           float quant_dc, uint32_t* select, QuantizerState* q,
+                           int32_t* raw) {
+  if (n <= kSelectOneGroup) {
+    hipLaunchKernelGGL(QuantizerKernel, dim3(1), dim3(kSelectThreads), 0, s, field,
+                       static_cast<int>(n), quant_dc, q, raw);
+    return CheckLaunch("QuantizerKernel");
+  }
+  // four blocks per thread: fewer work groups than that wait longer for their
+  // reads, more add more counts to the same words
+  const uint32_t groups = static_cast<uint32_t>(
+    std::min<size_t>((n + kSelectBatch * kSelectThreads - 1) / (kSelectBatch * kSelectThreads), 256));
   for (int kind = 0; kind < 2; ++kind) {
-    hipLaunchKernelGGL(RadixResetKernel, dim3(1), dim3(1), 0, s, select_state, k, kind);
-    for (int shift = 24; shift >= 0; shift -= 8) {
-      hipLaunchKernelGGL(RadixHistogramKernel, dim3(blocks), dim3(256), 0, s, field, n,
-                         shift, kind, select_state, hist);
-      hipLaunchKernelGGL(RadixPickKernel, dim3(1), dim3(64), 0, s, hist, shift, kind,
-                         select_state);
+    for (int pass = 0; pass < kSelectPasses; ++pass) {
+      hipLaunchKernelGGL(SelectPassKernel, dim3(groups), dim3(kSelectThreads), 0, s, field, n,
+                         kind, pass, quant_dc, reinterpret_cast<SelectState*>(select),
+                         select + kSelectStateWords, q);
     }
   }
-  hipLaunchKernelGGL(QuantizerParamsKernel, dim3(1), dim3(64), 0, s, select_state,
-                     quant_dc, q);
+  GJXL_AMD_TRY(CheckLaunch("SelectPassKernel"));
   hipLaunchKernelGGL(RawQuantKernel, dim3(CeilDiv(static_cast<uint32_t>(n), 256)), dim3(256),
                      0, s, field, n, q, raw);
   return CheckLaunch("RawQuantKernel");
@@ -1767,7 +2055,7 @@ GJXLResult LaunchCodeCoefficients(GJXLAmdDevice* d, const float* coefs,
                                   const int8_t* y_to_x, const int8_t* y_to_b,
                                   const QuantizerState* q, float x_mult,
                                   float b_mult, int32_t* quantized, float* dc,
-                                  int32_t* dc_quantized, float* dc_rec) {
+                                  int32_t* dc_quantized) {
   (void)cells;
   const AqLayout l = MakeAqLayout(width, height);
   CodingParams p;
@@ -1776,21 +2064,25 @@ GJXLResult LaunchCodeCoefficients(GJXLAmdDevice* d, const float* coefs,
   static const DcBasisTable table = HostDcBasis();
   p.dc_basis = table;
   const size_t n = static_cast<size_t>(l.bw) * l.bh;
-  GJXL_AMD_TRY(ForEachStrategy(lists, [&]<int kStrategy>(const uint32_t* entries,
-                                                         uint32_t count) {
-    hipLaunchKernelGGL(CodeTransformKernel<kStrategy>, StrategyGrid<kStrategy>(count),
-                       dim3(kAqThreads), 0, d->stream, coefs, l.store, entries, count, offsets,
-                       l.bw, raw, y_to_x, y_to_b, q, d->quant_tables, p, quantized, dc, n);
-    return CheckLaunch("CodeTransformKernel");
-  }));
+  CodeArgs a{l.store, n, l.bw, {}, lists.capacity, p};
+  std::copy_n(lists.counts, kStrategyStages, a.counts);
+  const StageGrid g = GridOf(lists);
+  hipLaunchKernelGGL(CodeTransformKernel, dim3(g.end[kStrategyStages - 1]), dim3(kAqThreads), 0,
+                     d->stream, g, a, coefs, lists.entries, offsets, raw, y_to_x, y_to_b, q,
+                     d->quant_tables, quantized, dc);
+  GJXL_AMD_TRY(CheckLaunch("CodeTransformKernel"));
   const dim3 groups(CeilDiv(l.bw, kDcGroup), CeilDiv(l.bh, kDcGroup), 2);
   const bool probed = ProbeBegin(d, GJXL_AMD_KERNEL_DC_QUANT);
   hipLaunchKernelGGL(DcQuantKernel, groups, dim3(kDcWorkGroup), 0, d->stream, dc, l.bw,
-                     l.bh, q, 1, dc_quantized);
+                     l.bh, q, kDcExtraPrecision, dc_quantized);
   ProbeEnd(d, probed);
-  GJXL_AMD_TRY(CheckLaunch("DcQuantKernel"));
+  return CheckLaunch("DcQuantKernel");
+}
+
+GJXLResult LaunchDcReconstruct(GJXLAmdDevice* d, const int32_t* dc_quantized, size_t n,
+                               const QuantizerState* q, float* dc_rec) {
   hipLaunchKernelGGL(DcReconstructKernel, dim3(CeilDiv(static_cast<uint32_t>(n), 256)),
-                     dim3(256), 0, d->stream, dc_quantized, n, q, 1, dc_rec);
+                     dim3(256), 0, d->stream, dc_quantized, n, q, kDcExtraPrecision, dc_rec);
   return CheckLaunch("DcReconstructKernel");
 }
 
@@ -1800,27 +2092,25 @@ GJXLResult LaunchReconstruct(GJXLAmdDevice* d, const int32_t* quantized,
                              const int32_t* raw,
                              const int8_t* y_to_x, const int8_t* y_to_b,
                              const QuantizerState* q, float x_mult, float b_mult,
-                             const float* dc_rec, float* smoothed,
-                             float* inv_sigma, float* out) {
+                             const int32_t* dc_quantized, float* dc_rec,
+                             float* smoothed, float* inv_sigma, float* out) {
   const AqLayout l = MakeAqLayout(width, height);
-  hipLaunchKernelGGL(EpfSigmaKernel, dim3(CeilDiv(l.bw, 256), l.bh), dim3(256), 0,
-                     d->stream, cells, l.bw, l.bh, raw, q, inv_sigma);
-  GJXL_AMD_TRY(CheckLaunch("EpfSigmaKernel"));
-  hipLaunchKernelGGL(SmoothDcKernel, dim3(CeilDiv(l.bw, 256), l.bh), dim3(256), 0,
-                     d->stream, dc_rec, l.bw, l.bh, q, smoothed);
-  GJXL_AMD_TRY(CheckLaunch("SmoothDcKernel"));
+  hipLaunchKernelGGL(BlockFieldsKernel, dim3(CeilDiv(l.bw, 256), l.bh), dim3(256), 0, d->stream,
+                     dc_quantized, l.bw, l.bh, q, kDcExtraPrecision, cells, raw, dc_rec, smoothed,
+                     inv_sigma);
+  GJXL_AMD_TRY(CheckLaunch("BlockFieldsKernel"));
   CodingParams p;
   p.x_mult = x_mult;
   p.b_mult = b_mult;
   static const DcBasisTable table = HostDcBasis();
   p.dc_basis = table;
-  return ForEachStrategy(lists, [&]<int kStrategy>(const uint32_t* entries, uint32_t count) {
-    hipLaunchKernelGGL(ReconstructKernel<kStrategy>, StrategyGrid<kStrategy>(count),
-                       dim3(kAqThreads), 0, d->stream, quantized, l.store, entries, count,
-                       offsets, width, height, raw, y_to_x, y_to_b, q, d->quant_tables,
-                       d->dct_bases, p, smoothed, out);
-    return CheckLaunch("ReconstructKernel");
-  });
+  ReconstructArgs a{l.store, width, height, {}, lists.capacity, p};
+  std::copy_n(lists.counts, kStrategyStages, a.counts);
+  const StageGrid g = GridOf(lists);
+  hipLaunchKernelGGL(ReconstructKernel, dim3(g.end[kStrategyStages - 1]), dim3(kAqThreads), 0,
+                     d->stream, g, a, quantized, lists.entries, offsets, raw, y_to_x, y_to_b, q,
+                     d->quant_tables, d->dct_bases, smoothed, out);
+  return CheckLaunch("ReconstructKernel");
 }
 
 }  // namespace gjxl_amd

@@ -58,12 +58,14 @@ GJXLResult ValidateSession(GJXLAmdAqSession* s) {
 constexpr int kMaxIterations = 62;  // scores hold iterations + 1 words
 constexpr int kErrorWord = 7;       // in the stats buffer
 
-__global__ void CopyWordKernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst) {
-  if (threadIdx.x == 0) *dst = *src;
-}
-
 __global__ void ZeroWordKernel(uint32_t* __restrict__ dst) {
   if (threadIdx.x == 0) *dst = 0;
+}
+
+// stats: 0-2 the matrix statistics, 4-5 the field's minimum and maximum, 6
+// the layout's error, kErrorWord the updates', 8.. the strategies' counts.
+__global__ void ResetStatsKernel(uint32_t* __restrict__ stats) {
+  if (threadIdx.x < 16 && threadIdx.x != 3) stats[threadIdx.x] = threadIdx.x == 4 ? 0xffffffffu : 0u;
 }
 
 __global__ void ZeroWordsKernel(uint32_t* __restrict__ p, size_t n) {
@@ -156,7 +158,7 @@ void SessionGeometry(GJXLAmdAqSession* s, uint32_t width, uint32_t height, size_
   z[GJXL_AMD_AQ_COEFFICIENTS] = 4 * 3 * store;
   z[GJXL_AMD_AQ_ADJUSTED_FIELD] = 4 * n;
   z[GJXL_AMD_AQ_STATS] = 4 * 16;
-  z[GJXL_AMD_AQ_SELECT] = 4 * (4 + 256);
+  z[GJXL_AMD_AQ_SELECT] = 4 * gjxl_amd::kSelectScratchWords;
   z[GJXL_AMD_AQ_QUANTIZER] = sizeof(gjxl_amd::QuantizerState);
   z[GJXL_AMD_AQ_RAW_QUANT] = 4 * n;
   z[GJXL_AMD_AQ_Y_TO_X] = tiles;
@@ -176,11 +178,13 @@ void SessionGeometry(GJXLAmdAqSession* s, uint32_t width, uint32_t height, size_
   z[GJXL_AMD_AQ_STRATEGY_LISTS] = 4 * gjxl_amd::kStrategyStages * n;
 }
 
-// Zeroes the coefficient stores (their unused group tails must read zero)
-// and the statistics words on the device stream, then waits.
+// Zeroes the coefficient stores (their unused group tails must read zero),
+// the statistics words and the selection scratch on the device stream, then
+// waits.
 GJXLResult ClearStores(GJXLAmdAqSession* s) {
   GJXLResult r = GJXL_OK;
-  for (int id : {GJXL_AMD_AQ_COEFFICIENTS, GJXL_AMD_AQ_QUANTIZED, GJXL_AMD_AQ_STATS}) {
+  for (int id : {GJXL_AMD_AQ_COEFFICIENTS, GJXL_AMD_AQ_QUANTIZED, GJXL_AMD_AQ_STATS,
+                 GJXL_AMD_AQ_SELECT}) {
     if (r != GJXL_OK) break;
     hipLaunchKernelGGL(ZeroWordsKernel, dim3(1024), dim3(256), 0, s->device->stream,
                        static_cast<uint32_t*>(s->buffers[id]), s->sizes[id] / 4);
@@ -213,16 +217,16 @@ GJXLResult ResizeAqSession(GJXLAmdAqSession* s, uint32_t width, uint32_t height)
   return ClearStores(s);
 }
 
-// The quantizing part of an evaluation: quantizer, final CfL, coefficient
-// coding and DC (what tokenization reads); the session is validated and
-// prepared.
-GJXLResult AqQuantize(GJXLAmdAqSession* s, const float* quant_field) {
+namespace {
+
+// Quantizer, final CfL, coefficient coding and DC.
+GJXLResult Quantize(GJXLAmdAqSession* s, const float* quant_field) {
   GJXLAmdDevice* d = s->device;
   hipStream_t st = d->stream;
   const size_t n = static_cast<size_t>(s->layout.bw) * s->layout.bh;
   uint32_t* select = Buf<uint32_t>(s, GJXL_AMD_AQ_SELECT);
   auto* q = Buf<QuantizerState>(s, GJXL_AMD_AQ_QUANTIZER);
-  GJXL_AMD_TRY(LaunchQuantizer(st, quant_field, n, s->quant_dc, select, select + 4, q,
+  GJXL_AMD_TRY(LaunchQuantizer(st, quant_field, n, s->quant_dc, select, q,
                                Buf<int32_t>(s, GJXL_AMD_AQ_RAW_QUANT)));
   GJXL_AMD_TRY(LaunchFinalCfl(d, Buf<float>(s, GJXL_AMD_AQ_COEFFICIENTS), s->pw, s->ph,
                               s->cells, Buf<uint32_t>(s, GJXL_AMD_AQ_OFFSETS),
@@ -234,9 +238,20 @@ GJXLResult AqQuantize(GJXLAmdAqSession* s, const float* quant_field) {
     Buf<uint32_t>(s, GJXL_AMD_AQ_OFFSETS), Lists(s), Buf<int32_t>(s, GJXL_AMD_AQ_RAW_QUANT),
     Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_X), Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_B), q,
     s->x_mult, s->b_mult, Buf<int32_t>(s, GJXL_AMD_AQ_QUANTIZED),
-    Buf<float>(s, GJXL_AMD_AQ_DC), Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED),
-    Buf<float>(s, GJXL_AMD_AQ_DC_RECONSTRUCTED)));
+    Buf<float>(s, GJXL_AMD_AQ_DC), Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED)));
   return GJXL_OK;
+}
+
+}  // namespace
+
+// The quantizing part of an evaluation (what tokenization reads) with the
+// reconstructed DC; the session is validated and prepared.
+GJXLResult AqQuantize(GJXLAmdAqSession* s, const float* quant_field) {
+  GJXL_AMD_TRY(Quantize(s, quant_field));
+  return LaunchDcReconstruct(s->device, Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED),
+                             static_cast<size_t>(s->layout.bw) * s->layout.bh,
+                             Buf<QuantizerState>(s, GJXL_AMD_AQ_QUANTIZER),
+                             Buf<float>(s, GJXL_AMD_AQ_DC_RECONSTRUCTED));
 }
 
 }  // namespace gjxl_amd
@@ -305,10 +320,11 @@ GJXLResult gjxl_amd_aq_prepare(GJXLAmdAqSession* s, const float* opsin,
   s->cells = cells;
   s->target = butteraugli_target;
   using namespace gjxl_amd;
-  // the invalid-distance flag of the updates that follow this preparation
-  hipLaunchKernelGGL(ZeroWordKernel, dim3(1), dim3(64), 0, st,
-                     Buf<uint32_t>(s, GJXL_AMD_AQ_STATS) + kErrorWord);
-  GJXL_AMD_TRY(CheckLaunch("ZeroWordKernel"));
+  // the statistics' start values, among them the invalid-distance flag of
+  // the updates that follow this preparation
+  hipLaunchKernelGGL(ResetStatsKernel, dim3(1), dim3(64), 0, st,
+                     Buf<uint32_t>(s, GJXL_AMD_AQ_STATS));
+  GJXL_AMD_TRY(CheckLaunch("ResetStatsKernel"));
   GJXL_AMD_TRY(LaunchMatrixStats(st, opsin, s->width, s->height, s->pw, s->ph,
                                  Buf<uint32_t>(s, GJXL_AMD_AQ_STATS)));
   const size_t blocks = static_cast<size_t>(s->layout.bw) * s->layout.bh;
@@ -396,13 +412,13 @@ GJXLResult gjxl_amd_aq_evaluate(GJXLAmdAqSession* s, const float* quant_field) {
   GJXLAmdDevice* d = s->device;
   hipStream_t st = d->stream;
   auto* q = Buf<QuantizerState>(s, GJXL_AMD_AQ_QUANTIZER);
-  GJXL_AMD_TRY(AqQuantize(s, quant_field));
+  GJXL_AMD_TRY(Quantize(s, quant_field));
   GJXL_AMD_TRY(LaunchReconstruct(
     d, Buf<int32_t>(s, GJXL_AMD_AQ_QUANTIZED), s->pw, s->ph, s->cells,
     Buf<uint32_t>(s, GJXL_AMD_AQ_OFFSETS), Lists(s), Buf<int32_t>(s, GJXL_AMD_AQ_RAW_QUANT),
     Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_X), Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_B), q, s->x_mult,
-    s->b_mult, Buf<float>(s, GJXL_AMD_AQ_DC_RECONSTRUCTED),
-    Buf<float>(s, GJXL_AMD_AQ_DC_SMOOTHED), Buf<float>(s, GJXL_AMD_AQ_INVERSE_SIGMA),
+    s->b_mult, Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED),
+    Buf<float>(s, GJXL_AMD_AQ_DC_RECONSTRUCTED), Buf<float>(s, GJXL_AMD_AQ_DC_SMOOTHED), Buf<float>(s, GJXL_AMD_AQ_INVERSE_SIGMA),
     Buf<float>(s, GJXL_AMD_AQ_RECONSTRUCTED)));
   return LaunchLoopFiltersAndColor(
     st, Buf<float>(s, GJXL_AMD_AQ_RECONSTRUCTED), s->pw, s->ph, s->width, s->height,
@@ -451,10 +467,9 @@ GJXLResult gjxl_amd_aq_run(GJXLAmdAqSession* s, GJXLAmdButteraugli* b,
   for (int it = 0; it <= iterations; ++it) {
     GJXL_AMD_TRY(gjxl_amd_aq_evaluate(s, field));
     GJXL_AMD_TRY(gjxl_amd::ButteraugliCompare(b, Buf<float>(s, GJXL_AMD_AQ_LINEAR), nullptr));
-    hipLaunchKernelGGL(CopyWordKernel, dim3(1), dim3(64), 0, st, b->score_bits,
-                       score_bits + it);
     GJXL_AMD_TRY(gjxl_amd::LaunchReduceDistanceMap(st, b->map, s->width, s->height, s->cells,
-                                                   s->layout.bw, s->layout.bh, distance));
+                                                   s->layout.bw, s->layout.bh, distance,
+                                                   b->score_bits, score_bits + it));
     if (it == iterations) break;
     GJXL_AMD_TRY(gjxl_amd_aq_update(s, field, distance, it, butteraugli_target));
   }

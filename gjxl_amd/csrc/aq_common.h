@@ -242,13 +242,17 @@ GJXLResult LaunchAnchorDct(GJXLAmdDevice* d, const float* opsin, int width,
 GJXLResult LaunchAdjustField(hipStream_t s, const uint8_t* cells, int width,
                              int height, float target, const float* in,
                              float* out);
+// stats: 3 words, zero beforehand.
 GJXLResult LaunchMatrixStats(hipStream_t s, const float* opsin, int width,
                              int height, int padded_w, int padded_h,
                              uint32_t* stats);
+// range: the minimum, all ones beforehand, and the maximum, zero beforehand.
 GJXLResult LaunchRange(hipStream_t s, const float* v, size_t n, uint32_t* range);
+// Words of device scratch for the quantizer's selection.
+constexpr size_t kSelectScratchWords = 16 + 2048;
 GJXLResult LaunchQuantizer(hipStream_t s, const float* field, size_t n,
-                           float quant_dc, uint32_t* select_state,
-                           uint32_t* hist, QuantizerState* q, int32_t* raw);
+                           float quant_dc, uint32_t* select, QuantizerState* q,
+                           int32_t* raw);
 GJXLResult LaunchFinalCfl(GJXLAmdDevice* d, const float* coefs, int width,
                           int height, const uint8_t* cells,
                           const uint32_t* offsets, const int32_t* raw,
@@ -261,15 +265,17 @@ GJXLResult LaunchCodeCoefficients(GJXLAmdDevice* d, const float* coefs,
                                   const int8_t* y_to_x, const int8_t* y_to_b,
                                   const QuantizerState* q, float x_mult,
                                   float b_mult, int32_t* quantized, float* dc,
-                                  int32_t* dc_quantized, float* dc_rec);
+                                  int32_t* dc_quantized);
+GJXLResult LaunchDcReconstruct(GJXLAmdDevice* d, const int32_t* dc_quantized, size_t n,
+                               const QuantizerState* q, float* dc_rec);
 GJXLResult LaunchReconstruct(GJXLAmdDevice* d, const int32_t* quantized,
                              int width, int height, const uint8_t* cells,
                              const uint32_t* offsets, const StrategyLists& lists,
                              const int32_t* raw,
                              const int8_t* y_to_x, const int8_t* y_to_b,
                              const QuantizerState* q, float x_mult, float b_mult,
-                             const float* dc_rec, float* smoothed,
-                             float* inv_sigma, float* out);
+                             const int32_t* dc_quantized, float* dc_rec,
+                             float* smoothed, float* inv_sigma, float* out);
 GJXLResult LaunchLoopFiltersAndColor(hipStream_t s, const float* reconstructed,
                                      int pw, int ph, int w, int h,
                                      const float* inverse_sigma,

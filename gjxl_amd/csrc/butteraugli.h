@@ -71,9 +71,11 @@ void CarveButteraugli(GJXLAmdButteraugli* b);
 GJXLResult ResizeButteraugli(GJXLAmdButteraugli* b, uint32_t width, uint32_t height);
 
 // a17: per-transform 1.2 * (mean d^16)^(1/16) broadcast over the covered
-// blocks.  map: width x height (unpadded); cells: (pw/8) x (ph/8).
+// blocks.  map: width x height (unpadded); cells: (pw/8) x (ph/8).  With a
+// score word, it is copied to score_out (the loop keeps every evaluation's).
 GJXLResult LaunchReduceDistanceMap(hipStream_t s, const float* map, int width,
                                    int height, const uint8_t* cells, int bw,
-                                   int bh, float* out);
+                                   int bh, float* out, const uint32_t* score = nullptr,
+                                   uint32_t* score_out = nullptr);
 
 }  // namespace gjxl_amd

@@ -182,10 +182,6 @@ T* TokenBuffer(GJXLAmdTokenizer* t, int id) {
   return static_cast<T*>(p);
 }
 
-__global__ void CopyScoreKernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst) {
-  if (threadIdx.x == 0) *dst = *src;
-}
-
 GJXLResult ValidateOptions(const GJXLAmdPlainPathOptions* o) {
   if (o == nullptr || o->struct_size < sizeof(GJXLAmdPlainPathOptions)) {
     return Fail(GJXL_ERROR_INVALID_ARGUMENT, "plain path options are missing or too small");
@@ -335,11 +331,10 @@ GJXLResult RunBack(GJXLAmdPlainPath* p, bool costs_ready) {
     GJXL_AMD_TRY(Mark(p, GJXL_AMD_STAGE_AQ_EVALUATE));
     GJXL_AMD_TRY(gjxl_amd::ButteraugliCompare(p->butteraugli, decoded, nullptr));
     GJXL_AMD_TRY(Mark(p, GJXL_AMD_STAGE_BUTTERAUGLI_COMPARE));
-    hipLaunchKernelGGL(CopyScoreKernel, dim3(1), dim3(64), 0, st, p->butteraugli->score_bits,
-                       p->score_words + it);
-    GJXL_AMD_TRY(gjxl_amd::CheckLaunch("CopyScoreKernel"));
     GJXL_AMD_TRY(gjxl_amd::LaunchReduceDistanceMap(st, p->butteraugli->map, p->width, p->height,
-                                                   p->cells, p->bw, p->bh, distance));
+                                                   p->cells, p->bw, p->bh, distance,
+                                                   p->butteraugli->score_bits,
+                                                   p->score_words + it));
     bool more = it < planned;
     if (!more && head != nullptr) {
       // the judge: the 3-norm of the block distances; the learned run goes

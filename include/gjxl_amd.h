@@ -238,7 +238,7 @@ enum {
   GJXL_AMD_AQ_ADJUSTED_FIELD,       /* f32 AdjustQuantField output */
   GJXL_AMD_AQ_STATS,                /* u32[16]: matrix stats 0-2, range 4-5,
                                        grid error 6, strategy counts 8-14 */
-  GJXL_AMD_AQ_SELECT,               /* u32[4 + 256]: median / MAD selection */
+  GJXL_AMD_AQ_SELECT,               /* u32 scratch: median / MAD selection */
   GJXL_AMD_AQ_QUANTIZER,            /* quantizer state (10 words) */
   GJXL_AMD_AQ_RAW_QUANT,            /* i32 per block: adjusted raw quant */
   GJXL_AMD_AQ_Y_TO_X,               /* i8 per 64x64 tile: final CfL */

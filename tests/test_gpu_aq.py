@@ -161,3 +161,31 @@ def test_aq_dc_wide_groups(device):
     assert np.abs(want["dc_q"][:, :, 256:]).max() < 2**18
     _check_evaluation(s, fe, setup, setup["adjusted"], w, h)
     s.close()
+
+
+@pytest.mark.parametrize("w,h", [(8, 8), (264, 40), (1024, 1024), (1032, 1024), (1544, 1032)])
+@pytest.mark.parametrize("kind", ["spread", "ties", "constant"])
+def test_quantizer_selection(device, w, h, kind):
+    """The quantizer's exact median and MAD on both sides of the one-group
+    limit (16,384 blocks), with ties and a constant field, against a sort."""
+    print(f"quantizer {w}x{h} {kind}", flush=True)
+    rng = np.random.default_rng(w + h)
+    bh, bw = h // 8, w // 8
+    opsin = device.array(rng.uniform(0.0, 0.5, (3, h, w)).astype(np.float32))
+    field = {"spread": np.exp(rng.normal(0.0, 2.0, (bh, bw))),
+             "ties": rng.integers(1, 5, (bh, bw)) * 0.375,
+             "constant": np.full((bh, bw), 0.71)}[kind].astype(np.float32)
+    s = gjxl_amd.AqSession(device, w, h)
+    s.prepare(opsin, opsin, device.array(np.full((bh, bw), 1, np.uint8)),
+              device.array(np.full((bh, bw), 0.7, np.float32)))
+    for _ in range(2):  # the second selection finds the scratch as the first left it
+        s.evaluate(device.array(field))
+        q = s.buffer("quantizer", (10,), np.uint32).numpy()
+        n = field.size
+        median = np.sort(field.reshape(-1))[n // 2]
+        mad = np.sort(np.abs(field.reshape(-1) - median))[n // 2]
+        scale = np.float32(65536.0) * (median - mad) / np.float32(5.0)
+        want = int(min(max(scale, np.float32(1.0)), np.float32(32768.0)))
+        dc = int(float(np.float32(s.policy()["quant_dc"]) * np.float32(4096.0)) * 1.6)
+        assert int(q[2]) == (max(dc, 1) if want > dc else want)
+    s.close()

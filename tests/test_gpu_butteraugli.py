@@ -108,6 +108,30 @@ def test_reduce_distance_map(device):
     assert _bits_equal(got, want)
 
 
+@pytest.mark.parametrize("w,h", [(61, 70), (129, 135), (256, 64)])
+def test_reduce_distance_map_footprints(device, w, h):
+    """Transforms of every size at the map's ragged edges, and 32x32 ones across
+    the 64-pixel tiles of the kernel."""
+    bw, bh = (w + 7) // 8, (h + 7) // 8
+    codes = {(4, 4): 5, (4, 2): 11, (2, 4): 10, (2, 2): 4, (2, 1): 7, (1, 2): 6, (1, 1): 0}
+    rng = np.random.default_rng(w)
+    cells = np.zeros((bh, bw), np.uint8)
+    covered = np.zeros((bh, bw), bool)
+    for by in range(bh):
+        for bx in range(bw):
+            if covered[by, bx]:
+                continue
+            sizes = [k for k in codes if bx + k[0] <= bw and by + k[1] <= bh and
+                     not covered[by:by + k[1], bx:bx + k[0]].any()]
+            cw, ch = sizes[0] if bx % 5 == 2 else sizes[rng.integers(len(sizes))]
+            cells[by:by + ch, bx:bx + cw] = codes[(cw, ch)] << 1
+            cells[by, bx] |= 1
+            covered[by:by + ch, bx:bx + cw] = True
+    dmap = rng.uniform(0.0, 3.0, (h, w)).astype(np.float32)
+    got = gjxl_amd.reduce_distance_map(device, device.array(dmap), device.array(cells)).numpy()
+    assert _bits_equal(got, binding.reduce_distance_map(dmap, cells))
+
+
 @pytest.mark.parametrize("w,h,seed", [(64, 64, 1), (200, 136, 4), (8, 8, 3), (72, 40, 7),
                                       (512, 512, 1)])
 def test_aq_loop_parity(device, w, h, seed):
