@@ -2055,7 +2055,7 @@ GJXLResult LaunchCodeCoefficients(GJXLAmdDevice* d, const float* coefs,
                                   const int8_t* y_to_x, const int8_t* y_to_b,
                                   const QuantizerState* q, float x_mult,
                                   float b_mult, int32_t* quantized, float* dc,
-                                  int32_t* dc_quantized) {
+                                  int32_t* dc_quantized, hipEvent_t coded) {
   (void)cells;
   const AqLayout l = MakeAqLayout(width, height);
   CodingParams p;
@@ -2071,6 +2071,7 @@ GJXLResult LaunchCodeCoefficients(GJXLAmdDevice* d, const float* coefs,
                      d->stream, g, a, coefs, lists.entries, offsets, raw, y_to_x, y_to_b, q,
                      d->quant_tables, quantized, dc);
   GJXL_AMD_TRY(CheckLaunch("CodeTransformKernel"));
+  if (coded != nullptr) GJXL_AMD_TRY(Check(hipEventRecord(coded, d->stream), "hipEventRecord"));
   const dim3 groups(CeilDiv(l.bw, kDcGroup), CeilDiv(l.bh, kDcGroup), 2);
   const bool probed = ProbeBegin(d, GJXL_AMD_KERNEL_DC_QUANT);
   hipLaunchKernelGGL(DcQuantKernel, groups, dim3(kDcWorkGroup), 0, d->stream, dc, l.bw,

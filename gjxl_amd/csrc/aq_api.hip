@@ -220,7 +220,7 @@ GJXLResult ResizeAqSession(GJXLAmdAqSession* s, uint32_t width, uint32_t height)
 namespace {
 
 // Quantizer, final CfL, coefficient coding and DC.
-GJXLResult Quantize(GJXLAmdAqSession* s, const float* quant_field) {
+GJXLResult Quantize(GJXLAmdAqSession* s, const float* quant_field, hipEvent_t coded) {
   GJXLAmdDevice* d = s->device;
   hipStream_t st = d->stream;
   const size_t n = static_cast<size_t>(s->layout.bw) * s->layout.bh;
@@ -238,7 +238,7 @@ GJXLResult Quantize(GJXLAmdAqSession* s, const float* quant_field) {
     Buf<uint32_t>(s, GJXL_AMD_AQ_OFFSETS), Lists(s), Buf<int32_t>(s, GJXL_AMD_AQ_RAW_QUANT),
     Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_X), Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_B), q,
     s->x_mult, s->b_mult, Buf<int32_t>(s, GJXL_AMD_AQ_QUANTIZED),
-    Buf<float>(s, GJXL_AMD_AQ_DC), Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED)));
+    Buf<float>(s, GJXL_AMD_AQ_DC), Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED), coded));
   return GJXL_OK;
 }
 
@@ -246,12 +246,34 @@ GJXLResult Quantize(GJXLAmdAqSession* s, const float* quant_field) {
 
 // The quantizing part of an evaluation (what tokenization reads) with the
 // reconstructed DC; the session is validated and prepared.
-GJXLResult AqQuantize(GJXLAmdAqSession* s, const float* quant_field) {
-  GJXL_AMD_TRY(Quantize(s, quant_field));
+GJXLResult AqQuantize(GJXLAmdAqSession* s, const float* quant_field, hipEvent_t coded) {
+  GJXL_AMD_TRY(Quantize(s, quant_field, coded));
   return LaunchDcReconstruct(s->device, Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED),
                              static_cast<size_t>(s->layout.bw) * s->layout.bh,
                              Buf<QuantizerState>(s, GJXL_AMD_AQ_QUANTIZER),
                              Buf<float>(s, GJXL_AMD_AQ_DC_RECONSTRUCTED));
+}
+
+GJXLResult AqEvaluate(GJXLAmdAqSession* s, const float* quant_field, hipEvent_t coded) {
+  GJXL_AMD_TRY(ValidateSession(s));
+  if (!s->prepared || quant_field == nullptr) {
+    return Fail(GJXL_ERROR_INVALID_ARGUMENT, "AQ evaluation needs a prepared session and a field");
+  }
+  GJXLAmdDevice* d = s->device;
+  hipStream_t st = d->stream;
+  auto* q = Buf<QuantizerState>(s, GJXL_AMD_AQ_QUANTIZER);
+  GJXL_AMD_TRY(Quantize(s, quant_field, coded));
+  GJXL_AMD_TRY(LaunchReconstruct(
+    d, Buf<int32_t>(s, GJXL_AMD_AQ_QUANTIZED), s->pw, s->ph, s->cells,
+    Buf<uint32_t>(s, GJXL_AMD_AQ_OFFSETS), Lists(s), Buf<int32_t>(s, GJXL_AMD_AQ_RAW_QUANT),
+    Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_X), Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_B), q, s->x_mult,
+    s->b_mult, Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED),
+    Buf<float>(s, GJXL_AMD_AQ_DC_RECONSTRUCTED), Buf<float>(s, GJXL_AMD_AQ_DC_SMOOTHED), Buf<float>(s, GJXL_AMD_AQ_INVERSE_SIGMA),
+    Buf<float>(s, GJXL_AMD_AQ_RECONSTRUCTED)));
+  return LaunchLoopFiltersAndColor(
+    st, Buf<float>(s, GJXL_AMD_AQ_RECONSTRUCTED), s->pw, s->ph, s->width, s->height,
+    Buf<float>(s, GJXL_AMD_AQ_INVERSE_SIGMA), Buf<float>(s, GJXL_AMD_AQ_FILTERED),
+    Buf<float>(s, GJXL_AMD_AQ_LINEAR), 255.0f);
 }
 
 }  // namespace gjxl_amd
@@ -404,26 +426,7 @@ GJXLResult gjxl_amd_aq_split_forward_dct(GJXLAmdAqSession* s) {
 }
 
 GJXLResult gjxl_amd_aq_evaluate(GJXLAmdAqSession* s, const float* quant_field) {
-  GJXL_AMD_TRY(ValidateSession(s));
-  if (!s->prepared || quant_field == nullptr) {
-    return Fail(GJXL_ERROR_INVALID_ARGUMENT, "AQ evaluation needs a prepared session and a field");
-  }
-  using namespace gjxl_amd;
-  GJXLAmdDevice* d = s->device;
-  hipStream_t st = d->stream;
-  auto* q = Buf<QuantizerState>(s, GJXL_AMD_AQ_QUANTIZER);
-  GJXL_AMD_TRY(Quantize(s, quant_field));
-  GJXL_AMD_TRY(LaunchReconstruct(
-    d, Buf<int32_t>(s, GJXL_AMD_AQ_QUANTIZED), s->pw, s->ph, s->cells,
-    Buf<uint32_t>(s, GJXL_AMD_AQ_OFFSETS), Lists(s), Buf<int32_t>(s, GJXL_AMD_AQ_RAW_QUANT),
-    Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_X), Buf<int8_t>(s, GJXL_AMD_AQ_Y_TO_B), q, s->x_mult,
-    s->b_mult, Buf<int32_t>(s, GJXL_AMD_AQ_DC_QUANTIZED),
-    Buf<float>(s, GJXL_AMD_AQ_DC_RECONSTRUCTED), Buf<float>(s, GJXL_AMD_AQ_DC_SMOOTHED), Buf<float>(s, GJXL_AMD_AQ_INVERSE_SIGMA),
-    Buf<float>(s, GJXL_AMD_AQ_RECONSTRUCTED)));
-  return LaunchLoopFiltersAndColor(
-    st, Buf<float>(s, GJXL_AMD_AQ_RECONSTRUCTED), s->pw, s->ph, s->width, s->height,
-    Buf<float>(s, GJXL_AMD_AQ_INVERSE_SIGMA), Buf<float>(s, GJXL_AMD_AQ_FILTERED),
-    Buf<float>(s, GJXL_AMD_AQ_LINEAR), 255.0f);
+  return gjxl_amd::AqEvaluate(s, quant_field, nullptr);
 }
 
 GJXLResult gjxl_amd_aq_update(GJXLAmdAqSession* s, float* quant_field,

@@ -39,8 +39,11 @@ struct StrategyLists {
 GJXLResult ResizeAqSession(GJXLAmdAqSession* s, uint32_t width, uint32_t height);
 // The quantizing part of gjxl_amd_aq_evaluate (quantizer, final CfL,
 // coefficient coding, DC) without reconstruction and loop filters; the
-// session is validated and prepared.
-GJXLResult AqQuantize(GJXLAmdAqSession* s, const float* quant_field);
+// session is validated and prepared.  With an event, it is recorded where
+// the coefficients and the raw quant are final, before the DC.
+GJXLResult AqQuantize(GJXLAmdAqSession* s, const float* quant_field, hipEvent_t coded = nullptr);
+// gjxl_amd_aq_evaluate, with the same event.
+GJXLResult AqEvaluate(GJXLAmdAqSession* s, const float* quant_field, hipEvent_t coded);
 
 // The split-precision forward DCT of every transform of a frame into the
 // per-group coefficient store (split_dct.hip).
@@ -265,7 +268,7 @@ GJXLResult LaunchCodeCoefficients(GJXLAmdDevice* d, const float* coefs,
                                   const int8_t* y_to_x, const int8_t* y_to_b,
                                   const QuantizerState* q, float x_mult,
                                   float b_mult, int32_t* quantized, float* dc,
-                                  int32_t* dc_quantized);
+                                  int32_t* dc_quantized, hipEvent_t coded);
 GJXLResult LaunchDcReconstruct(GJXLAmdDevice* d, const int32_t* dc_quantized, size_t n,
                                const QuantizerState* q, float* dc_rec);
 GJXLResult LaunchReconstruct(GJXLAmdDevice* d, const int32_t* quantized,

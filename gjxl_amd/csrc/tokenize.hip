@@ -982,6 +982,8 @@ GJXLResult FrameStatisticsResult(GJXLAmdTokenizer* t, const uint32_t* words,
 
 size_t FrameStatisticsWords() { return kStatWords; }
 
+void TokenizerUseDevice(GJXLAmdTokenizer* t, GJXLAmdDevice* device) { t->device = device; }
+
 GJXLResult ResizeTokenizer(GJXLAmdTokenizer* t, uint32_t width, uint32_t height) {
   if (width == 0 || height == 0 || width > (1u << 16) || height > (1u << 16)) {
     return Fail(GJXL_ERROR_INVALID_ARGUMENT, "tokenizer geometry is invalid");
