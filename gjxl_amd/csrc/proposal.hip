@@ -260,69 +260,121 @@ __global__ __launch_bounds__(64 * kConvWaves) void ConvKernel(
 
 constexpr int kGradGroups = 256;
 
-// One wave per work group over tiles_per_group runs of 16 positions: the
-// positions are the MFMA's K dimension.  A = the masked output gradient
-// (output channel x position), B = the shifted inputs (position x input
-// channel); D accumulates dW of every tap in registers.  Partial sums per
-// group go to `partial` ([group][9][32][kCin] then 32 bias sums).
+// A work group takes tiles_per_group runs of 16 positions: the positions are
+// the MFMA's K dimension.  A = the masked output gradient (output channel x
+// position), B = the shifted inputs (position x input channel); D accumulates
+// dW of every tap in registers, one 16 x 16 block of output and input channels
+// per wave.  A lane's operand is four positions of one channel, two bytes each
+// and a position apart: gathered from memory those reads bound the kernel
+// (23 us a layer at 32 x 32 x 32 positions, now 13), so kGradTiles runs with
+// the rows above and below pass through LDS, read once in 8-byte pieces that
+// are all in flight together.  The odd position stride spreads the four
+// position groups of an operand over different banks.  Partial sums per group
+// go to `partial` ([group][9][32][kCin] then 32 bias sums).
+constexpr int kGradTiles = 4;
+
+template <int kCin>
+constexpr int kGradThreads = 64 * 2 * (kCin / 16);
+
 template <int kCin, bool kMask>
-__global__ __launch_bounds__(64) void WeightGradKernel(
+__global__ __launch_bounds__(kGradThreads<kCin>) void WeightGradKernel(
   const uint16_t* __restrict__ grad, const uint16_t* __restrict__ mask,
   const uint16_t* __restrict__ in, int n, int h, int w, int64_t tiles_per_group,
   float* __restrict__ partial) {
-  constexpr int KC = kCin / 16;
   constexpr int kStride = kTaps * kChannels * kCin + kChannels;
-  const int lane = threadIdx.x;
+  constexpr int kThreads = kGradThreads<kCin>;
+  constexpr int kInPieces = kCin / 4, kOutPieces = kChannels / 4;  // of 8 bytes, per position
+  constexpr int kRowLoads = (3 * 18 * kInPieces + kThreads - 1) / kThreads;
+  constexpr int kOutRuns = kThreads / (16 * kOutPieces);  // runs that one pass over `grad` covers
+  __shared__ alignas(8) uint16_t rows[kGradTiles][3 * 18][kCin + 4];
+  __shared__ alignas(8) uint16_t outs[kGradTiles][16][kChannels + 4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int mt = wave & 1, kc = wave >> 1;  // this wave's output and input channels
   const int r16 = lane & 15, q4 = (lane >> 4) * 4;
-  Float4 acc[2][kTaps][KC];
+  Float4 acc[kTaps];
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-    for (int t = 0; t < kTaps; ++t)
-#pragma unroll
-      for (int kc = 0; kc < KC; ++kc) acc[mt][t][kc] = Float4{0.0f, 0.0f, 0.0f, 0.0f};
-  float bsum[2] = {0.0f, 0.0f};
+  for (int t = 0; t < kTaps; ++t) acc[t] = Float4{0.0f, 0.0f, 0.0f, 0.0f};
+  float bsum = 0.0f;
   const int tiles_w = (w + 15) / 16;
   const int64_t tiles = static_cast<int64_t>(n) * h * tiles_w;
   const int64_t first = static_cast<int64_t>(blockIdx.x) * tiles_per_group;
   const int64_t last = first + tiles_per_group < tiles ? first + tiles_per_group : tiles;
-  for (int64_t tile = first; tile < last; ++tile) {
-    const int tx = static_cast<int>(tile % tiles_w);
-    const int64_t row = tile / tiles_w;
-    const int y = static_cast<int>(row % h);
-    const int64_t frame_row0 = row - y;
-    Bf16x4 a[2];
+  int tx = static_cast<int>(first % tiles_w);
+  int64_t row = first / tiles_w;  // frame * h + y
+  int y = static_cast<int>(row % h);
+  for (int64_t base = first; base < last; base += kGradTiles) {
+    uint2 in_piece[kGradTiles][kRowLoads], out_piece[kGradTiles / kOutRuns];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int x = tx * 16 + q4 + i;
-      const bool ok = x < w;
-      const size_t at = ok ? (static_cast<size_t>(row) * w + x) * kChannels : 0;
+    for (int t = 0; t < kGradTiles; ++t) {
+      const bool live = base + t < last;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        uint16_t g = grad[at + 16 * mt + r16];
-        if constexpr (kMask) g = mask[at + 16 * mt + r16] != 0 ? g : 0;
-        g = ok ? g : 0;
-        a[mt][i] = static_cast<short>(g);
-        bsum[mt] += FromBf16(g);
+      for (int k = 0; k < kRowLoads; ++k) {
+        const int c = threadIdx.x + k * kThreads, at = c / kInPieces;
+        const int dy = at / 18 - 1, x = tx * 16 + at % 18 - 1;
+        const bool ok = live && at < 3 * 18 && y + dy >= 0 && y + dy < h && x >= 0 && x < w;
+        in_piece[t][k] = make_uint2(0, 0);
+        if (ok) {
+          in_piece[t][k] = *reinterpret_cast<const uint2*>(
+            in + (static_cast<size_t>(row + dy) * w + x) * kCin + 4 * (c % kInPieces));
+        }
+      }
+      const int run = static_cast<int>(threadIdx.x) / (16 * kOutPieces);
+      if (run == t % kOutRuns) {
+        const int c = threadIdx.x % (16 * kOutPieces), x = tx * 16 + c / kOutPieces;
+        uint2 g = make_uint2(0, 0);
+        if (live && x < w) {
+          const size_t at = (static_cast<size_t>(row) * w + x) * kChannels + 4 * (c % kOutPieces);
+          g = *reinterpret_cast<const uint2*>(grad + at);
+          if constexpr (kMask) {
+            const uint2 m = *reinterpret_cast<const uint2*>(mask + at);
+            g.x &= ((m.x & 0xFFFFu) != 0 ? 0xFFFFu : 0) | (m.x >> 16 != 0 ? 0xFFFF0000u : 0);
+            g.y &= ((m.y & 0xFFFFu) != 0 ? 0xFFFFu : 0) | (m.y >> 16 != 0 ? 0xFFFF0000u : 0);
+          }
+        }
+        out_piece[t / kOutRuns] = g;
+      }
+      if (++tx == tiles_w) {
+        tx = 0;
+        ++row;
+        if (++y == h) y = 0;
+      }
+    }
+    __syncthreads();  // the last batch is read
+#pragma unroll
+    for (int t = 0; t < kGradTiles; ++t) {
+#pragma unroll
+      for (int k = 0; k < kRowLoads; ++k) {
+        const int c = threadIdx.x + k * kThreads, at = c / kInPieces;
+        if (at < 3 * 18) {
+          *reinterpret_cast<uint2*>(&rows[t][at][4 * (c % kInPieces)]) = in_piece[t][k];
+        }
       }
     }
 #pragma unroll
-    for (int t = 0; t < kTaps; ++t) {
-      const int yy = y + t / 3 - 1;
+    for (int k = 0; k < kGradTiles / kOutRuns; ++k) {
+      const int c = threadIdx.x % (16 * kOutPieces);
+      const int t = k * kOutRuns + static_cast<int>(threadIdx.x) / (16 * kOutPieces);
+      *reinterpret_cast<uint2*>(&outs[t][c / kOutPieces][4 * (c % kOutPieces)]) = out_piece[k];
+    }
+    __syncthreads();
 #pragma unroll
-      for (int kc = 0; kc < KC; ++kc) {
+    for (int s = 0; s < kGradTiles; ++s) {
+      Bf16x4 a;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint16_t g = outs[s][q4 + i][16 * mt + r16];
+        a[i] = static_cast<short>(g);
+        bsum += FromBf16(g);
+      }
+#pragma unroll
+      for (int t = 0; t < kTaps; ++t) {
         Bf16x4 b;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int x = tx * 16 + q4 + i, xx = x + t % 3 - 1;
-          const bool ok = x < w && yy >= 0 && yy < h && xx >= 0 && xx < w;
-          const size_t at = ok ? (static_cast<size_t>(frame_row0 + yy) * w + xx) * kCin : 0;
-          const uint16_t v = in[at + 16 * kc + r16];
-          b[i] = static_cast<short>(ok ? v : 0);
+          b[i] = static_cast<short>(rows[s][t / 3 * 18 + q4 + i + t % 3][16 * kc + r16]);
         }
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-          acc[mt][t][kc] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mt], b, acc[mt][t][kc], 0, 0, 0);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
       }
     }
   }
@@ -330,31 +382,37 @@ __global__ __launch_bounds__(64) void WeightGradKernel(
   // 16 kc + r16
   float* p = partial + static_cast<size_t>(blockIdx.x) * kStride;
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
+  for (int t = 0; t < kTaps; ++t)
 #pragma unroll
-    for (int t = 0; t < kTaps; ++t)
-#pragma unroll
-      for (int kc = 0; kc < KC; ++kc)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          p[(t * kChannels + 16 * mt + q4 + i) * kCin + 16 * kc + r16] = acc[mt][t][kc][i];
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt) {
-    float v = bsum[mt];
-    v += __shfl_xor(v, 16);
-    v += __shfl_xor(v, 32);
-    if (lane < 16) p[kTaps * kChannels * kCin + 16 * mt + lane] = v;
+    for (int i = 0; i < 4; ++i)
+      p[(t * kChannels + 16 * mt + q4 + i) * kCin + 16 * kc + r16] = acc[t][i];
+  if (kc == 0) {
+    bsum += __shfl_xor(bsum, 16);
+    bsum += __shfl_xor(bsum, 32);
+    if (lane < 16) p[kTaps * kChannels * kCin + 16 * mt + lane] = bsum;
   }
 }
 
-// out[j] = sum over groups of partial[g][j], groups in order.
-__global__ __launch_bounds__(256) void ReduceKernel(const float* __restrict__ partial,
-                                                    int groups, int stride,
-                                                    float* __restrict__ out) {
+// out[j] = sum over groups of partial[g][j], groups in order.  The reads of
+// kReduceBatch groups are in flight together: one after another they took the
+// memory's latency 256 times (60 us a layer, now 5).
+constexpr int kReduceThreads = 64, kReduceBatch = 32;
+
+__global__ __launch_bounds__(kReduceThreads) void ReduceKernel(const float* __restrict__ partial,
+                                                               int groups, int stride,
+                                                               float* __restrict__ out) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= stride) return;
   float s = 0.0f;
-  for (int g = 0; g < groups; ++g) s += partial[static_cast<size_t>(g) * stride + j];
+  int g = 0;
+  for (; g + kReduceBatch <= groups; g += kReduceBatch) {
+    float v[kReduceBatch];
+#pragma unroll
+    for (int k = 0; k < kReduceBatch; ++k) v[k] = partial[static_cast<size_t>(g + k) * stride + j];
+#pragma unroll
+    for (int k = 0; k < kReduceBatch; ++k) s += v[k];
+  }
+  for (; g < groups; ++g) s += partial[static_cast<size_t>(g) * stride + j];
   out[j] = s;
 }
 
@@ -902,17 +960,17 @@ GJXLResult gjxl_amd_proposal_backward(GJXLAmdProposal* net, const uint8_t* label
     const int cin = LayerInputs(L);
     const int stride = LayerWeights(L) + kChannels;
     if (L == 0) {
-      hipLaunchKernelGGL((WeightGradKernel<kFeatures, true>), dim3(groups), dim3(64), 0, st,
+      hipLaunchKernelGGL((WeightGradKernel<kFeatures, true>), dim3(groups), dim3(kGradThreads<kFeatures>), 0, st,
                          g_cur, mask, in, ni, hi, wi, per_group, net->partial);
     } else if (mask != nullptr) {
-      hipLaunchKernelGGL((WeightGradKernel<kChannels, true>), dim3(groups), dim3(64), 0, st,
+      hipLaunchKernelGGL((WeightGradKernel<kChannels, true>), dim3(groups), dim3(kGradThreads<kChannels>), 0, st,
                          g_cur, mask, in, ni, hi, wi, per_group, net->partial);
     } else {
-      hipLaunchKernelGGL((WeightGradKernel<kChannels, false>), dim3(groups), dim3(64), 0, st,
+      hipLaunchKernelGGL((WeightGradKernel<kChannels, false>), dim3(groups), dim3(kGradThreads<kChannels>), 0, st,
                          g_cur, mask, in, ni, hi, wi, per_group, net->partial);
     }
     GJXL_AMD_TRY(CheckLaunch("WeightGradKernel"));
-    hipLaunchKernelGGL(ReduceKernel, dim3(CeilDiv(stride, 256)), dim3(256), 0, st,
+    hipLaunchKernelGGL(ReduceKernel, dim3(CeilDiv(stride, kReduceThreads)), dim3(kReduceThreads), 0, st,
                        net->partial, groups, stride, net->grads + ParamOffset(L));
     GJXL_AMD_TRY(CheckLaunch("ReduceKernel"));
     (void)cin;
