@@ -938,24 +938,201 @@ __global__ void FillNanKernel(float* __restrict__ p, size_t n) {
 
 // ---- a10: greedy merge, one work group per 64x64 tile ----------------------
 
-constexpr int kStageStrategy[7] = {kDct8, kDct16x8, kDct8x16, kDct16x16,
-                                   kDct32x16, kDct16x32, kDct32x32};
-
 constexpr int kSearchThreads = 64;
 
-// The tile's search state lives across the wave: lane i keeps block i's
-// cell (strategy << 1 | anchor), cost, priority and seven candidate costs in
-// registers.  Every lane runs the search with the same (uniform) values and
-// reads a block's state with readlane, writes it with a per-lane select: a few cycles
-// where an LDS round trip costs about a hundred, and the search is one long
-// chain of such accesses.
+__device__ __forceinline__ bool LaneOf(uint64_t mask) {
+  return __builtin_amdgcn_inverse_ballot_w64(mask);
+}
+
+// The search over one 64x64 tile, block i = 8 ly + lx in lane i.
+//
+// It is a chain of small decisions, so that its time is the instructions of a
+// lone wave.  What a decision asks of the transforms laid so far is kept as
+// masks over the 64 blocks in scalar registers: a boundary is crossed where a
+// block below (right of) it is not in the top row (left column) of its
+// transform.  One decision is taken for every block of a mask at once,
+// whatever the lanes outside it compute; costs are lane registers.  Transforms
+// whose blocks are disjoint and whose order does not matter share a step: a
+// tile of 8 x 8 blocks takes 32 steps instead of 58 decisions.  A walk from
+// anchor to anchor with one readlane per block took 129 us at 1288 x 968, the
+// masks take 10 us (one decision at a time from masks: 30 us).
+//
+// The masks say what the walk (src/codec/ac_strategy.cpp:172-213) says as long
+// as every transform lies whole.  Only a sum of costs that is infinite lets a
+// half be laid that may not be: `torn` then, and the tile is searched again
+// by TornSearch.
 struct TileSearch {
-  int bw, bh;
-  int tbx, tby;  // tile origin in blocks
-  int tw, th;
-  int cell;      // this lane's block
+  uint64_t top = ~uint64_t{0}, left = ~uint64_t{0};  // DCT8 everywhere; set outside the frame
+  uint64_t of16x8 = 0, of8x16 = 0, of16x16 = 0, of32x16 = 0, of16x32 = 0, of32x32 = 0;
+  uint64_t torn = 0;
+  int lane;
   float cost;
-  int prio;
+  float table[7];  // [stage]
+
+  // the value k lanes on; lanes past the tile's end get any
+  __device__ __forceinline__ float Ahead(float v, int k) const {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane + k), __float_as_int(v)));
+  }
+
+  // m's blocks and the w - 1 right of (h - 1 below) each; powers of two
+  __device__ __forceinline__ static uint64_t Wide(uint64_t m, int w) {
+    if (w >= 2) m |= m << 1;
+    if (w >= 4) m |= m << 2;
+    return m;
+  }
+  __device__ __forceinline__ static uint64_t Tall(uint64_t m, int h) {
+    if (h >= 2) m |= m << 8;
+    if (h >= 4) m |= m << 16;
+    return m;
+  }
+  // blocks from which on n in a row (column) are set
+  __device__ __forceinline__ static uint64_t Row(uint64_t m, int n) {
+    m &= m >> 1;
+    return n == 2 ? m : m & m >> 2;
+  }
+  __device__ __forceinline__ static uint64_t Column(uint64_t m, int n) {
+    m &= m >> 8;
+    return n == 2 ? m : m & m >> 16;
+  }
+
+  // transforms whose top left blocks are `anchors`
+  __device__ __forceinline__ void Lay(uint64_t anchors, int strategy, uint64_t& of) {
+    const int cw = CoveredW(strategy), ch = CoveredH(strategy);
+    of |= Tall(Wide(anchors, cw), ch);
+    top |= Wide(anchors, cw);
+    left |= Tall(anchors, ch);
+    cost = LaneOf(anchors) ? table[StageOf(strategy)] : cost;
+  }
+  __device__ __forceinline__ void Clear(uint64_t region) {
+    top &= ~region;
+    left &= ~region;
+    of16x8 &= ~region;
+    of8x16 &= ~region;
+    of16x16 &= ~region;
+    of32x16 &= ~region;
+    of16x32 &= ~region;
+    of32x32 &= ~region;
+    cost = LaneOf(region) ? 0.0f : cost;
+  }
+
+  // src/codec/ac_strategy.cpp:340-384.  The blocks that merges cover are
+  // disjoint whatever the costs are, so that a priority never holds one back.
+  __device__ __forceinline__ void TryMerge(int strategy, uint64_t act, uint64_t& of) {
+    if (act == 0) return;
+    const int cw = CoveredW(strategy), ch = CoveredH(strategy);
+    float current = 0.0f + cost;
+    for (int dy = 0; dy < ch; ++dy)
+      for (int dx = dy == 0 ? 1 : 0; dx < cw; ++dx) current += Ahead(cost, 8 * dy + dx);
+    act &= ~__ballot(table[StageOf(strategy)] >= current);
+    Clear(Tall(Wide(act, cw), ch));
+    Lay(act, strategy, of);
+  }
+
+  // :404-589.  right, below: the halves' candidates, of the lanes half a side
+  // ahead.
+  template <int kBlocks>
+  __device__ __forceinline__ void Divide(uint64_t act, float right, float below) {
+    constexpr int half = kBlocks / 2;
+    constexpr int vs = kBlocks == 2 ? kDct16x8 : kDct32x16;
+    constexpr int hs = kBlocks == 2 ? kDct8x16 : kDct16x32;
+    constexpr int ss = kBlocks == 2 ? kDct16x16 : kDct32x32;
+    uint64_t& of_vs = kBlocks == 2 ? of16x8 : of32x16;
+    uint64_t& of_hs = kBlocks == 2 ? of8x16 : of16x32;
+    uint64_t& of_ss = kBlocks == 2 ? of16x16 : of32x32;
+    // nothing crosses the tile's own boundary
+    constexpr uint64_t kLastRows = ~(~uint64_t{0} >> 8 * kBlocks);
+    constexpr uint64_t kLastColumns = 0x0101010101010101ull * (0xFF & ~(0xFF >> kBlocks));
+    const uint64_t row = Row(top, kBlocks), column = Column(left, kBlocks);
+    act &= row & (row >> 8 * kBlocks | kLastRows) & column & (column >> kBlocks | kLastColumns);
+    if (act == 0) return;
+    const uint64_t no_v = ~(column >> half), no_h = ~(row >> 8 * half);
+    const uint64_t no_vl = no_v | of_vs, no_vr = no_v | of_vs >> half;
+    const uint64_t no_ht = no_h | of_hs, no_hb = no_h | of_hs >> 8 * half;
+    // the quadrants' costs, each summed row by row
+    float q00 = 0.0f + cost, q01, q10, q11;
+    if constexpr (kBlocks == 4) {
+      const float c1 = Ahead(cost, 1), c2 = Ahead(cost, 8), c3 = Ahead(cost, 9);
+      q00 = ((q00 + c1) + c2) + c3;
+    }
+    q01 = Ahead(q00, half);
+    q10 = Ahead(q00, 8 * half);
+    q11 = Ahead(q00, 9 * half);
+    constexpr float kUnavailable = 3.40282347e+38f;
+    const float vl = LaneOf(no_vl) ? kUnavailable : table[StageOf(vs)];
+    const float vr = LaneOf(no_vr) ? kUnavailable : right;
+    const float ht = LaneOf(no_ht) ? kUnavailable : table[StageOf(hs)];
+    const float hb = LaneOf(no_hb) ? kUnavailable : below;
+    const float sq = table[StageOf(ss)];
+    const float vcost = StdMin(vl, q00 + q10) + StdMin(vr, q01 + q11);
+    const float hcost = StdMin(ht, q00 + q01) + StdMin(hb, q10 + q11);
+    const uint64_t lay_s = act & __ballot(sq < vcost) & __ballot(sq < hcost);
+    const uint64_t v = act & ~lay_s & __ballot(vcost < hcost), h = act & ~lay_s & ~v;
+    const uint64_t lay_vl = v & __ballot(vl < q00 + q10), lay_vr = v & __ballot(vr < q01 + q11);
+    const uint64_t lay_ht = h & __ballot(ht < q00 + q01), lay_hb = h & __ballot(hb < q10 + q11);
+    // an unavailable half loses against every finite sum
+    torn |= (lay_vl & no_vl) | (lay_vr & no_vr) | (lay_ht & no_ht) | (lay_hb & no_hb);
+    const uint64_t lay_v = lay_vl | lay_vr << half, lay_h = lay_ht | lay_hb << 8 * half;
+    if ((lay_s | lay_v | lay_h) == 0) return;
+    Clear(Tall(Wide(lay_s, kBlocks) | Wide(lay_v, half), kBlocks) |
+          Tall(Wide(lay_h, kBlocks), half));
+    Lay(lay_s, ss, of_ss);
+    Lay(lay_v, vs, of_vs);
+    Lay(lay_h, hs, of_hs);
+  }
+
+  // :591-773 SearchTile over tw x th blocks; this lane's cell
+  __device__ __forceinline__ int Run(int tw, int th) {
+    const int lx = lane % 8, ly = lane / 8;
+    const float right2 = Ahead(table[StageOf(kDct16x8)], 1);
+    const float below2 = Ahead(table[StageOf(kDct8x16)], 8);
+    const float right4 = Ahead(table[StageOf(kDct32x16)], 2);
+    const float below4 = Ahead(table[StageOf(kDct16x32)], 16);
+    const uint64_t at2 = __ballot(lx + 2 <= tw && ly + 2 <= th);
+    const uint64_t at4 = __ballot(lx + 4 <= tw && ly + 4 <= th);
+    const uint64_t even = __ballot(lx % 2 == 0 && ly % 2 == 0);
+    const uint64_t fourth = __ballot(lx % 4 == 0 && ly % 4 == 0);
+    // The squares on even blocks are disjoint, and no transform crosses their
+    // sides; so are the halves in an odd last column and row.
+    TryMerge(kDct16x8, __ballot(lx + 1 == tw && ly + 2 <= th) & even, of16x8);
+    Divide<2>(at2 & even, right2, below2);
+    TryMerge(kDct8x16, __ballot(lx + 2 <= tw && ly + 1 == th) & even, of8x16);
+    // the same one size up
+    Divide<4>(at4 & fourth, right4, below4);
+    TryMerge(kDct16x32, __ballot(lx + 4 <= tw && ly + 2 <= th && ly + 4 > th) & fourth, of16x32);
+    TryMerge(kDct32x16, __ballot(lx + 2 <= tw && lx + 4 > tw && ly + 4 <= th) & fourth, of32x16);
+    // The other squares, row by row.  In an even row only odd columns are
+    // left, two apart: disjoint, and what one lays leaves the side that it
+    // shares with the next as it was, so that the row is one step.  In an odd
+    // row each overlaps the next.
+    for (uint64_t rest = at2 & ~even; rest != 0;) {
+      const int first = __builtin_ctzll(rest);
+      const uint64_t step = first & 8 ? rest & -rest : rest & (uint64_t{0xFF} << (first & ~7));
+      rest &= ~step;
+      Divide<2>(step, right2, below2);
+    }
+    for (uint64_t rest = at4 & even & ~fourth; rest != 0; rest &= rest - 1) {
+      Divide<4>(rest & -rest, right4, below4);
+    }
+    int strategy = kDct8;
+    strategy = LaneOf(of16x8) ? kDct16x8 : strategy;
+    strategy = LaneOf(of8x16) ? kDct8x16 : strategy;
+    strategy = LaneOf(of16x16) ? kDct16x16 : strategy;
+    strategy = LaneOf(of32x16) ? kDct32x16 : strategy;
+    strategy = LaneOf(of16x32) ? kDct16x32 : strategy;
+    strategy = LaneOf(of32x32) ? kDct32x32 : strategy;
+    return strategy << 1 | static_cast<int>(LaneOf(top & left));
+  }
+};
+
+// The same search for a tile in which a transform was laid across another's
+// boundary (see TileSearch): block by block, with the walk itself.  Every lane
+// holds the same values; a block's cell and cost are read with readlane and
+// written with a per-lane select.
+struct TornSearch {
+  int tw, th;
+  int lane;
+  int cell = (kDct8 << 1) | 1;
+  float cost;
   float table[7];  // [stage]
 
   __device__ __forceinline__ int Cell(int lx, int ly) const {
@@ -964,41 +1141,27 @@ struct TileSearch {
   __device__ __forceinline__ float Cost(int lx, int ly) const {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cost), ly * 8 + lx));
   }
-  __device__ __forceinline__ int Prio(int lx, int ly) const {
-    return __builtin_amdgcn_readlane(prio, ly * 8 + lx);
-  }
-  int lane;
-  // a uniform value into one lane: a compare and a select
-  __device__ __forceinline__ void SetCell(int lx, int ly, int v) {
-    cell = lane == ly * 8 + lx ? v : cell;
-  }
-  __device__ __forceinline__ void SetCost(int lx, int ly, float v) {
-    cost = lane == ly * 8 + lx ? v : cost;
-  }
-  __device__ __forceinline__ void SetPrio(int lx, int ly, int v) {
-    prio = lane == ly * 8 + lx ? v : prio;
-  }
   // strategy is a constant at every call site, so the stage folds
   __device__ __forceinline__ float Table(int strategy, int lx, int ly) const {
     return __int_as_float(
       __builtin_amdgcn_readlane(__float_as_int(table[StageOf(strategy)]), ly * 8 + lx));
   }
 
-  __device__ __forceinline__ void Set(int lx, int ly, int strategy) {
+  __device__ __forceinline__ void Lay(int lx, int ly, int strategy, float c) {
     const int cw = CoveredW(strategy), ch = CoveredH(strategy);
-    for (int dy = 0; dy < ch; ++dy)
-      for (int dx = 0; dx < cw; ++dx)
-        SetCell(lx + dx, ly + dy, (strategy << 1) | (dx == 0 && dy == 0));
+    const int dx = lane % 8 - lx, dy = lane / 8 - ly;
+    const bool covered = dx >= 0 && dx < cw && dy >= 0 && dy < ch, anchor = dx == 0 && dy == 0;
+    cell = covered ? strategy << 1 | static_cast<int>(anchor) : cell;
+    cost = covered ? (anchor ? c : 0.0f) : cost;
   }
 
-  // src/codec/ac_strategy.cpp:172-191 (global block coordinates)
-  __device__ __forceinline__ bool CrossesHorizontal(int sx, int y, int ex) const {
-    if (sx >= bw || y >= bh || y % 8 == 0) return false;
-    ex = min(ex, bw);
-    const int limit = sx & ~7;
-    while (sx != limit && !(Cell(sx - tbx, y - tby) & 1)) --sx;
+  // src/codec/ac_strategy.cpp:172-191
+  __device__ __forceinline__ bool CrossesHorizontal(int sx, int y, int n) const {
+    if (sx >= tw || y >= th || y % 8 == 0) return false;
+    const int ex = min(sx + n, tw);
+    while (sx != 0 && !(Cell(sx, y) & 1)) --sx;
     for (int x = sx; x < ex;) {
-      const int c = Cell(x - tbx, y - tby);
+      const int c = Cell(x, y);
       if (!(c & 1)) return true;
       x += CoveredW(c >> 1);
     }
@@ -1006,60 +1169,37 @@ struct TileSearch {
   }
 
   // :193-213
-  __device__ __forceinline__ bool CrossesVertical(int x, int sy, int ey) const {
-    if (x >= bw || sy >= bh || x % 8 == 0) return false;
-    ey = min(ey, bh);
-    const int limit = sy & ~7;
-    while (sy != limit && !(Cell(x - tbx, sy - tby) & 1)) --sy;
+  __device__ __forceinline__ bool CrossesVertical(int x, int sy, int n) const {
+    if (x >= tw || sy >= th || x % 8 == 0) return false;
+    const int ey = min(sy + n, th);
+    while (sy != 0 && !(Cell(x, sy) & 1)) --sy;
     for (int y = sy; y < ey;) {
-      const int c = Cell(x - tbx, y - tby);
+      const int c = Cell(x, y);
       if (!(c & 1)) return true;
       y += CoveredH(c >> 1);
     }
     return false;
   }
 
-  __device__ __forceinline__ void SetCostForTransform(int lx, int ly, int strategy, float c) {
-    const int cw = CoveredW(strategy), ch = CoveredH(strategy);
-    for (int dy = 0; dy < ch; ++dy)
-      for (int dx = 0; dx < cw; ++dx) SetCost(lx + dx, ly + dy, 0.0f);
-    SetCost(lx, ly, c);
-  }
-
   // :340-384
-  __device__ __forceinline__ void TryMerge(int strategy, int lx, int ly, int priority) {
-    const int cw = CoveredW(strategy), ch = CoveredH(strategy);
+  __device__ __forceinline__ void TryMerge(int strategy, int lx, int ly) {
     float current = 0.0f;
-    for (int dy = 0; dy < ch; ++dy) {
-      for (int dx = 0; dx < cw; ++dx) {
-        if (Prio(lx + dx, ly + dy) >= priority) return;
-        current += Cost(lx + dx, ly + dy);
-      }
-    }
+    for (int dy = 0; dy < CoveredH(strategy); ++dy)
+      for (int dx = 0; dx < CoveredW(strategy); ++dx) current += Cost(lx + dx, ly + dy);
     const float candidate = Table(strategy, lx, ly);
     if (candidate >= current) return;
-    for (int dy = 0; dy < ch; ++dy) {
-      for (int dx = 0; dx < cw; ++dx) {
-        SetCost(lx + dx, ly + dy, 0.0f);
-        SetPrio(lx + dx, ly + dy, priority);
-      }
-    }
-    Set(lx, ly, strategy);
-    SetCost(lx, ly, candidate);
+    Lay(lx, ly, strategy, candidate);
   }
 
   // :404-589
-  __device__ __forceinline__ void FirstLevelDivision(int blocks, int lx, int ly) {
+  __device__ __forceinline__ void Divide(int blocks, int lx, int ly) {
     const int half = blocks / 2;
-    const int bx = tbx + lx, by = tby + ly;
-    if (CrossesHorizontal(bx, by, bx + blocks) ||
-        CrossesHorizontal(bx, by + blocks, bx + blocks) ||
-        CrossesVertical(bx, by, by + blocks) ||
-        CrossesVertical(bx + blocks, by, by + blocks)) {
+    if (CrossesHorizontal(lx, ly, blocks) || CrossesHorizontal(lx, ly + blocks, blocks) ||
+        CrossesVertical(lx, ly, blocks) || CrossesVertical(lx + blocks, ly, blocks)) {
       return;
     }
-    const bool allow_v = !CrossesVertical(bx + half, by, by + blocks);
-    const bool allow_h = !CrossesHorizontal(bx, by + half, bx + blocks);
+    const bool allow_v = !CrossesVertical(lx + half, ly, blocks);
+    const bool allow_h = !CrossesHorizontal(lx, ly + half, blocks);
     float q00 = 0.0f, q01 = 0.0f, q10 = 0.0f, q11 = 0.0f;  // [row][col]
     for (int dy = 0; dy < blocks; ++dy) {
       for (int dx = 0; dx < blocks; ++dx) {
@@ -1085,83 +1225,76 @@ struct TileSearch {
     const float vcost = StdMin(vl, q00 + q10) + StdMin(vr, q01 + q11);
     const float hcost = StdMin(ht, q00 + q01) + StdMin(hb, q10 + q11);
     if (sq < vcost && sq < hcost) {
-      Set(lx, ly, ss);
-      SetCostForTransform(lx, ly, ss, sq);
+      Lay(lx, ly, ss, sq);
     } else if (vcost < hcost) {
-      if (vl < q00 + q10) { Set(lx, ly, vs); SetCostForTransform(lx, ly, vs, vl); }
-      if (vr < q01 + q11) { Set(lx + half, ly, vs); SetCostForTransform(lx + half, ly, vs, vr); }
+      if (vl < q00 + q10) Lay(lx, ly, vs, vl);
+      if (vr < q01 + q11) Lay(lx + half, ly, vs, vr);
     } else {
-      if (ht < q00 + q01) { Set(lx, ly, hs); SetCostForTransform(lx, ly, hs, ht); }
-      if (hb < q10 + q11) { Set(lx, ly + half, hs); SetCostForTransform(lx, ly + half, hs, hb); }
+      if (ht < q00 + q01) Lay(lx, ly, hs, ht);
+      if (hb < q10 + q11) Lay(lx, ly + half, hs, hb);
+    }
+  }
+
+  // :591-773 SearchTile
+  __device__ __forceinline__ void Run() {
+    for (int y = 0; tw % 2 == 1 && y + 2 <= th; y += 2) TryMerge(kDct16x8, tw - 1, y);
+    for (int y = 0; y < th; y += 2) {
+      for (int x = 0; x + 2 <= tw; x += 2) {
+        if (y + 1 < th) Divide(2, x, y);
+        else TryMerge(kDct8x16, x, y);
+      }
+    }
+    for (int y = 0; y + 2 <= th; y += 4) {
+      for (int x = 0; x + 4 <= tw; x += 4) {
+        if (y + 3 < th) Divide(4, x, y);
+        else TryMerge(kDct16x32, x, y);
+      }
+    }
+    for (int y = 0; tw % 4 >= 2 && y + 4 <= th; y += 4) TryMerge(kDct32x16, tw & ~3, y);
+    for (int y = 0; y + 1 < th; ++y) {
+      for (int x = 1 - y % 2; x + 1 < tw; x += 2 - y % 2) Divide(2, x, y);
+    }
+    for (int y = 0; y + 3 < th; y += 2) {
+      for (int x = y % 4 == 0 ? 2 : 0; x + 3 < tw; x += y % 4 == 0 ? 4 : 2) Divide(4, x, y);
     }
   }
 };
 
 // grid: one work group of one wave per tile.  Lane i loads block i's seven
-// candidate costs and initialises its state; the wave runs the search
-// (src/codec/ac_strategy.cpp:591-773 SearchTile); lane i stores block i's
-// cell.
+// candidate costs; the wave runs the search; lane i stores block i's cell.
 __global__ __launch_bounds__(kSearchThreads) void SearchKernel(
   const float* __restrict__ costs, int bw, int bh, float target,
   uint8_t* __restrict__ out_cells) {
   const int tiles_w = (bw + 7) / 8;
-  const int tile = blockIdx.x;
-  TileSearch s;
-  s.bw = bw;
-  s.bh = bh;
-  s.tbx = (tile % tiles_w) * 8;
-  s.tby = (tile / tiles_w) * 8;
-  s.tw = min(8, bw - s.tbx);
-  s.th = min(8, bh - s.tby);
+  const int tbx = static_cast<int>(blockIdx.x) % tiles_w * 8;  // tile origin in blocks
+  const int tby = static_cast<int>(blockIdx.x) / tiles_w * 8;
+  const int tw = min(8, bw - tbx), th = min(8, bh - tby);
   const int i = threadIdx.x, lx = i % 8, ly = i / 8;
-  s.lane = i;
-  const bool inside = lx < s.tw && ly < s.th;
+  const bool inside = lx < tw && ly < th;
   const size_t plane = static_cast<size_t>(bw) * bh;
-  const size_t block = static_cast<size_t>(s.tby + (inside ? ly : 0)) * bw + s.tbx + (inside ? lx : 0);
-  float v[7];
+  const size_t block = static_cast<size_t>(tby + (inside ? ly : 0)) * bw + tbx + (inside ? lx : 0);
+  TileSearch s;
+  s.lane = i;
 #pragma unroll
-  for (int st = 0; st < 7; ++st) v[st] = costs[st * plane + block];
+  for (int st = 0; st < 7; ++st) s.table[st] = costs[st * plane + block];
 #pragma unroll
-  for (int st = 0; st < 7; ++st) s.table[st] = inside ? v[st] : 0.0f;
-  s.cell = (kDct8 << 1) | 1;
-  s.prio = 0;
+  for (int st = 0; st < 7; ++st) s.table[st] = inside ? s.table[st] : 0.0f;
   const float baseline = 1.0f + -0.4f / (target + 1.4f);
-  s.cost = inside ? s.table[StageOf(kDct8)] * baseline : 0.0f;
-  constexpr int kMergeStrategy[4] = {kDct16x8, kDct8x16, kDct16x32, kDct32x16};
-  constexpr int kMergePriority[4] = {2, 2, 4, 4};
+  const float dct8_cost = inside ? s.table[StageOf(kDct8)] * baseline : 0.0f;
+  s.cost = dct8_cost;
+  int cell = s.Run(tw, th);
+  if (s.torn != 0) {
+    TornSearch t;
+    t.tw = tw;
+    t.th = th;
+    t.lane = i;
+    t.cost = dct8_cost;
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int st = kMergeStrategy[m];
-    const int cw = CoveredW(st), ch = CoveredH(st);
-    for (int y = 0; y + ch <= s.th; y += ch) {
-      for (int x = 0; x + cw <= s.tw; x += cw) {
-        if (y + 3 < s.th && x + 3 < s.tw) {
-          if (st == kDct16x32) {
-            if ((y | x) % 4 == 0) s.FirstLevelDivision(4, x, y);
-            continue;
-          }
-          if (st == kDct32x16) continue;
-        }
-        if ((st == kDct16x32 && y % 4 != 0) || (st == kDct32x16 && x % 4 != 0)) continue;
-        if (y + 1 < s.th && x + 1 < s.tw) {
-          if (st == kDct8x16) {
-            if ((y | x) % 2 == 0) s.FirstLevelDivision(2, x, y);
-            continue;
-          }
-          if (st == kDct16x8) continue;
-        }
-        if ((st == kDct8x16 && y % 2 == 1) || (st == kDct16x8 && x % 2 == 1)) continue;
-        s.TryMerge(st, x, y, kMergePriority[m]);
-      }
-    }
+    for (int st = 0; st < 7; ++st) t.table[st] = s.table[st];
+    t.Run();
+    cell = t.cell;
   }
-  for (int y = 0; y + 1 < s.th; ++y)
-    for (int x = 0; x + 1 < s.tw; ++x)
-      if ((y | x) % 2 != 0) s.FirstLevelDivision(2, x, y);
-  for (int y = 0; y + 3 < s.th; y += 2)
-    for (int x = 0; x + 3 < s.tw; x += 2)
-      if ((y | x) % 4 != 0) s.FirstLevelDivision(4, x, y);
-  if (inside) out_cells[block] = static_cast<uint8_t>(s.cell);
+  if (inside) out_cells[block] = static_cast<uint8_t>(cell);
 }
 
 template <int kStrategy>

@@ -83,3 +83,27 @@ def test_ac_search_full_size_4032x3024(device):
     _check_costs(got_costs[:, :16], want)
     kinds = np.unique(cells >> 1)
     assert len(kinds) >= 4, kinds
+
+
+@pytest.mark.parametrize("kind", ["close", "infinite"])
+def test_search_tile_shapes(device, kind):
+    """The merge over every width and height of a tile in blocks, alone and as
+    the last tile of a larger frame: whole tiles, odd and even remainders.
+    The candidates are near the sums that they compete with, so that every
+    shape is laid somewhere, ties included; "infinite" adds infinite and NaN
+    costs to all stages, DCT8 too."""
+    rng = np.random.default_rng(11)
+    blocks = np.array([1, 2, 2, 4, 8, 8, 16], np.float32).reshape(7, 1, 1)
+    laid = set()
+    for bh in (*range(1, 10), 13, 22):
+        for bw in (*range(1, 10), 15, 52):
+            costs = blocks * rng.choice(np.float32([0.7, 0.8, 0.85, 1.0, 1.2]), (7, bh, bw))
+            if kind == "infinite":
+                at = rng.random(costs.shape)
+                costs[at < 0.08] = np.inf
+                costs[at > 0.98] = np.nan
+            costs = costs.astype(np.float32)
+            got = device.ac_strategy_search(device.array(costs)).numpy()
+            assert np.array_equal(got, binding.search_from_costs(costs)), (bw, bh)
+            laid |= set(np.unique(got >> 1).tolist())
+    assert laid == {0, 4, 5, 6, 7, 10, 11}
