@@ -325,6 +325,16 @@ struct CostShape {
   static constexpr int kPositions = kNx * kNy;
 };
 
+// Waves per SIMD: a group has two, and a CU's LDS holds three groups (two of
+// DCT8's, with its 16 candidates' own values).  The kernel issues for two
+// thirds of its time and waits at its barriers for the rest, the more the
+// longer one wave's ordered sums take: the third group (the pixel mask, 4 KB
+// a group, out of LDS and the registers bounded to 80) and those sums with
+// their reads ahead and on different banks took the seven strategies from 614
+// to 553 us at 1288 x 968.
+template <int kStrategy>
+constexpr int kCostWavesPerSimd = kStrategy == kDct8 ? 4 : 6;
+
 // One work group's work: kCands anchor positions of one 64x64 tile
 // (group.y), positions group.x * kCands + k of the tile's raster list, or
 // (kListed) entries group.x * kCands + k of a list of anchors (x | y << 16,
@@ -353,18 +363,20 @@ __device__ __forceinline__ void CostWork(
   constexpr bool kPad = H == 32;
   constexpr int HP = kPad ? H + 1 : H, NP = W * HP;
   // Storage order (coefficient index i = u * H + v when H >= W) is padded
-  // the same way: slot i + i / H; for H < W (i = v * W + u) it is unpadded.
-  constexpr bool kPadStorage = kPad && H >= W;
-  auto storage_slot = [](int i) { return kPadStorage ? i + i / H : i; };
+  // likewise, by four words so that 16 values stay aligned to 16 bytes.  Four
+  // more words per plane spread the planes of the ordered sums, one lane
+  // each, over the banks.
+  auto storage_slot = [](int i) { return kPad ? i + 4 * (i / 32) : i; };
+  constexpr int AS = (kPad ? N + N / 8 : N) + 4, BS = kPad ? NP : N + 4;
+  static_assert(AS >= NP && BS >= NP && AS % 4 == 0 && BS % 4 == 0);
   // A: pixels (transposed, [x][y], column stride HP); then sqrt(|rounded|)
   //    in (padded) storage order
   // B: coefficients ([v][u]); residuals (transposed, [u][v], column stride
   //    HP); loss terms ([y][x])
   // T: binary64 rows of the separable passes, stride TS
-  __shared__ float A[KC * NP];
-  __shared__ float B[KC * NP];
+  __shared__ alignas(16) float A[KC * AS];
+  __shared__ alignas(16) float B[KC * BS];
   __shared__ double T[KC * H * TS];
-  __shared__ float mask[K * N];  // pixel mask of each candidate, raster order
   __shared__ int nnz[K][3];
   __shared__ float sums[K][3][2];
   __shared__ float qn[K];
@@ -437,18 +449,16 @@ __device__ __forceinline__ void CostWork(
 
   // Every global read of the work group is issued here, in the order the
   // results are needed (reads complete in issue order): the pixels, which
-  // the first barrier waits for, then the mask, the quantisation table
-  // entries of the elements this thread quantises and the quant-field and
-  // CfL inputs, which reach LDS behind the forward passes.
+  // the first barrier waits for, then the quantisation table entries of the
+  // elements this thread quantises and the quant-field and CfL inputs, which
+  // reach LDS behind the forward passes.
   // Each strategy's slots hold a whole number of elements per thread, so
   // every read below is unconditional: a candidate that is not launched
   // reads element 0 of the plane and discards it.  (A read under a branch
   // makes the compiler wait for the earlier reads at the branch's join.)
   constexpr int kPer = KC * N / kCostThreads;
-  constexpr int kMaskPer = K * N / kCostThreads;
   static_assert(N % 64 == 0, "a wave's elements lie in one candidate channel");
-  static_assert(KC * N == kPer * kCostThreads && K * N == kMaskPer * kCostThreads,
-                "whole elements per thread");
+  static_assert(KC * N == kPer * kCostThreads, "whole elements per thread");
   float pixel[kPer], dq_e[kPer], inv_e[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
@@ -460,17 +470,6 @@ __device__ __forceinline__ void CostWork(
     const size_t at = c * plane + static_cast<size_t>(by * 8 + r / W) * width + bx * 8 + r % W;
     const float v = opsin[live ? at : 0];
     pixel[j] = live ? v : 0.0f;
-  }
-  float mask_e[kMaskPer];
-#pragma unroll
-  for (int j = 0; j < kMaskPer; ++j) {
-    const int e = tid + j * kCostThreads;
-    const int k = e / N, r = e % N;
-    int bx, by;
-    const bool live = candidate(k, &bx, &by);
-    const size_t at = static_cast<size_t>(by * 8 + r / W) * width + bx * 8 + r % W;
-    const float v = pixel_mask[live ? at : 0];
-    mask_e[j] = live ? v : 0.0f;
   }
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
@@ -518,7 +517,7 @@ __device__ __forceinline__ void CostWork(
     const int e = tid + j * kCostThreads;
     if (e < KC * N) {
       const int kc = e / N, r = e % N;
-      A[kc * NP + (r % W) * HP + r / W] = pixel[j];
+      A[kc * AS + (r % W) * HP + r / W] = pixel[j];
     }
   }
   __syncthreads();
@@ -535,7 +534,7 @@ __device__ __forceinline__ void CostWork(
     const int g = task % (W / kOut), r = (task / (W / kOut)) * 64 + lane;
     if (r < kRows) {
       const int kc = r / H, y = r % H;
-      const float* src = A + kc * NP + y;
+      const float* src = A + kc * AS + y;
       double acc[kOut] = {};
 #pragma unroll 4
       for (int x = 0; x < W; ++x) {
@@ -563,15 +562,10 @@ __device__ __forceinline__ void CostWork(
         for (int j = 0; j < kOut; ++j) acc[j] += fvT[y * H + g * kOut + j] * v;
       }
 #pragma unroll
-      for (int j = 0; j < kOut; ++j) B[kc * N + (g * kOut + j) * W + u] = static_cast<float>(acc[j]);
+      for (int j = 0; j < kOut; ++j) B[kc * BS + (g * kOut + j) * W + u] = static_cast<float>(acc[j]);
     }
   }
-  // the reads issued at the start: mask into LDS, quant norms and CfL
-#pragma unroll
-  for (int j = 0; j < kMaskPer; ++j) {
-    const int e = tid + j * kCostThreads;
-    if (e < K * N) mask[e] = mask_e[j];
-  }
+  // the reads issued at the start: quant norms and CfL
   if (tid < K && ok) {
     float norm;
     if constexpr (kBlocks == 1) {
@@ -609,12 +603,12 @@ __device__ __forceinline__ void CostWork(
       const int k = kc / 3, c = kc % 3;
       const int v = rem / W, u = rem % W;
       const int i = CoefficientIndex<W, H>(v, u);
-      const float dec = B[e] - B[(k * 3 + 1) * N + rem] * cfl[k][c];
+      const float dec = B[kc * BS + rem] - B[(k * 3 + 1) * BS + rem] * cfl[k][c];
       const float scaled = dec * inv_e[j] * qn[k];
       const float rounded = roundf(scaled);
       const float diff = scaled - rounded;
       residual[j] = dq_e[j] * diff;
-      A[kc * NP + storage_slot(i)] = sqrtf(fabsf(rounded));
+      A[kc * AS + storage_slot(i)] = sqrtf(fabsf(rounded));
       // a wave's 64 elements lie in one candidate channel (N is a multiple
       // of 64): one LDS add of the wave's nonzero count
       const int count = __popcll(__ballot(rounded != 0.0f));
@@ -628,16 +622,31 @@ __device__ __forceinline__ void CostWork(
     if (e < KC * N) {
       const int kc = e / N, rem = e % N;
       const int v = rem / W, u = rem % W;
-      B[kc * NP + u * HP + v] = residual[j];
+      B[kc * BS + u * HP + v] = residual[j];
     }
   }
   __syncthreads();
+  // The mask values of this lane's outputs of the last pass, one task a wave,
+  // read behind the pass before it: kept in LDS from the start they were the
+  // 4 KB that held a CU at two work groups.
+  constexpr int kColTasks = kColBlocks * (H / kOut);
+  static_assert(kColTasks <= kWaves);
+  const int col = wave / (H / kOut) * 64 + lane, y0 = wave % (H / kOut) * kOut;
+  const bool last = wave < kColTasks && col < kCols;
+  float m[kOut];
+  if (last) {
+    const int k = col / (3 * W);
+    const size_t at = valid[k] ? static_cast<size_t>(bys[k] * 8 + y0) * width + bxs[k] * 8 + col % W : 0;
+    const size_t step = valid[k] ? width : 0;
+#pragma unroll
+    for (int j = 0; j < kOut; ++j) m[j] = pixel_mask[at + j * step];
+  }
   // Inverse horizontal: T[v][x] = sum_u res(v, u) * ih[u][x].
   for (int task = wave; task < kRowBlocks * (W / kOut); task += kWaves) {
     const int g = task % (W / kOut), r = (task / (W / kOut)) * 64 + lane;
     if (r < kRows) {
       const int kc = r / H, v = r % H;
-      const float* src = B + kc * NP + v;
+      const float* src = B + kc * BS + v;
       double acc[kOut] = {};
 #pragma unroll 4
       for (int u = 0; u < W; ++u) {
@@ -653,33 +662,28 @@ __device__ __forceinline__ void CostWork(
   __syncthreads();
   // Inverse vertical and the masked 8th power (:935-952) into B, raster.
   // 12, 0, 4 for X, Y, B (selects, not a table: no memory access)
-  for (int task = wave; task < kColBlocks * (H / kOut); task += kWaves) {
-    const int g = task % (H / kOut), col = (task / (H / kOut)) * 64 + lane;
-    if (col < kCols) {
-      const int kc = col / W, x = col % W;
-      const int k = kc / 3, c = kc % 3;
-      const float mask_offset = c == 0 ? 12.0f : c == 2 ? 4.0f : 0.0f;
-      const double* src = T + kc * H * TS + x;
-      double acc[kOut] = {};
+  if (last) {
+    const int kc = col / W, x = col % W;
+    const int k = kc / 3, c = kc % 3;
+    const float mask_offset = c == 0 ? 12.0f : c == 2 ? 4.0f : 0.0f;
+    const double* src = T + kc * H * TS + x;
+    double acc[kOut] = {};
 #pragma unroll 4
-      for (int v = 0; v < H; ++v) {
-        const double t = src[v * TS];
+    for (int v = 0; v < H; ++v) {
+      const double t = src[v * TS];
 #pragma unroll
-        for (int j = 0; j < kOut; ++j) acc[j] += iv[v * H + g * kOut + j] * t;
-      }
+      for (int j = 0; j < kOut; ++j) acc[j] += iv[v * H + y0 + j] * t;
+    }
 #pragma unroll
-      for (int j = 0; j < kOut; ++j) {
-        const int y = g * kOut + j;
-        float weighted = 0.0f;
-        if (valid[k]) {
-          const float m = mask[k * N + y * W + x];
-          weighted = (m + mask_offset) * static_cast<float>(acc[j]);
-          weighted *= weighted;
-          weighted *= weighted;
-          weighted *= weighted;
-        }
-        B[kc * N + y * W + x] = weighted;
+    for (int j = 0; j < kOut; ++j) {
+      float weighted = 0.0f;
+      if (valid[k]) {
+        weighted = (m[j] + mask_offset) * static_cast<float>(acc[j]);
+        weighted *= weighted;
+        weighted *= weighted;
+        weighted *= weighted;
       }
+      B[kc * BS + (y0 + j) * W + x] = weighted;
     }
   }
   __syncthreads();
@@ -687,20 +691,29 @@ __device__ __forceinline__ void CostWork(
   if (tid < K * 6) {
     const int k = tid / 6, c = (tid / 2) % 3, kind = tid % 2;
     // kind 0: A in (padded) storage order; kind 1: B in raster order
-    const float* src = kind == 0 ? A + (k * 3 + c) * NP : B + (k * 3 + c) * N;
-    const bool padded = kind == 0 && kPadStorage;
+    const float* src = kind == 0 ? A + (k * 3 + c) * AS : B + (k * 3 + c) * BS;
+    const int column = kPad && kind == 0 ? 36 : 32;  // words from 32 values to the next 32
+    // the next 16 values are on their way while 16 are added
+    float4 cur[4], next[4];
+    auto read = [&](int base, float4* v) __attribute__((always_inline)) {
+      const float4* at = reinterpret_cast<const float4*>(
+        __builtin_assume_aligned(src + base / 32 * column + base % 32, 16));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = at[q];
+    };
     float s = 0.0f;
-    // batches of 16: the loads of a batch issue before its ordered adds
-    for (int base = 0; base < N; base += 16) {
-      // kind 0 reads the padded slots i + i / H: a batch lies in one padded
-      // column for H >= 16 and in two for H = 8 (the second one word on)
-      const float* lo = src + base + (padded ? base / H : 0);
-      const float* hi = lo + (padded && H < 16 ? 1 : 0);
-      float v[16];
+    read(0, cur);
+    for (int base = 16; base <= N; base += 16) {
+      if (base < N) read(base, next);
 #pragma unroll
-      for (int m = 0; m < 16; ++m) v[m] = (m >= 8 && H < 16 ? hi : lo)[m];
+      for (int q = 0; q < 4; ++q) {
+        s += cur[q].x;
+        s += cur[q].y;
+        s += cur[q].z;
+        s += cur[q].w;
+      }
 #pragma unroll
-      for (int m = 0; m < 16; ++m) s += v[m];
+      for (int q = 0; q < 4; ++q) cur[q] = next[q];
     }
     sums[k][c][kind] = s;
   }
@@ -740,7 +753,7 @@ __device__ __forceinline__ void CostWork(
 // (consecutive in dispatch order) share its pixels, and the XCD-aware order
 // keeps them on one L2.
 template <int kStrategy>
-__global__ __launch_bounds__(kCostThreads) void CandidateCostKernel(
+__global__ __launch_bounds__(kCostThreads, kCostWavesPerSimd<kStrategy>) void CandidateCostKernel(
   const float* __restrict__ opsin, int width, int height,
   const float* __restrict__ quant_field, const float* __restrict__ pixel_mask,
   const int8_t* __restrict__ y_to_x, const int8_t* __restrict__ y_to_b,
@@ -784,7 +797,7 @@ __global__ __launch_bounds__(256) void CandidateListKernel(
 
 // Listed candidates: group x takes entries x * kCands ... of the list.
 template <int kStrategy>
-__global__ __launch_bounds__(kCostThreads) void CandidateCostListKernel(
+__global__ __launch_bounds__(kCostThreads, kCostWavesPerSimd<kStrategy>) void CandidateCostListKernel(
   const float* __restrict__ opsin, int width, int height,
   const float* __restrict__ quant_field, const float* __restrict__ pixel_mask,
   const int8_t* __restrict__ y_to_x, const int8_t* __restrict__ y_to_b,
