@@ -1278,10 +1278,11 @@ constexpr int kDcYRing = 16;           // >= 2D slots of quantized Y per row
 constexpr int kDcRowThreads = kDcGroup / 2;
 constexpr int kDcWorkGroup = 2 * kDcRowThreads;
 
-// (1 << 24) / (i + 1) for the arguments the predictor forms: e >> shift
-// is below 64 and the final weight sum minus one below 32, so one table of
-// 128 entries covers both (filled per work group).
-constexpr int kReciprocals = 128;
+// (1 << 24) / (i + 1) for the arguments the predictor forms: the final weight
+// sum minus one is below 32, and e >> shift below 64, whose entries are kept
+// times the largest weights 13 and 12 (filled per work group).
+constexpr int kReciprocals = 64, kReciprocals13 = 64, kReciprocals12 = 128;
+constexpr int kReciprocalWords = 192;
 
 // Bit width of e + 1 for a 32-bit e (33 for 2^32 - 1).
 __device__ __forceinline__ int BitWidthPlusOne(uint32_t e) {
@@ -1292,11 +1293,10 @@ __device__ __forceinline__ int BitWidth32(uint32_t v) {
 }
 
 // What the row below reads of a sample (x, y): its quantized value,
-// prediction error and sub-predictor errors, and q(x, y - 1).
+// prediction error and sub-predictor errors.
 struct DcCell {
   int32_t q = 0, err = 0;
   uint32_t e[4] = {0, 0, 0, 0};
-  int32_t q_up = 0;
 };
 
 // The predictor state a row keeps in registers: its own last two samples.
@@ -1312,9 +1312,13 @@ struct DcRowState {
 // 32-bit arithmetic gives the 64-bit results.
 constexpr int32_t kDcNarrowQ = 1 << 18;
 constexpr int32_t kDcNarrowErr = 1 << 21;
+// The 32-bit evaluation adds this to samples times eight and to predictions:
+// differences are the same, the order as unsigned words is the order as
+// signed ones, and the signed 24-bit multiplier does not see it.
+constexpr int32_t kDcBias = 1 << 30;
 
 // One sample (x, y) of one channel from its north-east, north and
-// north-west cells (the north-north value is n.q_up) and the row state:
+// north-west cells and the row state:
 // weighted prediction, quantisation of the residual, update of the row
 // state.  Returns the sample's cell.  Row 0 reads all-zero north cells, so
 // the reference's zero errors and zero "up" value above the first row need
@@ -1335,14 +1339,12 @@ __device__ __forceinline__ DcCell DcSample(const DcCell& ne, const DcCell& n, co
   using I = std::conditional_t<kWide, int64_t, int32_t>;
   using U = std::conditional_t<kWide, uint64_t, uint32_t>;
   constexpr uint8_t kCoeff[7] = {16, 10, 7, 7, 7, 0, 0};
-  constexpr uint8_t kMaxWeights[4] = {13, 12, 12, 12};
+  constexpr I kBias = kWide ? 0 : kDcBias;
   // quantized neighbours
   const I up = n.q;
   const I W_ = x ? st.q1 : up;
   const I N_ = y ? up : W_;
-  const I NW_ = x && y ? nw.q : W_;
   const I NE_ = y && has_ne ? ne.q : N_;
-  const I NN_ = y > 1 ? n.q_up : N_;
   // Predict (prediction.h:75-123)
   uint32_t weights[4];
   uint32_t weight_sum = 0;
@@ -1352,11 +1354,11 @@ __device__ __forceinline__ DcCell DcSample(const DcCell& ne, const DcCell& n, co
     const uint32_t e_ne = has_ne ? ne.e[i] : north;
     const uint32_t e_nw = x ? nw.e[i] + st.e2[i] : north;
     const uint32_t e = north + e_ne + e_nw;
-    int shift = BitWidthPlusOne(e) - 6;
+    // (in 32 bits an error is below 2^29 whatever the step, and e + 1 is the
+    // sum of at most six and one: no overflow)
+    int shift = (kWide ? BitWidthPlusOne(e) : 32 - __clz(static_cast<int>(e + 1))) - 6;
     if (shift < 0) shift = 0;
-    // k * r as k * (r - 1) + k: r - 1 < 2^24 fits the 24-bit multiplier
-    const uint32_t k = kMaxWeights[i];
-    weights[i] = 4 + ((__umul24(reciprocal[e >> shift] - 1, k) + k) >> shift);
+    weights[i] = 4 + (reciprocal[(i == 0 ? kReciprocals13 : kReciprocals12) + (e >> shift)] >> shift);
     weight_sum += weights[i];
   }
   const unsigned log_weight = BitWidth32(weight_sum) - 1;
@@ -1370,7 +1372,9 @@ __device__ __forceinline__ DcCell DcSample(const DcCell& ne, const DcCell& n, co
   const I en = n.err;
   const I enw = x ? nw.err : en;
   const I ene = has_ne ? ne.err : en;
-  const I n8 = N_ * 8, w8 = W_ * 8, ne8 = NE_ * 8, nw8 = NW_ * 8, nn8 = NN_ * 8;
+  // (the coefficients of the north-west and north-north samples are zero)
+  static_assert(kCoeff[5] == 0 && kCoeff[6] == 0, "unused samples");
+  const I n8 = N_ * 8 + kBias, w8 = W_ * 8 + kBias, ne8 = NE_ * 8 + kBias;
   // the reference's sums of products, with the three equal error
   // coefficients of the last one factored (the same integer)
   static_assert(kCoeff[2] == kCoeff[3] && kCoeff[3] == kCoeff[4], "factored coefficients");
@@ -1385,14 +1389,15 @@ __device__ __forceinline__ DcCell DcSample(const DcCell& ne, const DcCell& n, co
     c3 = __mul24(enw + en + ene, static_cast<int32_t>(kCoeff[2]));
   }
   I pred[4];
-  pred[0] = w8 + ne8 - n8;
+  pred[0] = w8 - n8 + ne8;
   pred[1] = n8 - (c1 >> 5);
   pred[2] = w8 - (c2 >> 5);
-  pred[3] = n8 - ((c3 + (nn8 - n8) * kCoeff[5] + (nw8 - w8) * kCoeff[6]) >> 5);
+  pred[3] = n8 - (c3 >> 5);
   I sum = static_cast<I>((weight_sum >> 1) - 1);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    // within the 32-bit bounds |pred| < 2^23 fits the signed 24-bit multiplier
+    // within the 32-bit bounds |pred| < 2^23 fits the signed 24-bit multiplier,
+    // which drops the bias
     if constexpr (kWide) {
       sum += pred[i] * static_cast<I>(weights[i]);
     } else {
@@ -1402,30 +1407,46 @@ __device__ __forceinline__ DcCell DcSample(const DcCell& ne, const DcCell& n, co
   // the table entry is below 2^24: a signed 32-bit operand
   I prediction = static_cast<I>(
     (static_cast<int64_t>(sum) *
-     static_cast<int64_t>(static_cast<int32_t>(reciprocal[weight_sum - 1]))) >> 24);
+     static_cast<int64_t>(static_cast<int32_t>(reciprocal[weight_sum - 1]))) >> 24) + kBias;
   if (((en ^ ew) | (en ^ enw)) <= 0) {
     I lo = w8 < ne8 ? w8 : ne8;
     lo = lo < n8 ? lo : n8;
     I hi = w8 > ne8 ? w8 : ne8;
     hi = hi > n8 ? hi : n8;
-    prediction = prediction < lo ? lo : (prediction > hi ? hi : prediction);
+    prediction = prediction < lo ? lo : prediction;
+    prediction = prediction > hi ? hi : prediction;
   }
-  const I predicted = (prediction + 3) >> 3;
+  const I predicted = (prediction + (3 - kBias)) >> 3;
   // quantise the residual (dc_quantization.cpp:176-203)
   float residual = value * inv;
   residual -= static_cast<float>(predicted);
-  if (residual > -0.62f && residual < 0.62f) residual = 0;
-  float rounded = roundf(residual);
-  if (rounded > 2 || rounded < -2) rounded = roundf(residual * 0.5f) * 2;
-  // rounded holds an integer
-  const int32_t ir = static_cast<int32_t>(rounded);
+  int32_t ir;
+  if constexpr (kWide) {
+    if (residual > -0.62f && residual < 0.62f) residual = 0;
+    float rounded = roundf(residual);
+    if (rounded > 2 || rounded < -2) rounded = roundf(residual * 0.5f) * 2;
+    // rounded holds an integer
+    ir = static_cast<int32_t>(rounded);
+  } else {
+    // The same by truncation: from 0.62 up to 2^23 in magnitude, r + 0.5 and
+    // r / 2 + 0.5 never round up to an integer that they are below.  Larger
+    // ones, clamped so that the conversions hold, and NaN, which the clamp
+    // takes to a bound, leave q's bound: the sample is flagged.
+    constexpr float kLimit = 1 << 30;
+    residual = __builtin_amdgcn_fmed3f(residual, -kLimit, kLimit);
+    const float half = copysignf(0.5f, residual);
+    const int32_t one = static_cast<int32_t>(residual + half);
+    const int32_t two = static_cast<int32_t>(__builtin_fmaf(residual, 0.5f, half)) << 1;
+    ir = fabsf(residual) >= 2.5f ? two : one;
+    ir = fabsf(residual) < 0.62f ? 0 : ir;
+  }
   DcCell out;
   // the low 32 bits of predicted + ir
   out.q = static_cast<int32_t>(static_cast<uint32_t>(predicted) + static_cast<uint32_t>(ir));
-  out.q_up = n.q;
   // Update (prediction.h:124-144); unsigned arithmetic wraps where a 32-bit
   // evaluation leaves its bounds (the sample is then flagged)
-  const I scaled = static_cast<I>(static_cast<U>(static_cast<I>(out.q)) << 3);
+  const I scaled =
+    static_cast<I>((static_cast<U>(static_cast<I>(out.q)) << 3) + static_cast<U>(kBias));
   out.err = static_cast<int32_t>(static_cast<U>(prediction) - static_cast<U>(scaled));
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -1434,11 +1455,8 @@ __device__ __forceinline__ DcCell DcSample(const DcCell& ne, const DcCell& n, co
       const U magnitude = dd < 0 ? U(0) - static_cast<U>(dd) : static_cast<U>(dd);
       out.e[i] = static_cast<uint32_t>((magnitude + 3) >> 3);
     } else {
-      // |pred - scaled| + 3 on sign-flipped words (the order of signed words
-      // as unsigned ones); within the bounds the difference fits 32 bits
-      constexpr uint32_t kFlip = 0x80000000u;
-      out.e[i] = __usad(static_cast<uint32_t>(pred[i]) ^ kFlip,
-                        static_cast<uint32_t>(scaled) ^ kFlip, 3u) >> 3;
+      // |pred - scaled| + 3: biased words are positive within the bounds
+      out.e[i] = __usad(static_cast<uint32_t>(pred[i]), static_cast<uint32_t>(scaled), 3u) >> 3;
     }
     st.e2[i] = st.e1[i];
     st.e1[i] = active ? out.e[i] : 0u;
@@ -1466,12 +1484,11 @@ __device__ __forceinline__ DcCell CellFromLaneAbove(const int32_t (&edge)[8], co
   for (int i = 0; i < 4; ++i) {
     r.e[i] = static_cast<uint32_t>(FromLaneAbove(edge[2 + i], static_cast<int32_t>(c.e[i])));
   }
-  r.q_up = FromLaneAbove(edge[6], c.q_up);
   return r;
 }
 
 struct DcShared {
-  uint32_t reciprocal[kReciprocals];
+  uint32_t reciprocal[kReciprocalWords];
   // [channel slot][writing wave][x % kDcEdgeRing]: lane 63's cells; slot
   // kDcEdgeRing of every ring holds zeros (row 0's north)
   int32_t edge[2][2][kDcEdgeRing + 1][8];
@@ -1587,7 +1604,6 @@ struct DcWavefront {
           e[1] = cells[j].err;
 #pragma unroll
           for (int i = 0; i < 4; ++i) e[2 + i] = static_cast<int32_t>(cells[j].e[i]);
-          e[6] = cells[j].q_up;
         }
       }
       // orders the edge and Y rings between waves
@@ -1609,7 +1625,12 @@ __global__ __launch_bounds__(kDcWorkGroup) void DcQuantKernel(
   const QuantizerState* __restrict__ qstate, int extra_precision,
   int32_t* __restrict__ quantized) {
   __shared__ DcShared sh;
-  if (threadIdx.x < kReciprocals) sh.reciprocal[threadIdx.x] = (1u << 24) / (threadIdx.x + 1);
+  if (threadIdx.x < kReciprocals) {
+    const uint32_t r = (1u << 24) / (threadIdx.x + 1);
+    sh.reciprocal[threadIdx.x] = r;
+    sh.reciprocal[kReciprocals13 + threadIdx.x] = 13 * r;
+    sh.reciprocal[kReciprocals12 + threadIdx.x] = 12 * r;
+  }
   if (threadIdx.x < 2 * 2 * 8) {
     sh.edge[threadIdx.x / 16][(threadIdx.x / 8) % 2][kDcEdgeRing][threadIdx.x % 8] = 0;
   }
