@@ -974,8 +974,9 @@ __device__ __forceinline__ bool LaneOf(uint64_t mask) {
 // whatever the lanes outside it compute; costs are lane registers.  Transforms
 // whose blocks are disjoint and whose order does not matter share a step: a
 // tile of 8 x 8 blocks takes 32 steps instead of 58 decisions.  A walk from
-// anchor to anchor with one readlane per block took 129 us at 1288 x 968, the
-// masks take 10 us (one decision at a time from masks: 30 us).
+// anchor to anchor with one readlane per block took 108 us at 512 x 512, 129 us
+// at 1288 x 968 and 172 us at 4032 x 3024; the masks take 8, 10 and 15 us (one
+// decision at a time from masks: 30 us at 1288 x 968).
 //
 // The masks say what the walk (src/codec/ac_strategy.cpp:172-213) says as long
 // as every transform lies whole.  Only a sum of costs that is infinite lets a

@@ -401,27 +401,39 @@ __global__ __launch_bounds__(256) void AdjustFieldKernel(
 }
 
 // Non-negative float maxima through their bit patterns (order-free), one
-// atomic per work group.
+// atomic per maximum and work group.  A work group walks down 256 columns,
+// rows [blockIdx.y * rows, + rows), with the row above in registers: a column
+// and row per element by 64-bit division bound the kernel before (37 us at
+// 512x512, 74 us at 4032x3024; now 11 and 65).
 __global__ __launch_bounds__(256) void MatrixStatsKernel(
   const float* __restrict__ opsin, int width, int height, int stride,
-  size_t plane, uint32_t* __restrict__ stats) {
+  size_t plane, int rows, uint32_t* __restrict__ stats) {
   const float* X = opsin;
   const float* Y = opsin + plane;
   const float* B = opsin + 2 * plane;
   float xe = 0.0f, be = 0.0f, ex = 0.0f;
-  const size_t n = static_cast<size_t>(width) * height;
-  for (size_t k = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; k < n;
-       k += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const int x = static_cast<int>(k % width), y = static_cast<int>(k / width);
-    if (x < 1 || y < 1) continue;
-    const size_t i = static_cast<size_t>(y) * stride + x, l = i - 1, u = i - stride;
-    xe = DStdMax(xe, DStdMax(fabsf(X[i] - X[l]), fabsf(X[i] - X[u])));
-    const float d = B[i] - Y[i];
-    be = DStdMax(be, DStdMax(fabsf(d - (B[l] - Y[l])), fabsf(d - (B[u] - Y[u]))));
-    float e = B[i] - 1.2f * Y[i];
-    if (e >= 0.0f) {
-      e *= fabsf(B[i] - B[l]) + fabsf(B[i] - B[u]);
-      ex = DStdMax(ex, e);
+  const int x = blockIdx.x * 256 + threadIdx.x;
+  const int first = static_cast<int>(blockIdx.y) * rows, last = min(height, first + rows);
+  const int y0 = max(first, 1);
+  if (x >= 1 && x < width && y0 < last) {
+    size_t i = static_cast<size_t>(y0 - 1) * stride + x;
+    float xu = X[i], yu = Y[i], bu = B[i];
+#pragma unroll 4
+    for (int y = y0; y < last; ++y) {
+      i += stride;
+      const float xi = X[i], yi = Y[i], bi = B[i];
+      const float xl = X[i - 1], yl = Y[i - 1], bl = B[i - 1];
+      xe = DStdMax(xe, DStdMax(fabsf(xi - xl), fabsf(xi - xu)));
+      const float d = bi - yi;
+      be = DStdMax(be, DStdMax(fabsf(d - (bl - yl)), fabsf(d - (bu - yu))));
+      float e = bi - 1.2f * yi;
+      if (e >= 0.0f) {
+        e *= fabsf(bi - bl) + fabsf(bi - bu);
+        ex = DStdMax(ex, e);
+      }
+      xu = xi;
+      yu = yi;
+      bu = bi;
     }
   }
   uint32_t v[3] = {__float_as_uint(xe), __float_as_uint(be), __float_as_uint(ex)};
@@ -2017,10 +2029,13 @@ GJXLResult LaunchAdjustField(hipStream_t s, const uint8_t* cells, int width,
 GJXLResult LaunchMatrixStats(hipStream_t s, const float* opsin, int width,
                              int height, int padded_w, int padded_h,
                              uint32_t* stats) {
-  hipLaunchKernelGGL(MatrixStatsKernel,
-                     dim3(ReductionGroups(static_cast<size_t>(width) * height)), dim3(256), 0,
+  // four rows a group, or as many as keep the groups, whose atomics meet on
+  // three words, at about a thousand
+  const uint32_t strips = CeilDiv(width, 256);
+  const int rows = std::max(4, static_cast<int>(CeilDiv(height, std::max(1024u / strips, 1u))));
+  hipLaunchKernelGGL(MatrixStatsKernel, dim3(strips, CeilDiv(height, rows)), dim3(256), 0,
                      s, opsin, width, height, padded_w,
-                     static_cast<size_t>(padded_w) * padded_h, stats);
+                     static_cast<size_t>(padded_w) * padded_h, rows, stats);
   return CheckLaunch("MatrixStatsKernel");
 }
 

@@ -189,3 +189,21 @@ def test_quantizer_selection(device, w, h, kind):
         dc = int(float(np.float32(s.policy()["quant_dc"]) * np.float32(4096.0)) * 1.6)
         assert int(q[2]) == (max(dc, 1) if want > dc else want)
     s.close()
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (1, 9), (9, 1), (2, 2), (257, 5), (256, 33), (513, 1030)])
+def test_matrix_statistics(device, w, h):
+    """The matrix statistics over strips of 256 columns and segments of four
+    and more rows: no neighbour at all, one row or column, a strip of one
+    column, segments that end with the image.  Maxima, so that any order
+    gives the reference's value bit for bit."""
+    rng = np.random.default_rng(w * 31 + h)
+    pw, ph = (w + 7) // 8 * 8, (h + 7) // 8 * 8
+    ops = rng.uniform(-0.02, 0.6, (3, ph, pw)).astype(np.float32)
+    fe = {"opsin": ops, "pre": ops, "cells": np.ones((ph // 8, pw // 8), np.uint8),
+          "quant_field": np.full((ph // 8, pw // 8), 0.5, np.float32)}
+    s = gjxl_amd.AqSession(device, w, h)
+    s.prepare(*_device_inputs(device, fe), 1.0)
+    device.synchronize()
+    got = s.buffer("stats", (3,)).numpy()
+    _same("stats", got, binding.aq_setup(fe, w, h)["stats"])
