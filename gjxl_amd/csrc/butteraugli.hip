@@ -38,6 +38,7 @@
 #include "butteraugli.h"
 #include "libm_port.h"
 #include "tables.h"
+#include "tile_mirror.h"
 
 namespace gjxl_amd {
 namespace {
@@ -52,12 +53,6 @@ struct Taps {
 constexpr float kSigmas[kSigmaCount] = {1.2f, 7.15593339443f, 3.22489901262f,
                                         1.56416327805f, 2.7f};
 
-// Mirrored coordinate for -size <= c < 2 * size (one reflection), by selects.
-// (Both scales are at least 8 pixels a side.)
-__device__ __forceinline__ int BMirrorOnce(int c, int size) {
-  c = c < 0 ? -c - 1 : c;
-  return c >= size ? 2 * size - 1 - c : c;
-}
 __device__ __forceinline__ float BMax(float a, float b) { return a < b ? b : a; }
 
 // ---- Gaussian blurs --------------------------------------------------------
@@ -438,6 +433,9 @@ __device__ __forceinline__ void Absorbance(float r, float g, float b, bool clamp
 // tiles are read: four reads per sample of an image that the full scale has
 // just pulled into the caches, instead of a launch that wrote and re-read
 // three planes.
+// Both scales are at least 8 pixels a side, and every lane of a tile reads: in
+// a plane narrower than 33 pixels or lower than 9 also further outside it than
+// one reflection reaches (TileMirror holds those reads inside the image).
 constexpr int kOpsinTileW = 64, kOpsinTileH = 16;
 constexpr int kOpsinRows = kOpsinTileH / (kThreads / kOpsinTileW);  // per thread
 
@@ -472,11 +470,11 @@ __global__ __launch_bounds__(kThreads) void OpsinDynamicsKernel(OpsinArgs args) 
   constexpr int kStripCount = 3 * TH * 4;
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / 64));
-  const int sx = BMirrorOnce(x0 - 2 + lane, w);
+  const int sx = TileMirror(x0 - 2 + lane, w);
   const int e = min(static_cast<int>(threadIdx.x), kStripCount - 1);
   const int strip_c = e / 4 / TH;
-  const int strip_y = BMirrorOnce(y0 - 2 + e / 4 % TH, h);
-  const int strip_x = BMirrorOnce(x0 - 2 + 64 + e % 4, w);
+  const int strip_y = TileMirror(y0 - 2 + e / 4 % TH, h);
+  const int strip_x = TileMirror(x0 - 2 + 64 + e % 4, w);
   float rows[kWaveRows];
   float strip;
   if (at.scale == 0) {
@@ -484,7 +482,7 @@ __global__ __launch_bounds__(kThreads) void OpsinDynamicsKernel(OpsinArgs args) 
     for (int i = 0; i < kWaveRows; ++i) {
       const int row = wave * kWaveRows + i;
       const int c = row / TH, r = row % TH;
-      rows[i] = rgb[c * n + static_cast<size_t>(BMirrorOnce(y0 - 2 + r, h)) * w + sx];
+      rows[i] = rgb[c * n + static_cast<size_t>(TileMirror(y0 - 2 + r, h)) * w + sx];
     }
     strip = rgb[strip_c * n + static_cast<size_t>(strip_y) * w + strip_x];
   } else {
@@ -518,12 +516,12 @@ __global__ __launch_bounds__(kThreads) void OpsinDynamicsKernel(OpsinArgs args) 
 #pragma unroll
     for (int i = 0; i < kWaveRows; ++i) {
       const int row = wave * kWaveRows + i;
-      quads[i] = read(row / TH, sx, BMirrorOnce(y0 - 2 + row % TH, h));
+      quads[i] = read(row / TH, sx, TileMirror(y0 - 2 + row % TH, h));
     }
     const Quad strip_quad = read(strip_c, strip_x, strip_y);
 #pragma unroll
     for (int i = 0; i < kWaveRows; ++i) {
-      rows[i] = sum(quads[i], sx, BMirrorOnce(y0 - 2 + (wave * kWaveRows + i) % TH, h));
+      rows[i] = sum(quads[i], sx, TileMirror(y0 - 2 + (wave * kWaveRows + i) % TH, h));
     }
     strip = sum(strip_quad, strip_x, strip_y);
   }
