@@ -5,6 +5,7 @@
 #include <cmath>
 
 #include "common.h"
+#include "tile_mirror.h"
 
 namespace gjxl_amd {
 namespace {
@@ -21,12 +22,6 @@ __device__ __forceinline__ int MirrorInt(int c, int size) {
     phase = rem == 0 ? 0 : period - rem;
   }
   return static_cast<int>(phase < size ? phase : period - 1 - phase);
-}
-
-// MirrorInt for -size <= c < 2 * size (one reflection), by selects.
-__device__ __forceinline__ int MirrorOnce(int c, int size) {
-  c = c < 0 ? -c - 1 : c;
-  return c >= size ? 2 * size - 1 - c : c;
 }
 
 struct GaborishWeights {
@@ -113,8 +108,10 @@ __device__ __forceinline__ void EpfPixel(Sample S, float bis, int x, int y,
   for (int c = 0; c < 3; ++c) out[c] = sum[c] / weight_sum;
 }
 
-// kOnce: w and h are at least 4, so every coordinate the tile mirrors (at
-// most 4 outside the image) needs one reflection.
+// kOnce: w and h are at least 4, so every coordinate that an output needs (at
+// most 4 outside the image) needs one reflection; what a lane reads further
+// outside, in an image narrower than 34 or lower than 10, lies inside it
+// (TileMirror) and is never used.
 template <bool kOnce>
 __global__ __launch_bounds__(256) void LoopFilterKernel(
   const float* __restrict__ in, int in_stride, size_t in_plane, int w, int h,
@@ -129,7 +126,7 @@ __global__ __launch_bounds__(256) void LoopFilterKernel(
   const int x0 = tile_index.x * kLfTileW, y0 = tile_index.y * kLfTileH;
   const int bw = (w + 7) / 8;
   const size_t plane = static_cast<size_t>(w) * h;
-  auto mirror = [](int c, int size) { return kOnce ? MirrorOnce(c, size) : MirrorInt(c, size); };
+  auto mirror = [](int c, int size) { return kOnce ? TileMirror(c, size) : MirrorInt(c, size); };
   // The tile's 3 x kRawH rows of kRawW = 64 + 8 columns: each wave reads
   // kWaveRows whole rows, one lane per column of the first 64, with the row
   // address uniform (scalar arithmetic); the last 8 columns of every row are

@@ -3,9 +3,10 @@ in the line for every extent, and is the mirrored one wherever an output can
 need it.
 
 Compiles the product header for the host with g++ and walks over every tile
-and tile position of the opsin dynamics (64x16 tiles, halo 2, planes of 8
-pixels and more a side), at the full scale and at the half scale, which is read
-from the full one at twice the coordinate.
+and tile position of the kernels that use it: the opsin dynamics (64x16 tiles,
+halo 2, planes of 8 pixels and more a side, at the full scale and at the half
+scale, which is read from the full one at twice the coordinate) and the loop
+filters (64x16 tiles, halo 4, planes of 4 pixels and more).
 """
 import subprocess
 from pathlib import Path
@@ -44,8 +45,10 @@ static void Line(int size, int tile, int halo, int full) {
 }
 
 int main() {
-  for (int size = 8; size <= 1100; ++size) {
+  for (int size = 4; size <= 1100; ++size) {
     for (int tile : {64, 16}) {
+      Line(size, tile, 4, 0);
+      if (size < 8) continue;
       Line(size, tile, 2, 0);
       Line(size, tile, 2, 2 * size);
       Line(size, tile, 2, 2 * size - 1);
