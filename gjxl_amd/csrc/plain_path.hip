@@ -286,10 +286,14 @@ GJXLResult RunFront(GJXLAmdPlainPath* p, const uint8_t* srgb, size_t row_stride,
 }
 
 // The frame statistics of the coefficients that the device stream has coded
-// at p->coded, on the side stream, and their copy to the host; nothing waits.
+// at p->coded, on the side stream, and their copy to the host with the loop's
+// error flag (every update stands before the coding); nothing waits.
 GJXLResult TokensBegin(GJXLAmdPlainPath* p) {
   hipStream_t st = p->side->stream;
   GJXL_AMD_TRY(Check(hipStreamWaitEvent(st, p->coded, 0), "hipStreamWaitEvent"));
+  const uint32_t* stats = AqBuffer<uint32_t>(p->session, GJXL_AMD_AQ_STATS);
+  GJXL_AMD_TRY(Check(hipMemcpyAsync(p->host_words + 4, stats + 7, 4, hipMemcpyDeviceToHost, st),
+                     "hipMemcpyAsync(AQ error)"));
   gjxl_amd::TokenizerUseDevice(p->tokenizer, p->side);
   const GJXLResult r = gjxl_amd::FrameStatisticsEnqueue(
     p->tokenizer, AqBuffer<int32_t>(p->session, GJXL_AMD_AQ_QUANTIZED), p->cells,
@@ -304,10 +308,14 @@ GJXLResult TokensBegin(GJXLAmdPlainPath* p) {
 
 // The CPU-chosen tokenization inputs of effort 7 (coefficient orders and the
 // adaptive block-context map) from those statistics, the tokens and their
-// count; waits for the side stream twice.
+// count; waits for the side stream twice.  A loop that has failed ends here,
+// before any token reaches the caller's buffers.
 GJXLResult TokensFinish(GJXLAmdPlainPath* p) {
   hipStream_t st = p->side->stream;
   GJXL_AMD_TRY(Check(hipStreamSynchronize(st), "hipStreamSynchronize"));
+  if (p->host_words[4] != 0) {
+    return Fail(GJXL_ERROR_INTERNAL, "Adaptive quantization produced an invalid block distance");
+  }
   GJXL_AMD_TRY(gjxl_amd::FrameStatisticsResult(p->tokenizer, p->host_statistics,
                                                p->statistics));
   GJXL_AMD_TRY(gjxl_amd_entropy_inputs_from_statistics(p->statistics, p->options.effort,
@@ -414,13 +422,9 @@ GJXLResult RunBack(GJXLAmdPlainPath* p, bool costs_ready) {
   }
   // evaluations with a comparison (the unjudged last pass has none)
   p->evaluations_run = unjudged ? it : it + 1;
-  // the loop's error flag and scores, read by FinishRun
-  uint32_t* host = p->host_words;
-  uint32_t* stats = AqBuffer<uint32_t>(p->session, GJXL_AMD_AQ_STATS);
-  GJXL_AMD_TRY(Check(hipMemcpyAsync(host + 4, stats + 7, 4, hipMemcpyDeviceToHost, st),
-                     "hipMemcpyAsync(AQ error)"));
+  // the scores, read by FinishRun
   if (p->evaluations_run > 0) {
-    GJXL_AMD_TRY(Check(hipMemcpyAsync(host + 8, p->score_words, 4 * p->evaluations_run,
+    GJXL_AMD_TRY(Check(hipMemcpyAsync(p->host_words + 8, p->score_words, 4 * p->evaluations_run,
                                       hipMemcpyDeviceToHost, st), "hipMemcpyAsync(scores)"));
   }
   if (!tokens_done) GJXL_AMD_TRY(TokensFinish(p));
@@ -473,13 +477,9 @@ GJXLResult ReadTokens(GJXLAmdPlainPath* p, const GJXLAmdTokenOutput* out) {
 // or the caller's buffers when this returns.
 GJXLResult FinishRun(GJXLAmdPlainPath* p, bool costs_ready, const GJXLAmdTokenOutput* tokens) {
   GJXLResult r = RunBack(p, costs_ready);
-  const bool looped = r == GJXL_OK;
-  if (looped) r = ReadTokens(p, tokens);
+  if (r == GJXL_OK) r = ReadTokens(p, tokens);
   const GJXLResult side = Check(hipStreamSynchronize(p->side->stream), "hipStreamSynchronize");
   const GJXLResult main = Check(hipStreamSynchronize(p->device->stream), "hipStreamSynchronize");
-  if (looped && main == GJXL_OK && p->host_words[4] != 0) {
-    return Fail(GJXL_ERROR_INTERNAL, "Adaptive quantization produced an invalid block distance");
-  }
   GJXL_AMD_TRY(r);
   GJXL_AMD_TRY(side);
   GJXL_AMD_TRY(main);

@@ -165,6 +165,32 @@ def test_native_plain_path_matches_oracle_digests(device, name):
     path.close()
 
 
+def test_failed_run_leaves_the_token_buffers(device):
+    """A loop whose block distances are not finite (an intensity target far
+    from the 255 that the loop decodes with) fails with its own diagnostic and
+    before a token reaches the caller's buffers; the path then runs as if it
+    had not."""
+    w, h = 200, 136
+    srgb = synthetic.generate(w, h, seed=5)
+    path = gjxl_amd.NativePlainPath(device, w, h)
+    path.run(srgb)
+    want, scores = path.tokens(), path.scores()
+    path.reconfigure(w, h, intensity_target=1e5)
+    for buffer in (path.values, path.contexts, path.group_offsets):
+        buffer.array[:] = 7
+    print("plain path with an infinite block distance", flush=True)
+    with pytest.raises(gjxl_amd.GjxlError, match="INTERNAL.*invalid block distance"):
+        path.run(srgb)
+    for buffer in (path.values, path.contexts, path.group_offsets):
+        assert (buffer.array == 7).all()
+    path.reconfigure(w, h, intensity_target=255.0)
+    path.run(srgb)
+    assert path.scores() == scores
+    got = path.tokens()
+    assert all(np.array_equal(got[k], want[k]) for k in want)
+    path.close()
+
+
 def test_cpp_caller_matches_oracle_digests(tmp_path):
     """A C++ program built with g++ against include/gjxl_amd.h alone
     (tests/plain_path_caller.cpp) drives the path and writes its outputs."""
