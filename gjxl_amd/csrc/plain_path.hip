@@ -40,6 +40,11 @@ namespace {
 constexpr int kMaxMarks = 48;
 constexpr int kMaxEvaluations = 8;
 
+// What the side stream's marks around the tokens' stages stand before or after
+enum TokenMark {
+  kBeforeStatistics, kAfterInputs, kAfterTokenize, kBeforeRead, kAfterRead, kTokenMarks
+};
+
 // The path's own device buffers
 enum PathBuffer {
   kSrgb, kLinear, kOpsin, kPreprocessed, kQuantField, kStrategyMask, kPixelMask,
@@ -88,9 +93,8 @@ struct GJXLAmdPlainPath {
   hipEvent_t linear_ready = nullptr;
   hipEvent_t reference_ready = nullptr;
   // the tokens of the last pass run on that stream too, from its coded
-  // coefficients on; tokens_read orders their read-back before the run's end
+  // coefficients on
   hipEvent_t coded = nullptr;
-  hipEvent_t tokens_read = nullptr;
   // pinned host words: token status (4), AQ error (1), scores (kMaxEvaluations)
   uint32_t* host_words = nullptr;
   // pinned host copy of the frame statistics; the entropy inputs chosen
@@ -98,10 +102,13 @@ struct GJXLAmdPlainPath {
   uint32_t* host_statistics = nullptr;
   GJXLAmdFrameStatistics* statistics = nullptr;
   GJXLAmdEntropyInputs* entropy_inputs = nullptr;
-  // stage marks of the last run
+  // stage marks of the last run, and those of its tokens' stages on the side
+  // stream (TokenMark; whether the tokens were read back)
   hipEvent_t marks[kMaxMarks] = {};
   int32_t mark_stage[kMaxMarks] = {};
   int mark_count = 0;
+  hipEvent_t token_marks[kTokenMarks] = {};
+  bool tokens_read = false;
   uint64_t token_count = 0;
   float scores[kMaxEvaluations] = {};
   bool ran = false;
@@ -121,6 +128,10 @@ GJXLResult Mark(GJXLAmdPlainPath* p, int32_t stage) {
   if (p->mark_count >= kMaxMarks) return GJXL_OK;
   p->mark_stage[p->mark_count] = stage;
   return Check(hipEventRecord(p->marks[p->mark_count++], p->device->stream), "hipEventRecord");
+}
+
+GJXLResult MarkTokens(GJXLAmdPlainPath* p, TokenMark mark) {
+  return Check(hipEventRecord(p->token_marks[mark], p->side->stream), "hipEventRecord");
 }
 
 // The extent fields of a path and the byte size of each of its own buffers
@@ -291,6 +302,7 @@ GJXLResult RunFront(GJXLAmdPlainPath* p, const uint8_t* srgb, size_t row_stride,
 GJXLResult TokensBegin(GJXLAmdPlainPath* p) {
   hipStream_t st = p->side->stream;
   GJXL_AMD_TRY(Check(hipStreamWaitEvent(st, p->coded, 0), "hipStreamWaitEvent"));
+  GJXL_AMD_TRY(MarkTokens(p, kBeforeStatistics));
   const uint32_t* stats = AqBuffer<uint32_t>(p->session, GJXL_AMD_AQ_STATS);
   GJXL_AMD_TRY(Check(hipMemcpyAsync(p->host_words + 4, stats + 7, 4, hipMemcpyDeviceToHost, st),
                      "hipMemcpyAsync(AQ error)"));
@@ -322,6 +334,7 @@ GJXLResult TokensFinish(GJXLAmdPlainPath* p) {
                                                        p->entropy_inputs));
   gjxl_amd::TokenizerUseDevice(p->tokenizer, p->side);
   GJXLResult r = gjxl_amd_tokenizer_set_entropy_inputs(p->tokenizer, p->entropy_inputs);
+  if (r == GJXL_OK) r = MarkTokens(p, kAfterInputs);
   if (r == GJXL_OK) {
     r = gjxl_amd::TokenizeEnqueue(p->tokenizer,
                                   AqBuffer<int32_t>(p->session, GJXL_AMD_AQ_QUANTIZED), p->cells,
@@ -329,6 +342,7 @@ GJXLResult TokensFinish(GJXLAmdPlainPath* p) {
   }
   gjxl_amd::TokenizerUseDevice(p->tokenizer, p->device);
   GJXL_AMD_TRY(r);
+  GJXL_AMD_TRY(MarkTokens(p, kAfterTokenize));
   GJXL_AMD_TRY(Check(hipMemcpyAsync(p->host_words,
                                     TokenBuffer<uint32_t>(p->tokenizer, GJXL_AMD_TOKENS_STATUS),
                                     16, hipMemcpyDeviceToHost, st), "hipMemcpyAsync(status)"));
@@ -427,10 +441,7 @@ GJXLResult RunBack(GJXLAmdPlainPath* p, bool costs_ready) {
     GJXL_AMD_TRY(Check(hipMemcpyAsync(p->host_words + 8, p->score_words, 4 * p->evaluations_run,
                                       hipMemcpyDeviceToHost, st), "hipMemcpyAsync(scores)"));
   }
-  if (!tokens_done) GJXL_AMD_TRY(TokensFinish(p));
-  // (what these stages take beyond the evaluation that they run beside)
-  GJXL_AMD_TRY(Mark(p, GJXL_AMD_STAGE_ENTROPY_INPUTS));
-  return Mark(p, GJXL_AMD_STAGE_AC_TOKENIZE);
+  return tokens_done ? GJXL_OK : TokensFinish(p);
 }
 
 GJXLResult ReadTokens(GJXLAmdPlainPath* p, const GJXLAmdTokenOutput* out) {
@@ -445,6 +456,7 @@ GJXLResult ReadTokens(GJXLAmdPlainPath* p, const GJXLAmdTokenOutput* out) {
     return Fail(GJXL_ERROR_INVALID_ARGUMENT, "group offset output holds fewer than groups + 1");
   }
   hipStream_t st = p->side->stream;
+  GJXL_AMD_TRY(MarkTokens(p, kBeforeRead));
   const size_t count = static_cast<size_t>(p->token_count);
   if (out->values != nullptr && count > 0) {
     GJXL_AMD_TRY(Check(hipMemcpyAsync(out->values,
@@ -466,10 +478,8 @@ GJXLResult ReadTokens(GJXLAmdPlainPath* p, const GJXLAmdTokenOutput* out) {
                                       4 * (p->groups + 1), hipMemcpyDeviceToHost, st),
                        "hipMemcpyAsync(group offsets)"));
   }
-  GJXL_AMD_TRY(Check(hipEventRecord(p->tokens_read, st), "hipEventRecord"));
-  GJXL_AMD_TRY(Check(hipStreamWaitEvent(p->device->stream, p->tokens_read, 0),
-                     "hipStreamWaitEvent"));
-  return Mark(p, GJXL_AMD_STAGE_TOKEN_READBACK);
+  p->tokens_read = true;
+  return MarkTokens(p, kAfterRead);
 }
 
 // The back half, the read-back into `tokens` and the waits for both streams,
@@ -593,10 +603,12 @@ GJXLResult gjxl_amd_plain_path_create(GJXLAmdDevice* device, uint32_t width, uin
     r = Check(hipEventCreateWithFlags(&p->reference_ready, hipEventDisableTiming),
               "hipEventCreateWithFlags");
   }
-  for (hipEvent_t* e : {&p->coded, &p->tokens_read}) {
-    if (r == GJXL_OK) {
-      r = Check(hipEventCreateWithFlags(e, hipEventDisableTiming), "hipEventCreateWithFlags");
-    }
+  if (r == GJXL_OK) {
+    r = Check(hipEventCreateWithFlags(&p->coded, hipEventDisableTiming),
+              "hipEventCreateWithFlags");
+  }
+  for (hipEvent_t& e : p->token_marks) {
+    if (r == GJXL_OK) r = Check(hipEventCreate(&e), "hipEventCreate");
   }
   if (r == GJXL_OK) r = gjxl_amd_tokenizer_create(device, width, height, &p->tokenizer);
   if (r != GJXL_OK) {
@@ -623,7 +635,9 @@ void gjxl_amd_plain_path_destroy(GJXLAmdPlainPath* p) {
   if (p->linear_ready != nullptr) (void)hipEventDestroy(p->linear_ready);
   if (p->reference_ready != nullptr) (void)hipEventDestroy(p->reference_ready);
   if (p->coded != nullptr) (void)hipEventDestroy(p->coded);
-  if (p->tokens_read != nullptr) (void)hipEventDestroy(p->tokens_read);
+  for (hipEvent_t e : p->token_marks) {
+    if (e != nullptr) (void)hipEventDestroy(e);
+  }
   gjxl_amd_device_destroy(p->side);
   if (p->host_words != nullptr) (void)hipHostFree(p->host_words);
   if (p->host_statistics != nullptr) (void)hipHostFree(p->host_statistics);
@@ -701,6 +715,7 @@ GJXLResult BeginRun(GJXLAmdPlainPath* p, const GJXLAmdImage* image, const uint8_
   p->ran = false;
   p->front_done = false;
   p->mark_count = 0;
+  p->tokens_read = false;
   GJXL_AMD_TRY(Mark(p, GJXL_AMD_STAGE_BEGIN));
   const uint8_t* srgb = static_cast<const uint8_t*>(image->pixels);
   size_t stride = image->row_stride_bytes;
@@ -841,13 +856,23 @@ GJXLResult gjxl_amd_plain_path_stage_times(GJXLAmdPlainPath* p, int32_t* stages,
     return Fail(GJXL_ERROR_INVALID_ARGUMENT, "stage time outputs are null");
   }
   if (!p->ran) return Fail(GJXL_ERROR_INVALID_ARGUMENT, "the plain path has not completed a run");
-  const int n = p->mark_count - 1;
-  *count = n;
-  for (int i = 0; i < n && i < capacity; ++i) {
-    GJXL_AMD_TRY(Check(hipEventElapsedTime(&milliseconds[i], p->marks[i], p->marks[i + 1]),
-                       "hipEventElapsedTime"));
-    stages[i] = p->mark_stage[i + 1];
+  int n = 0;
+  auto span = [&](int32_t stage, hipEvent_t begin, hipEvent_t end) -> GJXLResult {
+    const int i = n++;
+    if (i >= capacity) return GJXL_OK;
+    stages[i] = stage;
+    return Check(hipEventElapsedTime(&milliseconds[i], begin, end), "hipEventElapsedTime");
+  };
+  for (int i = 1; i < p->mark_count; ++i) {
+    GJXL_AMD_TRY(span(p->mark_stage[i], p->marks[i - 1], p->marks[i]));
   }
+  const hipEvent_t* t = p->token_marks;
+  GJXL_AMD_TRY(span(GJXL_AMD_STAGE_ENTROPY_INPUTS, t[kBeforeStatistics], t[kAfterInputs]));
+  GJXL_AMD_TRY(span(GJXL_AMD_STAGE_AC_TOKENIZE, t[kAfterInputs], t[kAfterTokenize]));
+  if (p->tokens_read) {
+    GJXL_AMD_TRY(span(GJXL_AMD_STAGE_TOKEN_READBACK, t[kBeforeRead], t[kAfterRead]));
+  }
+  *count = n;
   return GJXL_OK;
 }
 

@@ -712,9 +712,12 @@ GJXL_AMD_API GJXLResult gjxl_amd_cost_queue_grids(GJXLAmdCostQueue* queue,
 /* internal.h:18-47): upload, XYB, Gaborish inverse, initial quant field,    */
 /* initial CfL, AC strategy search, AQ preparation, three Butteraugli-driven */
 /* evaluations with two field updates (effort 7), AC tokenization of the     */
-/* last evaluation and the read-back of its tokens.  One stream; the host    */
-/* waits for the matrix-scale statistics and for the token count.  The       */
-/* entropy coder and bitstream writer that consume the frame stay on the     */
+/* last evaluation and the read-back of its tokens.  The Butteraugli         */
+/* reference side and the tokens run on a second stream of the path's; the   */
+/* host waits for the matrix-scale statistics, the frame statistics, the     */
+/* token count and the end of both streams.  A run whose loop fails (an      */
+/* invalid block distance) leaves the caller's token buffers as they were.   */
+/* The entropy coder and bitstream writer that consume the frame stay on the */
 /* CPU (src/codestream/vardct/encoder.cpp).                                  */
 /* ---------------------------------------------------------------------- */
 typedef struct GJXLAmdPlainPath GJXLAmdPlainPath;
@@ -846,9 +849,15 @@ GJXL_AMD_API GJXLResult gjxl_amd_plain_path_run_back(GJXLAmdPlainPath* path,
                                                      int32_t costs_ready,
                                                      const GJXLAmdTokenOutput* tokens,
                                                      GJXLAmdPlainFrame* frame);
-/* Device time of each stage of the last completed run, from HIP events on
- * the device stream: stages[i] (GJXL_AMD_STAGE_*) took milliseconds[i];
- * *count receives the number of entries (evaluation stages repeat). */
+/* Device time of each stage of the last completed run, from HIP events:
+ * stages[i] (GJXL_AMD_STAGE_*) took milliseconds[i]; *count receives the
+ * number of entries (evaluation stages repeat).  The last entries, ENTROPY_
+ * INPUTS (the host's choice among them), AC_TOKENIZE and, when tokens were
+ * read back, TOKEN_READBACK, are times on the path's second stream, where
+ * these stages run beside the end of the last evaluation and its comparison:
+ * the entries add up to more than the run takes.  The others are times on the
+ * device stream; BUTTERAUGLI_PREPARE, which runs on the second stream too, is
+ * what is left of it there once the stages beside it are done. */
 GJXL_AMD_API GJXLResult gjxl_amd_plain_path_stage_times(
   GJXLAmdPlainPath* path, int32_t* stages, float* milliseconds,
   int32_t capacity, int32_t* count);

@@ -158,10 +158,20 @@ def test_native_plain_path_matches_oracle_digests(device, name):
         got.update(entropy_digests(None, path.entropy_inputs()))
         differ = [k for k in FRAME_KEYS if got[k] != want[k]]
         assert not differ, f"{name} run {run}: differs from the oracle at {differ}"
-    stages = [s for s, _ in path.stage_times()]
+    times = path.stage_times()
+    stages = [s for s, _ in times]
     assert stages[0] == "upload" and stages[-1] == "token_readback"
     assert "entropy_inputs" in stages
     assert stages.count("aq_evaluate") == 3
+    # the tokens' stages are timed where they run: their bytes come back no
+    # faster than a PCIe 5 x16 link carries them (64 GB/s), and the other two
+    # are 4 and 7 launches, none of them over in a microsecond
+    own = {s: ms for s, ms in times if s in ("entropy_inputs", "ac_tokenize", "token_readback")}
+    assert [s for s in stages if s in own] == ["entropy_inputs", "ac_tokenize", "token_readback"]
+    assert own["token_readback"] > 6 * count / 64e9 * 1e3
+    assert own["entropy_inputs"] > 3e-3 and own["ac_tokenize"] > 6e-3
+    path.run(srgb, read_tokens=False)
+    assert "token_readback" not in [s for s, _ in path.stage_times()]
     path.close()
 
 
