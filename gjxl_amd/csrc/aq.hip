@@ -1756,7 +1756,7 @@ __global__ __launch_bounds__(256) void BlockFieldsKernel(
 #pragma unroll
   for (int c = 0; c < 3; ++c) reconstructed[c * n + i] = dc[c][1][1];
   const bool edge = y == 0 || x == 0 || y + 1 >= bh || x + 1 >= bw;
-  constexpr float kSide = 0.20345139757231578f, kCorner = 0.0334829185966739f;
+  constexpr float kSide = 0.20345139757231578f, kCorner = 0.0334829185968739f;
   constexpr float kCenter = 1.0f - 4.0f * (kSide + kCorner);
   float smoothed[3];
   float gap = 0.5f;
