@@ -142,28 +142,41 @@ def _pmc_dispatches(path: str, counter: str) -> list[tuple[int, str, float]]:
     return rows
 
 
-def _stage_spans(names: list[str]) -> dict[str, list[tuple[int, int]]]:
-    """Dispatch index ranges (inclusive) of the AQ evaluations and the
-    Butteraugli compares in one counter run: an evaluation runs from a
-    FillWordsKernel (its first dispatch) to the next LoopFilterKernel; a
-    compare from the dispatch after that to the next ComposeKernel."""
-    spans = {"aq_evaluate": [], "butteraugli_compare": []}
-    last_fill = None
-    i = 0
-    while i < len(names):
-        if "FillWordsKernel" in names[i]:
-            last_fill = i
-        if "LoopFilterKernel" in names[i]:
-            if last_fill is not None:
-                spans["aq_evaluate"].append((last_fill, i))
-            j = i + 1
-            while j < len(names) and "ComposeKernel" not in names[j]:
-                j += 1
-            if j < len(names):
-                spans["butteraugli_compare"].append((i + 1, j))
-            last_fill = None
-        i += 1
-    return spans
+# the kernels of an AQ evaluation and of a Butteraugli compare
+STAGE_KERNELS = {
+    "aq_evaluate": ("QuantizerKernel", "SelectPassKernel", "RawQuantKernel", "FinalCflKernel",
+                    "CodeTransformKernel", "DcQuantKernel", "BlockFieldsKernel",
+                    "ReconstructKernel", "LoopFilterKernel"),
+    "butteraugli_compare": ("ExpandKernel", "OpsinDynamicsKernel", "BlurKernel",
+                            "DifferencesKernel", "ComposeKernel"),
+}
+
+
+def _kernel(name: str) -> str:
+    """The kernel of a dispatch's demangled name, without template arguments."""
+    import re
+    m = re.search(r"(\w+Kernel)\b", name)
+    return m.group(1) if m else name
+
+
+def _stage_dispatches(names: list[str]) -> dict[str, list[list[int]]]:
+    """Dispatch indexes of each AQ evaluation and each Butteraugli compare in
+    one counter run: an evaluation's kernels up to a LoopFilterKernel, and from
+    there a compare's up to the next ComposeKernel (the preparation, which has
+    the same kernels, comes before).  Other dispatches in between, those of the
+    last evaluation's tokens on the path's second stream, belong to neither."""
+    out = {stage: [] for stage in STAGE_KERNELS}
+    stage, span = "aq_evaluate", []
+    for i, name in enumerate(names):
+        kernel = _kernel(name)
+        if kernel not in STAGE_KERNELS[stage]:
+            continue
+        span.append(i)
+        if kernel == STAGE_KERNELS[stage][-1]:
+            out[stage].append(span)
+            stage = "butteraugli_compare" if stage == "aq_evaluate" else "aq_evaluate"
+            span = []
+    return out
 
 
 # kernel families whose HBM bytes per launch the counter summary reports
@@ -184,8 +197,8 @@ def pmc_summary(fetch_csv: str, write_csv: str) -> dict:
         factor = CALIBRATION_BYTES / (float(np.median(copies)) * 1024.0)
         names = [name for _, name, _ in rows]
         values = [v for _, _, v in rows]
-        for stage, spans in _stage_spans(names).items():
-            per = [sum(values[a:b + 1]) for a, b in spans]
+        for stage, spans in _stage_dispatches(names).items():
+            per = [sum(values[i] for i in span) for span in spans]
             entry = out.setdefault(stage, {"launches": len(per)})
             entry[counter] = round(float(np.mean(per)) * 1024.0 * factor)
         for family in TRAFFIC_KERNELS:
