@@ -146,6 +146,25 @@ def test_weight_gradients_over_runs(device, shape):
     net.close()
 
 
+def test_weight_gradients_beside_an_infinity(device):
+    """What lies past the end of a row adds nothing to a weight gradient, also
+    where the row's last sample is infinite: the taps that look to the left of
+    a position never meet that sample (the labels beside it are outside the
+    loss, so that every output gradient is finite)."""
+    n, h, w = 1, 6, 37
+    x, labels, targets = _problem(6, n, h, w)
+    x[:, :, -1, 3] = 0x7F80
+    labels[:, :, -14:] = P.IGNORE
+    net = prop.ProposalNet(device, n * h * w, _params(6))
+    feats, lab, tgt = device.array(x), device.array(labels), device.array(targets)
+    net.forward(feats, n, h, w)
+    net.backward(lab, tgt, 0.5, sums=False)
+    got = net.gradients()[:9 * 32 * P.FEATURES].reshape(9, 32, P.FEATURES)
+    assert np.isfinite(got[[0, 3, 6]]).all()
+    assert np.isfinite(np.delete(got, 3, axis=2)).all()
+    net.close()
+
+
 def test_adam_matches_oracle(device):
     x, labels, targets = _problem(4)
     n, h, w, _ = x.shape
