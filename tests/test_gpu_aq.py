@@ -163,31 +163,67 @@ def test_aq_dc_wide_groups(device):
     s.close()
 
 
+@pytest.fixture(scope="module")
+def zero_frame_raw():
+    """The raw quant that the coding of an all-zero 8x8 transform makes of each
+    raw quant 1..256 (no product of the coding depends on it then)."""
+    bh, bw = 64, 64
+    zeros = np.zeros((3, 8 * bh, 8 * bw), np.float32)
+    fe = {"opsin": zeros, "pre": zeros, "cells": np.full((bh, bw), 1, np.uint8),
+          "quant_field": np.full((bh, bw), 0.7, np.float32)}
+    setup = binding.aq_setup(fe, 8 * bw, 8 * bh)
+    # more than half of the blocks alike: no deviation, a scale of 3932
+    field = np.full((bh, bw), 0.3, np.float32)
+    field[:28] = np.linspace(1e-3, 30.0, 28 * bw).astype(np.float32).reshape(28, bw)
+    raw, _ = binding.quantizer_from_field(field, setup["quant_dc"])
+    table = np.zeros(257, np.int32)
+    table[raw] = binding.aq_evaluate(fe, setup, field, 8 * bw, 8 * bh)["raw"]
+    assert np.unique(raw).size == 256
+    return table
+
+
+def _selection_field(kind, rng, n):
+    if kind == "spread":
+        return np.exp(rng.normal(0.0, 2.0, n))
+    if kind == "ties":
+        return rng.integers(1, 5, n) * 0.1
+    if kind == "constant":
+        return np.full(n, 0.3)
+    # a median near 1000 and a deviation near 999.6: the scale is 13107 times
+    # their difference, 0.8 for a unit of the last place of either, so that
+    # the last digit of both selections counts
+    v, at, fifth = np.empty(n), rng.permutation(n), n // 5
+    v[at] = 1000.0 + rng.uniform(-0.02, 0.02, n)
+    v[at[:2 * fifth]] = rng.uniform(0.3, 0.5, 2 * fifth)
+    v[at[2 * fifth:4 * fifth]] = rng.uniform(1999.5, 1999.7, 2 * fifth)
+    return v
+
+
 @pytest.mark.parametrize("w,h", [(8, 8), (264, 40), (1024, 1024), (1032, 1024), (1544, 1032)])
-@pytest.mark.parametrize("kind", ["spread", "ties", "constant"])
-def test_quantizer_selection(device, w, h, kind):
+@pytest.mark.parametrize("kind", ["spread", "ties", "constant", "digits"])
+def test_quantizer_selection(device, zero_frame_raw, w, h, kind):
     """The quantizer's exact median and MAD on both sides of the one-group
-    limit (16,384 blocks), with ties and a constant field, against a sort."""
+    limit (16,384 blocks), against the oracle's sort: the state that they give,
+    all of it exactly, and every block's raw quant (of a frame of zeros, whose
+    coding changes a raw quant in a known way).  The DC's cap on the scale,
+    8813, hides a median: every field of more than one block stays below it."""
     print(f"quantizer {w}x{h} {kind}", flush=True)
-    rng = np.random.default_rng(w + h)
     bh, bw = h // 8, w // 8
-    opsin = device.array(rng.uniform(0.0, 0.5, (3, h, w)).astype(np.float32))
-    field = {"spread": np.exp(rng.normal(0.0, 2.0, (bh, bw))),
-             "ties": rng.integers(1, 5, (bh, bw)) * 0.375,
-             "constant": np.full((bh, bw), 0.71)}[kind].astype(np.float32)
+    zeros = device.array(np.zeros((3, h, w), np.float32))
+    field = _selection_field(kind, np.random.default_rng(w + h), bh * bw).astype(
+        np.float32).reshape(bh, bw)
     s = gjxl_amd.AqSession(device, w, h)
-    s.prepare(opsin, opsin, device.array(np.full((bh, bw), 1, np.uint8)),
+    s.prepare(zeros, zeros, device.array(np.full((bh, bw), 1, np.uint8)),
               device.array(np.full((bh, bw), 0.7, np.float32)))
+    raw, want = binding.quantizer_from_field(field, s.policy()["quant_dc"])
+    assert (w, h) == (8, 8) or want[2] < 8813
     for _ in range(2):  # the second selection finds the scratch as the first left it
         s.evaluate(device.array(field))
         q = s.buffer("quantizer", (10,), np.uint32).numpy()
-        n = field.size
-        median = np.sort(field.reshape(-1))[n // 2]
-        mad = np.sort(np.abs(field.reshape(-1) - median))[n // 2]
-        scale = np.float32(65536.0) * (median - mad) / np.float32(5.0)
-        want = int(min(max(scale, np.float32(1.0)), np.float32(32768.0)))
-        dc = int(float(np.float32(s.policy()["quant_dc"]) * np.float32(4096.0)) * 1.6)
-        assert int(q[2]) == (max(dc, 1) if want > dc else want)
+        assert (int(q[2]), int(q[3])) == (int(want[2]), int(want[3]))
+        for part in (slice(0, 2), slice(4, 10)):
+            _same("quantizer", q[part].view(np.float32), want[part])
+        _same("raw", s.buffer("raw_quant", (bh, bw), np.int32).numpy(), zero_frame_raw[raw])
     s.close()
 
 
