@@ -28,8 +28,8 @@
 // Every launch covers both scales: the work groups of the half scale follow
 // those of the full one.  An image has some fifty kernels' worth of stages,
 // and below about two megapixels each of them is over before the next launch
-// could have filled the chip (a 512x512 comparison and preparation took 88
-// launches of 4 to 16 us each; now 13).
+// could have filled the chip (a 512x512 preparation and comparison took 43 and
+// 45 launches of 4 to 16 us each; now 6 and 7).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -142,7 +142,7 @@ __device__ __forceinline__ float ConvolveBorder(Sample sample, Inside inside, fl
 // radius 16 at 77x45 34 to 23 us, at 1537x1153 75 to 66, at 4032x3024 250 to
 // 230.  The separate row and column kernels that this replaces wrote and read
 // a plane more per pass, re-read 8 + 2R rows for every eight outputs of a
-// column, and took 22 launches per image and scale pair where this takes
+// column, and took 36 launches per image and scale pair where this takes
 // four (all four radii at 4032x3024, reference image: 830 to 540 us; whole
 // preparation and comparison at 1537x1153: 1063 to 490).
 constexpr int kStripW = 128, kBandH = 16;
@@ -1530,9 +1530,6 @@ Taps HostTaps(float sigma) {
 
 inline dim3 Grid2(int w, int h, int z = 1) {
   return dim3(CeilDiv(static_cast<uint32_t>(w), kThreads), h, z);
-}
-inline dim3 Grid1(size_t n) {
-  return dim3(static_cast<uint32_t>((n + kThreads - 1) / kThreads));
 }
 
 const Taps& TapsOf(ButteraugliSigma s) {

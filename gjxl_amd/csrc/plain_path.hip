@@ -403,8 +403,12 @@ GJXLResult RunBack(GJXLAmdPlainPath* p, bool costs_ready) {
       GJXL_AMD_TRY(TokensBegin(p));
       break;
     }
-    // the last evaluation, as far as is known: the judge may ask for another,
-    // whose tokens then replace this one's
+    // The last evaluation, as far as is known: the judge may ask for another,
+    // whose tokens then replace this one's.  Waiting for the judge before the
+    // tokens begin saves a run that goes on at most 0.8 % (2048x1536: 4814 to
+    // 4774 us, 3500x2500: 9998 to 9925) and costs one that stops 3 to 10 %
+    // (700x500: 1443 to 1591 us, 3500x2500: 7743 to 8000); waiting for the
+    // token count only after the judge changes neither.
     const bool last = it >= planned;
     GJXL_AMD_TRY(gjxl_amd::AqEvaluate(p->session, field, last ? p->coded : nullptr));
     GJXL_AMD_TRY(Mark(p, GJXL_AMD_STAGE_AQ_EVALUATE));
